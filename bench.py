@@ -33,7 +33,9 @@ FLOP_PER_FACE = 28  # time to the plane (sub, div: 2) + drift (dt^2, 3 x positio
 FLOP_PER_RK4_STEP = 82  # folded hexapole RK4 step: 4 slope evaluations (r^2*cu 1, fract 1, spline 2 FMA, slope
 #                         mul + FMA: 9 each, plus r^2 = 3 at stages 2-4), stage points 16, slope sums and update
 #                         18, bore test r^2 3 (z and t are formed once per molecule from the step count)
-FLOP_ADJ_STEP = 204  # reverse of one RK4 step: 4 force+derivative evaluations, stage points, adjoint sums
+FLOP_ADJ_STEP = 158  # reverse of one RK4 step: 4 slope+derivative evaluations with r^2 (14 each), two slopes 6,
+#                      stage points 16, 4 transposed stage Jacobians (12 each), adjoint sums 32
+SMOOTH_WINDOW = 4  # steps between checkpoints: the reverse sweep recomputes all but the last of each window
 FLOP_SMOOTH_FACE = 23  # smoothed objective, per aperture face: drift, radius, sigmoid, product
 FLOP_SMOOTH_FACE_REV = 34  # its reverse: radius, sigmoid, factor derivative, drift adjoint
 PEAK_FP64 = 78.6  # TFLOP/s, MI355X FP64 vector
@@ -150,25 +152,21 @@ def timed_ms(ctx, fn, reps: int, warmup: int = 2) -> float:
 
 def smooth_flop(theta: np.ndarray, eps: np.ndarray, bl, K: int, max_steps: int, grad: bool) -> float:
     """FLOPs of one k_smooth launch for one parameter set, from each molecule's lens step count: the
-    forward sweep, and with grad the reverse sweep's recomputation (per checkpoint segment of length
-    Ls: the state every 8 steps, 8 (ceil(Ls/8) - 1) steps, then each 8-step window again, Ls - ceil(Ls/8)
-    steps), the adjoint of every step and the faces' reverse."""
+    forward sweep, and with grad the reverse sweep's recomputation (checkpoints every SMOOTH_WINDOW full
+    steps, whatever K asks for, while the checkpoint store stays within its bound, as it does here: all
+    but the last step of each window again), the adjoint of every step and the faces' reverse."""
     from trajectories import configs
 
     L, dt = bl.elements[1].L, bl.elements[1].dt
     vz = theta[-1] + configs.VZ_SIGMA * eps
-    nfull = np.clip(np.floor(L / (vz * dt)), 0, max_steps)
-    S = np.where(vz > 0, nfull + 1, 0).astype(np.int64)
+    nfull = np.where(vz > 0, np.clip(np.floor(L / (vz * dt)), 0, max_steps), 0)
+    steps = float((nfull + 1)[vz > 0].sum())
     faces = 4 * int((vz > 0).sum())  # three aperture faces and the lens entrance
-    f = FLOP_PER_RK4_STEP * float(S.sum()) + FLOP_SMOOTH_FACE * faces
+    f = FLOP_PER_RK4_STEP * steps + FLOP_SMOOTH_FACE * faces
     if not grad:
         return f
-    full, last = S // K, S % K
-    def recompute(Ls):
-        nsub = -(-Ls // 8)
-        return np.where(Ls > 0, 8 * (nsub - 1) + (Ls - nsub), 0)
-    rec = full * recompute(np.full_like(S, K)) + recompute(last)
-    return f + FLOP_PER_RK4_STEP * float(rec.sum()) + FLOP_ADJ_STEP * float(S.sum()) + FLOP_SMOOTH_FACE_REV * faces
+    rec = float((nfull - np.ceil(nfull / min(K, SMOOTH_WINDOW))).sum())
+    return f + FLOP_PER_RK4_STEP * rec + FLOP_ADJ_STEP * steps + FLOP_SMOOTH_FACE_REV * faces
 
 
 def bench_adjoint(ctx, n: int, K: int, reps: int = 5) -> dict:
@@ -226,9 +224,9 @@ def bench_adjoint(ctx, n: int, K: int, reps: int = 5) -> dict:
         "grad_vs_fd_max_rel_err": fd_err, "J": float(J1.to_host()[0]),
         "roofline": {"bound": "mfma", "engine": ENGINE, "achieved": achieved, "peak": PEAK_FP64, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP64, "kernel": "k_smooth<true>", "flop_per_launch": f_adj,
-                     "flop_rule": "forward %d/RK4 step + 23/face; reverse: recomputed steps %d each (two-level "
-                                  "checkpoints), 204 per step adjoint, 34 per face"
-                                  % (FLOP_PER_RK4_STEP, FLOP_PER_RK4_STEP)},
+                     "flop_rule": "forward %d/RK4 step + 23/face; reverse: recomputed steps %d each (3 of 4), "
+                                  "%d per step adjoint, 34 per face"
+                                  % (FLOP_PER_RK4_STEP, FLOP_PER_RK4_STEP, FLOP_ADJ_STEP)},
     }
 
 

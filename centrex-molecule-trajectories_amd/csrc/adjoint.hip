@@ -5,9 +5,9 @@
 // lens is integrated with the same classical RK4 (and the same FMA sequence) as the propagation
 // kernels.  With GRAD the wavefront then runs the reverse sweep:
 //   * aperture faces: the sigmoid factor's derivative and the adjoint of the ballistic drift;
-//   * lens: for each checkpoint segment (last first) the K steps are recomputed from the stored
-//     checkpoint into a per-wavefront recompute store, then the adjoint of each RK4 step is applied
-//     backwards, accumulating d/dV through the field scale and d/d(vz) through the final partial step;
+//   * lens: the adjoint of the final partial step (with d/dh, which carries d/d(vz)), then, for each
+//     checkpoint segment (last first), the segment's steps recomputed from the checkpoint and the
+//     adjoint of each full step applied backwards, accumulating d/dV through the field scale;
 //   * the mean axial speed collects the adjoint of vz.
 // Per-parameter sums are reduced over the wavefront (xor butterfly) at wave-uniform points and
 // written per work item; k_smooth_reduce adds the items of each parameter set in a fixed order,
@@ -15,9 +15,10 @@
 //
 // Workspace of one wavefront (doubles, lane-minor so that every access is one 512-byte row):
 //   faces [n_face_slots][4][64]   state (x, y, vx, vy) on each aperture face and lens entrance
-//   ckpt  [n_ck_slots][4][64]     lens state before steps 0, K, 2K, ...
-//   sub   [ceil(K/8)][4][64]      state every 8 steps of the segment being reversed
-// and, in LDS, a [8][4][64] window of recomputed step inputs per wavefront.
+//   ends  [n_lens][4][64]         lens state before the final partial step
+//   ckpt  [n_ck_slots][4][64]     lens state before full steps 0, K, 2K, ...
+//   sub   [ceil(K/kSub)][4][64]   state every kSub steps of the segment being reversed (K > kSub)
+// and, in LDS, a [kSub][4][64] window of recomputed step inputs per wavefront.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -38,17 +39,18 @@ struct SmoothArgs {
   double *partial;                // [n_items][n_params + 1]: gradient sums, then the J sum
   double *ws;                     // workspace, ws_stride doubles per wavefront
   unsigned long long *n_capped;   // may be null
+  unsigned long long *next;       // items handed out beyond each wavefront's first (zeroed before the launch)
   int64_t n, items_per_cfg, n_items, ws_stride;
   double z_src, sigma_vz, inv_s;
-  int n_params, K, max_steps, ck_per_lens, off_ck, off_sub;  // offsets in rows of 256 doubles
+  int n_params, K, max_steps, ck_per_lens, off_end, off_ck, off_sub;  // offsets in rows of 256 doubles
   int rec_lds;                  // LDS offset (doubles) of the per-wavefront recompute windows
 };
 
-// Inside a checkpoint segment the reverse sweep works in windows of kSub steps: the segment is
-// recomputed once to store the state every kSub steps (HBM rows, cache-resident), then each
-// window, last first, is recomputed into the wavefront's LDS slice and reversed.  With K <= kSub
-// (the default K = kSub) a segment is one window: every step is recomputed once.
-constexpr int kSub = 8;
+// Inside a checkpoint segment the reverse sweep works in windows of kSub steps: a segment of more
+// than one window is recomputed once to store the state every kSub steps (HBM rows, cache-resident),
+// then each window, last first, is recomputed into the wavefront's LDS slice and reversed.  With
+// K <= kSub a segment is one window: 1 - 1/kSub forward steps are recomputed per step.
+constexpr int kSub = 4;
 
 // sigmoid(w) and 1 - sigmoid(w) without cancellation.
 __device__ __forceinline__ void sigmoid2(double w, double &phi, double &omphi) {
@@ -77,134 +79,132 @@ __device__ __forceinline__ double drift_g_adj(double vx, double vy_after, double
   return taubar;
 }
 
-// Hexapole force and its derivatives at r2 = x^2 + y^2:
-//   f  = ks W'(u), u = min(cu r2, umax)       (a = f (x, y) - g y_hat; identical to force_hex_r2)
-//   d  = 2 ks cu dW'/du  (= 2 df/dr2; 0 where u is clamped)
-//   gv = df/dV = (f + ks cu dW'/du r2) / V    (ks and cu are both proportional to V)
-__device__ __forceinline__ void hex_eval_d(const WsRef &wsb, double umax, double ks, double cu, double kc2,
-                                           double invV, double r2, double &f, double &d, double &gv) {
-  const double u0 = r2 * cu;
-  const double u = clamp_to(u0, umax);
-  const unsigned k = (unsigned)(int)u;
-  const double s = __builtin_amdgcn_fract(u);
-  const dbl2_t ab = wsb.ab[k];
-  const double A = ab.x, Bc = ab.y, C = wsb.c[k];
-  const double P = __builtin_fma(__builtin_fma(A, s, Bc), s, C);
-  double dP = __builtin_fma(2.0 * A, s, Bc);
-  if (u0 > umax) dP = 0.0;
-  f = P * ks;
-  d = kc2 * dP;
-  gv = __builtin_fma(0.5 * d, r2, f) * invV;
+// A value that is the same in every lane, as a scalar register pair.  FP64 arithmetic has no scalar
+// unit, so the lens constants formed from a parameter set (20 doubles) would otherwise hold 40 vector
+// registers of every lane.
+__device__ __forceinline__ double uniform_f64(double v) {
+  return __longlong_as_double((long long)uniform_u64((unsigned long long)__double_as_longlong(v)));
 }
 
+__device__ __forceinline__ HexK uniform_hex_k(double ks, double h) {
+  const HexK k = hex_k(ks, h);
+  return HexK{uniform_f64(k.h), uniform_f64(k.hh), uniform_f64(k.c3), uniform_f64(k.c4), uniform_f64(k.cx),
+              uniform_f64(k.kh6)};
+}
+
+// One lens of one parameter set.  FOLD (hex_folds(ks)): slopes are s = W' p + (0, gk), gk = -g/ks, and the
+// step constants are hex_k(ks, h); otherwise slopes are accelerations and the constants hex_k(1, h).
 struct LensK {
   WsRef wsb;
-  double umax, ks, cu, kc2, invV, g;
+  double umax, cu;
+  double kf;  // the step constants' scale: ks (FOLD) or 1
+  double sl;  // slope per W': 1 (FOLD) or ks
+  double gs;  // the slope's constant part: gk (FOLD) or -g
+  double c2;  // 2 cu sl: d(slope scale)/d(r2) = c2/2 dW'/du
+  HexK hk;    // of the full step
 };
 
-// The forward sweep's lens step and its recomputation in the reverse sweep: full steps of the
-// lens's uniform h take the folded hexapole step with the constants formed once per lens (as the
-// propagation's lens kernel does), the final partial step hp takes lens_step; where the force scale
-// does not fold every step takes the plain RK4 step.  The forward sweep and both recomputations call
-// this one function, so a recomputed state equals the forward state bit for bit.
-struct SmoothStep {
-  HexK hk;
-  bool fold;
-};
-
-__device__ __forceinline__ SmoothStep smooth_step_k(const Force<CTRAJ_FORCE_WSPLINE_HEX> &F, double h) {
-  return SmoothStep{hex_k(F.ks, h), hex_folds(F.ks)};
+template <bool FOLD>
+__device__ __forceinline__ void smooth_slope(const LensK &L, double x, double y, double r2, double &sx, double &sy) {
+  if constexpr (FOLD) {
+    slope_hex_k(L.wsb, L.umax, L.cu, L.gs, x, y, r2, sx, sy);
+  } else {
+    const double f = wspline_eval(L.wsb, L.umax, r2 * L.cu) * L.sl;  // force_hex_r2
+    sx = f * x;
+    sy = __builtin_fma(f, y, L.gs);
+  }
 }
 
-__device__ __forceinline__ void smooth_step(const Force<CTRAJ_FORCE_WSPLINE_HEX> &F, const Tables &T, const WsRef &wsb,
-                                            const SmoothStep &S, bool full, double hp, double &x, double &y,
-                                            double &vx, double &vy, double r2, uint32_t &st) {
-  if (full && S.fold)
-    rk4_step_hex_k(wsb, T.umax, F.cu, F.gk, S.hk, x, y, vx, vy, r2);
-  else
-    lens_step<CTRAJ_FORCE_WSPLINE_HEX>(F, T, wsb, full ? S.hk.h : hp, x, y, vx, vy, r2, st);
+// The forward sweep's lens step and its recomputation in the reverse sweep (one function, so that a
+// recomputed state equals the forward state bit for bit): the propagation kernels' folded hexapole step,
+// or their plain RK4 step where the force scale does not fold.
+template <bool FOLD>
+__device__ __forceinline__ void smooth_step(const LensK &L, const HexK &K, double &x, double &y, double &vx, double &vy) {
+  rk4_expanded(
+      K, [&](double px, double py, double pr2, double &sx, double &sy) { smooth_slope<FOLD>(L, px, py, pr2, sx, sy); }, x,
+      y, vx, vy, __builtin_fma(x, x, y * y));
 }
 
-// Reverse of one classical RK4 step of size h from input state (x, y, vx, vy), derived from the
-// stages with their velocities formed; the forward step (rk4_expanded) forms the same stages in
-// expanded form, equal in exact arithmetic, so this is its adjoint up to rounding.
-// In: (pbx, pby, vbx, vby) = adjoint of the step's output.  Out: adjoint of its input.
-// Vbar accumulates d/dV; with WANT_H the derivative with respect to h is returned.
-template <bool WANT_H>
-__device__ __forceinline__ double rk4_adjoint(const LensK &L, double h, double x, double y, double vx, double vy,
+// The slope scale and its derivatives at r2: w = sl W'(u), u = min(cu r2, umax); dw = 2 dw/dr2 (0 where u
+// is clamped); gv = V dw/dV per unit sl (ks and cu are both proportional to V): W' + u dW'/du.
+template <bool FOLD>
+__device__ __forceinline__ void hex_eval_d(const LensK &L, double r2, double &w, double &dw, double &gv) {
+  const double u0 = r2 * L.cu;
+  const double u = clamp_to(u0, L.umax);
+  const unsigned k = (unsigned)(int)u;
+  const double s = __builtin_amdgcn_fract(u);
+  const dbl2_t ab = L.wsb.ab[k];
+  const double c = L.wsb.c[k];
+  const double t = __builtin_fma(ab.x, s, ab.y);
+  const double P = __builtin_fma(t, s, c);
+  double dP = __builtin_fma(ab.x, s, t);
+  if (u0 > L.umax) dP = 0.0;
+  w = FOLD ? P : P * L.sl;
+  dw = L.c2 * dP;
+  gv = __builtin_fma(u0, dP, P);
+}
+
+// Jacobian of one stage slope s = w(r2) p + const, transposed (it is symmetric: w I + dw p p^T), applied
+// to the slope's adjoint (sbx, sby); Vbar gathers the slope's dependence on V.
+__device__ __forceinline__ void slope_adj(double w, double dw, double gv, double px, double py, double sbx, double sby,
+                                          double &pbx, double &pby, double &Vbar) {
+  const double q = __builtin_fma(px, sbx, py * sby);
+  const double dq = dw * q;
+  Vbar = __builtin_fma(q, gv, Vbar);
+  pbx = __builtin_fma(w, sbx, dq * px);
+  pby = __builtin_fma(w, sby, dq * py);
+}
+
+// Reverse of one RK4 step with constants K from input state (x, y, vx, vy): the transposed derivative of
+// rk4_expanded's own form,
+//   x2 = x + h/2 v,  x3 = x2 + c3 s1,  x4 = (x + h v) + c4 s2,
+//   x' = (x + h v) + cx (s1 + s2 + s3),  v' = v + kh6 (s1 + 2 s2 + 2 s3 + s4),
+// which needs no stage velocities (52 operations on the adjoint where the classical stages take 85).
+// In: (pbx, pby, vbx, vby) = adjoint of the step's output.  Out: adjoint of its input.  Vbar gathers
+// V/sl d/dV; with WANT_H the derivative with respect to h is returned.
+// The sums of products are fused multiply-adds (the gradient is checked against the CPU adjoint to a
+// tolerance, not bit for bit).
+template <bool FOLD, bool WANT_H>
+__device__ __forceinline__ double rk4_adjoint(const LensK &L, const HexK &K, double x, double y, double vx, double vy,
                                               double &pbx, double &pby, double &vbx, double &vby, double &Vbar) {
-  const double hh = 0.5 * h, h6 = h * kSixth, h3 = 2.0 * h6;
-  const double g = L.g;
-  double f1, d1, g1, f2, d2, g2, f3, d3, g3, f4, d4, g4;
-  // forward stages with their velocities (the classical form: rk4_step's expanded stages up to rounding)
-  hex_eval_d(L.wsb, L.umax, L.ks, L.cu, L.kc2, L.invV, __builtin_fma(x, x, y * y), f1, d1, g1);
-  const double a1x = f1 * x, a1y = __builtin_fma(f1, y, -g);
-  const double p2x = __builtin_fma(hh, vx, x), p2y = __builtin_fma(hh, vy, y);
-  const double v2x = __builtin_fma(hh, a1x, vx), v2y = __builtin_fma(hh, a1y, vy);
-  hex_eval_d(L.wsb, L.umax, L.ks, L.cu, L.kc2, L.invV, __builtin_fma(p2x, p2x, p2y * p2y), f2, d2, g2);
-  const double a2x = f2 * p2x, a2y = __builtin_fma(f2, p2y, -g);
-  const double p3x = __builtin_fma(hh, v2x, x), p3y = __builtin_fma(hh, v2y, y);
-  const double v3x = __builtin_fma(hh, a2x, vx), v3y = __builtin_fma(hh, a2y, vy);
-  hex_eval_d(L.wsb, L.umax, L.ks, L.cu, L.kc2, L.invV, __builtin_fma(p3x, p3x, p3y * p3y), f3, d3, g3);
-  const double a3x = f3 * p3x, a3y = __builtin_fma(f3, p3y, -g);
-  const double p4x = __builtin_fma(h, v3x, x), p4y = __builtin_fma(h, v3y, y);
-  hex_eval_d(L.wsb, L.umax, L.ks, L.cu, L.kc2, L.invV, __builtin_fma(p4x, p4x, p4y * p4y), f4, d4, g4);
+  double w1, d1, g1, w2, d2, g2, w3, d3, g3, w4, d4, g4;
+  hex_eval_d<FOLD>(L, __builtin_fma(x, x, y * y), w1, d1, g1);
+  const double s1x = w1 * x, s1y = __builtin_fma(w1, y, L.gs);
+  const double p2x = __builtin_fma(K.hh, vx, x), p2y = __builtin_fma(K.hh, vy, y);
+  hex_eval_d<FOLD>(L, __builtin_fma(p2x, p2x, p2y * p2y), w2, d2, g2);
+  const double s2x = w2 * p2x, s2y = __builtin_fma(w2, p2y, L.gs);
+  const double p3x = __builtin_fma(K.c3, s1x, p2x), p3y = __builtin_fma(K.c3, s1y, p2y);
+  hex_eval_d<FOLD>(L, __builtin_fma(p3x, p3x, p3y * p3y), w3, d3, g3);
+  const double xvx = __builtin_fma(K.h, vx, x), xvy = __builtin_fma(K.h, vy, y);
+  const double p4x = __builtin_fma(K.c4, s2x, xvx), p4y = __builtin_fma(K.c4, s2y, xvy);
+  hex_eval_d<FOLD>(L, __builtin_fma(p4x, p4x, p4y * p4y), w4, d4, g4);
 
-  // The reverse sweep below forms each sum of products with fused multiply-adds (it is checked
-  // against the CPU adjoint to a tolerance, not bit for bit).
-  // stage 4: a4 = A(p4), p4 = p1 + h v3, v4 = v1 + h a3
-  const double ab4x = h6 * vbx, ab4y = h6 * vby;
-  double q = __builtin_fma(p4x, ab4x, p4y * ab4y);
-  double dq = d4 * q;
-  const double pb4x = __builtin_fma(f4, ab4x, dq * p4x), pb4y = __builtin_fma(f4, ab4y, dq * p4y);
-  Vbar = __builtin_fma(q, g4, Vbar);
-  const double vb4x = h6 * pbx, vb4y = h6 * pby;
-  double Px = pbx + pb4x, Py = pby + pb4y;
-  const double vb3x = __builtin_fma(h3, pbx, h * pb4x), vb3y = __builtin_fma(h3, pby, h * pb4y);
-  double Vx = vbx + vb4x, Vy = vby + vb4y;
-  const double ab3x = __builtin_fma(h3, vbx, h * vb4x), ab3y = __builtin_fma(h3, vby, h * vb4y);
-  // stage 3: a3 = A(p3), p3 = p1 + hh v2, v3 = v1 + hh a2
-  q = __builtin_fma(p3x, ab3x, p3y * ab3y);
-  dq = d3 * q;
-  const double pb3x = __builtin_fma(f3, ab3x, dq * p3x), pb3y = __builtin_fma(f3, ab3y, dq * p3y);
-  Vbar = __builtin_fma(q, g3, Vbar);
-  Px = Px + pb3x;
-  Py = Py + pb3y;
-  const double vb2x = __builtin_fma(h3, pbx, hh * pb3x), vb2y = __builtin_fma(h3, pby, hh * pb3y);
-  Vx = Vx + vb3x;
-  Vy = Vy + vb3y;
-  const double ab2x = __builtin_fma(h3, vbx, hh * vb3x), ab2y = __builtin_fma(h3, vby, hh * vb3y);
-  // stage 2: a2 = A(p2), p2 = p1 + hh v1, v2 = v1 + hh a1
-  q = __builtin_fma(p2x, ab2x, p2y * ab2y);
-  dq = d2 * q;
-  const double pb2x = __builtin_fma(f2, ab2x, dq * p2x), pb2y = __builtin_fma(f2, ab2y, dq * p2y);
-  Vbar = __builtin_fma(q, g2, Vbar);
-  Px = Px + pb2x;
-  Py = Py + pb2y;
-  Vx = __builtin_fma(h6, pbx, __builtin_fma(hh, pb2x, Vx) + vb2x);
-  Vy = __builtin_fma(h6, pby, __builtin_fma(hh, pb2y, Vy) + vb2y);
-  const double ab1x = __builtin_fma(h6, vbx, hh * vb2x), ab1y = __builtin_fma(h6, vby, hh * vb2y);
-  // stage 1: a1 = A(p1)
-  q = __builtin_fma(x, ab1x, y * ab1y);
-  dq = d1 * q;
-  Px = Px + __builtin_fma(f1, ab1x, dq * x);
-  Py = Py + __builtin_fma(f1, ab1y, dq * y);
-  Vbar = __builtin_fma(q, g1, Vbar);
+  const double s4bx = K.kh6 * vbx, s4by = K.kh6 * vby;
+  double pb4x, pb4y, pb3x, pb3y, pb2x, pb2y, pb1x, pb1y;
+  slope_adj(w4, d4, g4, p4x, p4y, s4bx, s4by, pb4x, pb4y, Vbar);
+  const double e1x = __builtin_fma(K.cx, pbx, s4bx), e1y = __builtin_fma(K.cx, pby, s4by);
+  const double e2x = e1x + s4bx, e2y = e1y + s4by;
+  slope_adj(w3, d3, g3, p3x, p3y, e2x, e2y, pb3x, pb3y, Vbar);
+  const double s2bx = __builtin_fma(K.c4, pb4x, e2x), s2by = __builtin_fma(K.c4, pb4y, e2y);
+  slope_adj(w2, d2, g2, p2x, p2y, s2bx, s2by, pb2x, pb2y, Vbar);
+  const double s1bx = __builtin_fma(K.c3, pb3x, e1x), s1by = __builtin_fma(K.c3, pb3y, e1y);
+  slope_adj(w1, d1, g1, x, y, s1bx, s1by, pb1x, pb1y, Vbar);
+  const double xvbx = pbx + pb4x, xvby = pby + pb4y, x2bx = pb2x + pb3x, x2by = pb2y + pb3y;
   double hbar = 0.0;
   if constexpr (WANT_H) {
-    const double a4x = f4 * p4x, a4y = __builtin_fma(f4, p4y, -g);
-    const double v4x = __builtin_fma(h, a3x, vx), v4y = __builtin_fma(h, a3y, vy);
-    const double Svx = ((vx + 2.0 * v2x) + 2.0 * v3x) + v4x, Svy = ((vy + 2.0 * v2y) + 2.0 * v3y) + v4y;
-    const double Sax = ((a1x + 2.0 * a2x) + 2.0 * a3x) + a4x, Say = ((a1y + 2.0 * a2y) + 2.0 * a3y) + a4y;
-    hbar = (((pbx * Svx + pby * Svy) + (vbx * Sax + vby * Say)) / 6.0 +
-            0.5 * (((pb2x * vx + pb2y * vy) + (vb2x * a1x + vb2y * a1y)) +
-                   ((pb3x * v2x + pb3y * v2y) + (vb3x * a2x + vb3y * a2y)))) +
-           ((pb4x * v3x + pb4y * v3y) + (vb4x * a3x + vb4y * a3y));
+    const double s3x = w3 * p3x, s3y = __builtin_fma(w3, p3y, L.gs);
+    const double s4x = w4 * p4x, s4y = __builtin_fma(w4, p4y, L.gs);
+    const double S3x = (s1x + s2x) + s3x, S3y = (s1y + s2y) + s3y;
+    const double kh = L.kf * K.h;
+    hbar = (pbx * (vx + (kh / 3.0) * S3x) + pby * (vy + (kh / 3.0) * S3y)) +
+           (L.kf * kSixth) * (vbx * ((S3x + s2x) + (s3x + s4x)) + vby * ((S3y + s2y) + (s3y + s4y))) +
+           0.5 * ((x2bx * vx + x2by * vy) + kh * (pb3x * s1x + pb3y * s1y)) +
+           (pb4x * (vx + kh * s2x) + pb4y * (vy + kh * s2y));
   }
-  pbx = Px;
-  pby = Py;
-  vbx = Vx;
-  vby = Vy;
+  pbx = (xvbx + x2bx) + pb1x;
+  pby = (xvby + x2by) + pb1y;
+  vbx = __builtin_fma(K.hh, x2bx, __builtin_fma(K.h, xvbx, vbx));
+  vby = __builtin_fma(K.hh, x2by, __builtin_fma(K.h, xvby, vby));
   return hbar;
 }
 
@@ -236,37 +236,157 @@ __device__ __forceinline__ void get4(const double *W, int slot, int lane, double
   d = r[192];
 }
 
-// z of the exit face of element e (CIRC: z1; LENS: its z0 parameter + L); z_src before the first.
+// z of the exit face of an element (CIRC: z1; LENS: its z0 parameter + L); z_src before the first.
 __device__ __forceinline__ double exit_z(const KBeam &B, const double *P, int e, int pidx_e, double z_src) {
   if (e < 0) return z_src;
-  const ctraj_elem &E = B.elems[e];
-  if (E.kind == CTRAJ_LENS) return P[pidx_e + 1] + E.p[3];
+  const ctraj_elem E = elem_at(B.elems, e);
+  if (E.kind == CTRAJ_LENS) return uniform_f64(P[pidx_e + 1]) + E.p[3];
   return E.z1;
 }
 
 __device__ __forceinline__ int n_params_of(const ctraj_elem &E) { return E.kind == CTRAJ_LENS ? 2 : 1; }
 
+__device__ __forceinline__ int wave_max(int v) {
+  for (int o = 1; o < 64; o <<= 1) v = max(v, __shfl_xor(v, o, 64));
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
+__device__ __forceinline__ LensK smooth_lens(const ctraj_elem &E, const Tables &T, double scale, double g) {
+  LensK L;
+  const double ks = E.p[4] * scale, cu = E.p[5] * scale;
+  const bool fold = hex_folds(ks);
+  L.wsb = ws_of(T, 0);
+  L.umax = T.umax;
+  L.cu = uniform_f64(cu);
+  L.kf = uniform_f64(fold ? ks : 1.0);
+  L.sl = uniform_f64(fold ? 1.0 : ks);
+  L.gs = uniform_f64(fold ? -g / ks : -g);
+  L.c2 = uniform_f64((2.0 * L.sl) * cu);
+  L.hk = uniform_hex_k(L.kf, E.p[2]);
+  return L;
+}
+
+// Where a wavefront keeps what the reverse sweep of one lens needs (workspace rows), and its LDS window.
+struct LensStore {
+  double *W;
+  int end, ck, sub;  // rows: the state before the partial step, checkpoints, states every kSub steps
+  int K;
+  lds_double *rec;
+};
+
+// Forward through one lens: nfull full steps (per lane; nmax is the wavefront's largest), then the partial
+// step hp.  The step loop and its counters are wave-uniform, so every checkpoint is one coalesced row.
+template <bool GRAD, bool FOLD>
+__device__ __forceinline__ void lens_forward(const LensK &L, const LensStore &S, int lane, bool ok, int nfull, int nmax,
+                                             double hp, double &x, double &y, double &vx, double &vy) {
+  int next = 0, slot = S.ck;
+  for (int s = 0; s < nmax; ++s) {
+    const bool mark = GRAD && s == next;
+    if (s < nfull) {
+      if constexpr (GRAD) {
+        if (mark) put4(S.W, slot, lane, x, y, vx, vy);
+      }
+      smooth_step<FOLD>(L, L.hk, x, y, vx, vy);
+    }
+    if (mark) {
+      next += S.K;
+      ++slot;
+    }
+  }
+  if (ok) {
+    if constexpr (GRAD) put4(S.W, S.end, lane, x, y, vx, vy);
+    smooth_step<FOLD>(L, hex_k(L.kf, hp), x, y, vx, vy);
+  }
+}
+
+// Reverse through one lens; returns d/dhp.
+template <bool FOLD>
+__device__ __forceinline__ double lens_reverse(const LensK &L, const LensStore &S, int lane, bool ok, int nfull, int nmax,
+                                               double hp, double &pbx, double &pby, double &vbx, double &vby,
+                                               double &Vbar) {
+  double x = 0.0, y = 0.0, vx = 0.0, vy = 0.0, hbar = 0.0;
+  if (ok) {
+    get4(S.W, S.end, lane, x, y, vx, vy);
+    hbar = rk4_adjoint<FOLD, true>(L, hex_k(L.kf, hp), x, y, vx, vy, pbx, pby, vbx, vby, Vbar);
+  }
+  if (nmax == 0) return hbar;
+  for (int sg = (nmax - 1) / S.K; sg >= 0; --sg) {
+    const int s0 = sg * S.K, s1 = min(s0 + S.K, nmax);
+    const int nsub = (s1 - s0 + kSub - 1) / kSub;
+    if (s0 < nfull) get4(S.W, S.ck + sg, lane, x, y, vx, vy);
+    if (nsub > 1) {  // the state every kSub steps of the segment
+      for (int q = 0; q < nsub; ++q) {
+        const int t0 = s0 + q * kSub;
+        if (t0 < nfull) put4(S.W, S.sub + q, lane, x, y, vx, vy);
+        if (q + 1 < nsub)
+          for (int s = t0; s < t0 + kSub; ++s)
+            if (s < nfull) smooth_step<FOLD>(L, L.hk, x, y, vx, vy);
+      }
+    }
+    // windows, last first: recompute into LDS (the last state stays in registers), then reverse
+    for (int q = nsub - 1; q >= 0; --q) {
+      const int t0 = s0 + q * kSub, t1 = min(t0 + kSub, s1);
+      if (nsub > 1 && t0 < nfull) get4(S.W, S.sub + q, lane, x, y, vx, vy);
+      for (int s = t0; s < t1 - 1; ++s) {
+        if (s < nfull) {
+          lds_double *r = S.rec + (s - t0) * 256;
+          r[0] = x;
+          r[64] = y;
+          r[128] = vx;
+          r[192] = vy;
+          smooth_step<FOLD>(L, L.hk, x, y, vx, vy);
+        }
+      }
+      for (int s = t1 - 1; s >= t0; --s) {
+        if (s < nfull) {
+          if (s < t1 - 1) {
+            const lds_double *r = S.rec + (s - t0) * 256;
+            x = r[0];
+            y = r[64];
+            vx = r[128];
+            vy = r[192];
+          }
+          (void)rk4_adjoint<FOLD, false>(L, L.hk, x, y, vx, vy, pbx, pby, vbx, vby, Vbar);
+        }
+      }
+    }
+  }
+  return hbar;
+}
+
+// What bounds it: VALU issue.  With GRAD a lens step costs 74 VALU instructions forward, 3/4 of that again
+// to recompute, and 143 to reverse (169 with the stage velocities formed), at four wavefronts per SIMD:
+// 128 registers (46 spilled, none inside a step loop) and 8 KB of window each, so that 16 wavefronts share
+// one 24 KB table per CU; with the lens constants in vector registers (233) and 16 KB windows it was two.
+// 10^6 molecules, one parameter set, K = 64: 5.5 -> 3.0 ms (the four wavefronts and the shorter reverse
+// step 5.5 -> 3.84, items from a counter -> 3.1); 16 sets of 100,003, K = 8: 7.35 -> 5.1 ms.  Without
+// GRAD 115 registers hold four wavefronts; five, six and eight (96, 80, 64 registers, no spill in the step
+// loop) measured the same or slower (1.69, 1.70, 1.76 ms against 1.70 for 12 x 2 10^5 molecules; 2.05
+// with a fixed share per wavefront).
 template <bool GRAD>
-__global__ void __launch_bounds__(512) k_smooth(KBeam B, KTab KT, SmoothArgs A) {
+__global__ void __launch_bounds__(GRAD ? 1024 : 512) k_smooth(KBeam B, KTab KT, SmoothArgs A) {
   extern __shared__ __attribute__((aligned(16))) double lds[];
   const Tables T = stage_tables(lds, KT);
   __syncthreads();
-  const WsRef wsb = ws_of(T, 0);
   const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t wpb = blockDim.x >> 6;
-  const int64_t gwave = (int64_t)blockIdx.x * wpb + (threadIdx.x >> 6);
+  const int64_t gwave = (int64_t)blockIdx.x * wpb + wave;
   const int64_t nwaves = (int64_t)gridDim.x * wpb;
   double *W = GRAD ? A.ws + gwave * A.ws_stride : nullptr;
+  LensStore S{W, 0, 0, A.off_sub, A.K, nullptr};
+  if constexpr (GRAD) S.rec = (lds_double *)(lds + A.rec_lds) + wave * (kSub * 256) + lane;
   const double g = B.g;
   const int np = A.n_params;
-  const int K = A.K;
   unsigned long long capped = 0;
 
-  for (int64_t item = gwave; item < A.n_items; item += nwaves) {
+  // A SIMD issues its oldest ready wavefront first, so with a fixed share per wavefront the oldest of a
+  // SIMD's four finished in half the time of the youngest, which then ran alone (1e6 molecules: 1.7 to 3.4 ms,
+  // wavefronts alive 63 % of the kernel's time); items taken from a counter keep all of them busy to the end.
+  for (int64_t item = gwave; item < A.n_items;) {
     const int64_t cfg = item / A.items_per_cfg;
     const int64_t i = (item - cfg * A.items_per_cfg) * 64 + lane;
     const double *P = A.params + cfg * np;
-    const double mu = P[np - 1];
     double x = 0.0, y = 0.0, vx = 0.0, vy = 0.0, vz = 1.0;
     bool ok = false;
     if (i < A.n) {
@@ -274,17 +394,17 @@ __global__ void __launch_bounds__(512) k_smooth(KBeam B, KTab KT, SmoothArgs A) 
       y = A.y[i];
       vx = A.vx[i];
       vy = A.vy[i];
-      vz = mu + A.sigma_vz * A.eps[i];
+      vz = P[np - 1] + A.sigma_vz * A.eps[i];
       ok = vz > 0.0;
       if (!ok) vz = 1.0;
     }
     double Jw = ok ? 1.0 : 0.0;  // product of the sigmoid factors
     double zc = A.z_src;
-    int fslot = 0, cslot = 0, pidx = 0;
+    int fslot = 0, lens = 0, pidx = 0;
 
     // ---------------- forward ----------------
     for (int e = 0; e < B.n_elems; ++e) {
-      const ctraj_elem &E = B.elems[e];
+      const ctraj_elem E = elem_at(B.elems, e);
       if (E.kind == CTRAJ_CIRC) {
         const double r = P[pidx];
         const int nf = E.z1 > E.z0 ? 2 : 1;
@@ -302,35 +422,32 @@ __global__ void __launch_bounds__(512) k_smooth(KBeam B, KTab KT, SmoothArgs A) 
         }
         pidx += 1;
       } else {  // CTRAJ_LENS
-        const double V = P[pidx], z0 = P[pidx + 1];
+        const double V = uniform_f64(P[pidx]), z0 = uniform_f64(P[pidx + 1]);
         const double scale = V / E.p[7];
-        const double ks0 = E.p[4] * scale;
-        const Force<CTRAJ_FORCE_WSPLINE_HEX> F{ks0, E.p[5] * scale, g, hex_folds(ks0) ? -g / ks0 : 0.0};
+        const LensK L = smooth_lens(E, T, scale, g);
         const double h = E.p[2], Ll = E.p[3];
-        const SmoothStep SK = smooth_step_k(F, h);
         if (!(scale >= 0.0)) {  // a negative or NaN field scale has no table: the set contributes 0
           ok = false;
           Jw = 0.0;
         }
+        int nfull = 0;
+        double hp = 0.0;
         if (ok) {
           drift_g(x, y, vx, vy, (z0 - zc) / vz, g);
           if constexpr (GRAD) put4(W, fslot, lane, x, y, vx, vy);
           uint32_t st = 0;
-          const int nfull = rk4_full_steps(Ll, vz, h, A.max_steps, st);
+          nfull = rk4_full_steps(Ll, vz, h, A.max_steps, st);
           capped += (st & CTRAJ_ST_CAPPED) ? 1u : 0u;
-          const double hp = Ll / vz - (double)nfull * h;
-          double r2 = __builtin_fma(x, x, y * y);
-          for (int s = 0; s <= nfull; ++s) {
-            if constexpr (GRAD) {
-              if (s % K == 0) put4(W, A.off_ck + cslot + s / K, lane, x, y, vx, vy);
-            }
-            smooth_step(F, T, wsb, SK, s < nfull, hp, x, y, vx, vy, r2, st);
-            r2 = __builtin_fma(x, x, y * y);
-          }
+          hp = Ll / vz - (double)nfull * h;
         }
+        const int nmax = wave_max(nfull);
+        S.end = A.off_end + lens;
+        S.ck = A.off_ck + lens * A.ck_per_lens;
+        if (hex_folds(E.p[4] * scale)) lens_forward<GRAD, true>(L, S, lane, ok, nfull, nmax, hp, x, y, vx, vy);
+        else lens_forward<GRAD, false>(L, S, lane, ok, nfull, nmax, hp, x, y, vx, vy);
         zc = z0 + Ll;
         ++fslot;
-        cslot += A.ck_per_lens;
+        ++lens;
         pidx += 2;
       }
     }
@@ -341,9 +458,9 @@ __global__ void __launch_bounds__(512) k_smooth(KBeam B, KTab KT, SmoothArgs A) 
       double pbx = 0.0, pby = 0.0, vbx = 0.0, vby = 0.0, vzbar = 0.0;
       double zexit_bar = 0.0;  // adjoint of the exit z of the element before the current one
       for (int e = B.n_elems - 1; e >= 0; --e) {
-        const ctraj_elem &E = B.elems[e];
+        const ctraj_elem E = elem_at(B.elems, e);
         pidx -= n_params_of(E);
-        const int pprev = e > 0 ? pidx - n_params_of(B.elems[e - 1]) : 0;
+        const int pprev = e > 0 ? pidx - n_params_of(elem_at(B.elems, e - 1)) : 0;
         const double zprev = exit_z(B, P, e - 1, pprev, A.z_src);
         if (E.kind == CTRAJ_CIRC) {
           const double r = P[pidx];
@@ -375,71 +492,30 @@ __global__ void __launch_bounds__(512) k_smooth(KBeam B, KTab KT, SmoothArgs A) 
           acc_add(a0, a1, a2, pidx, lane, wave_sum(rbar));
           zexit_bar = zfrom_bar;
         } else {  // CTRAJ_LENS
-          const double V = P[pidx], z0 = P[pidx + 1];
+          const double V = uniform_f64(P[pidx]), z0 = uniform_f64(P[pidx + 1]);
           const double scale = V / E.p[7];
-          const double ks = E.p[4] * scale, cu = E.p[5] * scale;
-          const LensK LK{wsb, T.umax, ks, cu, (2.0 * ks) * cu, 1.0 / V, g};
-          const Force<CTRAJ_FORCE_WSPLINE_HEX> F{ks, cu, g, hex_folds(ks) ? -g / ks : 0.0};
+          const LensK L = smooth_lens(E, T, scale, g);
           const double h = E.p[2], Ll = E.p[3];
-          const SmoothStep SK = smooth_step_k(F, h);
           double Vbar = 0.0, z0bar = zexit_bar, zfrom_bar = 0.0;
-          cslot -= A.ck_per_lens;
+          --lens;
           --fslot;
+          int nfull = 0;
+          double hp = 0.0;
           if (ok) {
             uint32_t st = 0;
-            const int nfull = rk4_full_steps(Ll, vz, h, A.max_steps, st);
-            const double hp = Ll / vz - (double)nfull * h;
-            const int ns = nfull + 1;
-            const int nseg = (ns + K - 1) / K;
-            lds_double *rec = (lds_double *)(lds + A.rec_lds) + (threadIdx.x >> 6) * (kSub * 256) + lane;
-            for (int sg = nseg - 1; sg >= 0; --sg) {
-              const int s0 = sg * K, s1 = min(s0 + K, ns);
-              const int nsub = (s1 - s0 + kSub - 1) / kSub;
-              double x, y, vx, vy;
-              get4(W, A.off_ck + cslot + sg, lane, x, y, vx, vy);
-              double r2 = __builtin_fma(x, x, y * y);
-              // the state every kSub steps of the segment (a one-window segment starts from the
-              // checkpoint itself, still in registers)
-              for (int q = 0; q < nsub; ++q) {
-                if (nsub > 1) put4(W, A.off_sub + q, lane, x, y, vx, vy);
-                if (q + 1 < nsub) {
-                  for (int s = s0 + q * kSub; s < s0 + (q + 1) * kSub; ++s) {
-                    smooth_step(F, T, wsb, SK, s < nfull, hp, x, y, vx, vy, r2, st);
-                    r2 = __builtin_fma(x, x, y * y);
-                  }
-                }
-              }
-              // windows, last first: recompute into LDS, then reverse
-              for (int q = nsub - 1; q >= 0; --q) {
-                const int t0 = s0 + q * kSub, t1 = min(t0 + kSub, s1);
-                if (nsub > 1) get4(W, A.off_sub + q, lane, x, y, vx, vy);
-                r2 = __builtin_fma(x, x, y * y);
-                for (int s = t0; s < t1 - 1; ++s) {
-                  lds_double *r = rec + (s - t0) * 256;
-                  r[0] = x;
-                  r[64] = y;
-                  r[128] = vx;
-                  r[192] = vy;
-                  smooth_step(F, T, wsb, SK, s < nfull, hp, x, y, vx, vy, r2, st);
-                  r2 = __builtin_fma(x, x, y * y);
-                }
-                for (int s = t1 - 1; s >= t0; --s) {
-                  if (s < t1 - 1) {
-                    const lds_double *r = rec + (s - t0) * 256;
-                    x = r[0];
-                    y = r[64];
-                    vx = r[128];
-                    vy = r[192];
-                  }
-                  if (s == nfull) {
-                    const double hbar = rk4_adjoint<true>(LK, hp, x, y, vx, vy, pbx, pby, vbx, vby, Vbar);
-                    vzbar = vzbar - hbar * ((Ll / vz) / vz);  // hp = L/vz - nfull h
-                  } else {
-                    (void)rk4_adjoint<false>(LK, h, x, y, vx, vy, pbx, pby, vbx, vby, Vbar);
-                  }
-                }
-              }
-            }
+            nfull = rk4_full_steps(Ll, vz, h, A.max_steps, st);
+            hp = Ll / vz - (double)nfull * h;
+          }
+          const int nmax = wave_max(nfull);
+          S.end = A.off_end + lens;
+          S.ck = A.off_ck + lens * A.ck_per_lens;
+          const double hbar =
+              hex_folds(E.p[4] * scale)
+                  ? lens_reverse<true>(L, S, lane, ok, nfull, nmax, hp, pbx, pby, vbx, vby, Vbar)
+                  : lens_reverse<false>(L, S, lane, ok, nfull, nmax, hp, pbx, pby, vbx, vby, Vbar);
+          if (ok) {
+            Vbar = (Vbar * L.sl) * (1.0 / V);
+            vzbar = vzbar - hbar * ((Ll / vz) / vz);  // hp = L/vz - nfull h
             // drift from the previous exit to the lens entrance z0
             double ex, ey, evx, evy;
             get4(W, fslot, lane, ex, ey, evx, evy);
@@ -461,6 +537,9 @@ __global__ void __launch_bounds__(512) k_smooth(KBeam B, KTab KT, SmoothArgs A) 
     if (lane <= np) out[lane] = a0;
     if (64 + lane <= np) out[64 + lane] = a1;
     if (128 + lane <= np) out[128 + lane] = a2;
+    unsigned long long t = 0;
+    if (lane == 0) t = atomicAdd(A.next, 1ull);
+    item = nwaves + (int64_t)uniform_u64(t);
   }
   if (A.n_capped) {
     const double c = wave_sum((double)capped);
@@ -469,27 +548,27 @@ __global__ void __launch_bounds__(512) k_smooth(KBeam B, KTab KT, SmoothArgs A) 
 }
 
 // J[c] = (sum of item J sums) / n and grad[c][j] = (sum of item sums) / n, each over the items of
-// parameter set c in a fixed order (strided per thread, then a fixed LDS tree).
+// parameter set c = blockIdx.x in a fixed order (strided per thread, then a fixed LDS tree).  One
+// workgroup per sum, j = blockIdx.y (the last is J): a workgroup's time is the latency of its strided
+// loads, so one workgroup for all seven sums of 10^6 molecules took 64 us.
 __global__ void __launch_bounds__(256) k_smooth_reduce(const double *partial, int64_t items_per_cfg, int np, double inv_n,
                                                        double *J, double *grad) {
   __shared__ double red[256];
   const int64_t c = blockIdx.x;
-  const double *base = partial + c * items_per_cfg * (int64_t)(np + 1);
-  for (int j = 0; j <= np; ++j) {
-    if (j < np && !grad) continue;
-    double s = 0.0;
-    for (int64_t it = threadIdx.x; it < items_per_cfg; it += blockDim.x) s += base[it * (np + 1) + j];
-    red[threadIdx.x] = s;
+  const int j = (int)blockIdx.y;
+  if (j < np && !grad) return;
+  const double *base = partial + c * items_per_cfg * (int64_t)(np + 1) + j;
+  double s = 0.0;
+  for (int64_t it = threadIdx.x; it < items_per_cfg; it += blockDim.x) s += base[it * (np + 1)];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int w = blockDim.x >> 1; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
     __syncthreads();
-    for (int w = blockDim.x >> 1; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-      if (j == np) J[c] = red[0] * inv_n;
-      else grad[c * np + j] = red[0] * inv_n;
-    }
-    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    if (j == np) J[c] = red[0] * inv_n;
+    else grad[c * np + j] = red[0] * inv_n;
   }
 }
 
@@ -555,16 +634,24 @@ int32_t ctraj_smooth_objective(ctraj_ctx *c, const ctraj_smooth *s) {
   if (s->ckpt_every < 1) return fail(c, CTRAJ_EINVAL, "ckpt_every must be >= 1");
   if (s->max_steps < 1) return fail(c, CTRAJ_EINVAL, "max_steps must be >= 1");
   const bool grad = s->grad != nullptr;
-  // with gradients, 8 wavefronts per workgroup share the tables and keep 16 KB of LDS each
-  const int block = s->block ? s->block : (grad ? 512 : 256);
-  if (block % 64 || block < 64 || block > 512) return fail(c, CTRAJ_EINVAL, "block must be a multiple of 64 up to 512");
+  const int block_req = s->block;
+  if (block_req % 64 || block_req < 0 || block_req > 512)
+    return fail(c, CTRAJ_EINVAL, "block must be a multiple of 64 up to 512");
   if (nl > 0 && (!c->d_ws || c->ws_states < 1)) return fail(c, CTRAJ_ESTATE, "no W' spline set");
 
   KTab kt = ctx_ktab(c);
   kt.ws_states = nl > 0 ? 1 : 0;  // state 0 only
   kt.rt_total = 0;
   const size_t lds_tab = ktab_lds_bytes(kt);
-  const size_t lds = lds_tab + (grad ? (size_t)(block / 64) * kSub * 256 * sizeof(double) : 0);
+  // with gradients each wavefront keeps a recompute window in LDS beside the tables: 16 wavefronts fit with
+  // one state's 24 KB table, fewer with a longer one
+  const size_t lds_wave = grad ? (size_t)kSub * 256 * sizeof(double) : 0;
+  int block = block_req ? block_req : 256;
+  if (grad && !block_req) {
+    block = 1024;
+    while (block > 64 && lds_tab + (size_t)(block / 64) * lds_wave > (size_t)c->lds_max) block -= 64;
+  }
+  const size_t lds = lds_tab + (size_t)(block / 64) * lds_wave;
   const void *kern = grad ? (const void *)k_smooth<true> : (const void *)k_smooth<false>;
   if ((rc = lds_limit(c, kern, lds)) != CTRAJ_OK) return rc;
   if ((rc = block_ok(c, kern, block)) != CTRAJ_OK) return rc;
@@ -580,26 +667,48 @@ int32_t ctraj_smooth_objective(ctraj_ctx *c, const ctraj_smooth *s) {
   A.sigma_vz = s->sigma_vz;
   A.inv_s = 1.0 / s->softness;
   A.n_params = np;
-  A.K = s->ckpt_every;
   A.max_steps = s->max_steps;
-  A.ck_per_lens = (s->max_steps + 1 + s->ckpt_every - 1) / s->ckpt_every;
-  A.off_ck = nf;
-  A.off_sub = nf + nl * A.ck_per_lens;
-  A.ws_stride = grad ? (int64_t)(A.off_sub + (s->ckpt_every + kSub - 1) / kSub) * 256 : 0;
+  A.off_end = nf;
+  A.off_ck = nf + nl;
+  // rows of 256 doubles per wavefront with checkpoints every K steps
+  auto layout = [&](int K) {
+    A.K = K;
+    A.ck_per_lens = (s->max_steps + K - 1) / K;
+    A.off_sub = A.off_ck + nl * A.ck_per_lens;
+    A.ws_stride = (int64_t)(A.off_sub + (K > kSub ? (K + kSub - 1) / kSub : 0)) * 256;
+  };
   A.rec_lds = (int)(lds_tab / sizeof(double));
 
   const int wpb = block / 64;
   int grid = grid_for(c, kern, block, lds, A.n_items * 64, 0);
   if (grad) {
-    // keep the checkpoint/recompute store within 4 GiB
-    const int64_t per_block = A.ws_stride * 8 * wpb;
-    const int64_t max_blocks = std::max<int64_t>(1, ((int64_t)4 << 30) / per_block);
-    grid = (int)std::min<int64_t>(grid, max_blocks);
-    if ((rc = ensure_buf(c, c->sm_ws, (size_t)per_block * grid)) != CTRAJ_OK) return rc;
+    // Checkpoints every kSub steps leave one window per segment and the fewest steps to recompute; the
+    // store then grows with the steps of the lens (1.1 GB for 4096 wavefronts and 520 steps), so it is
+    // taken while it stays within 2 GiB and can be had, and the caller's interval otherwise
+    const int64_t dense_max = (int64_t)2 << 30, ws_max = (int64_t)4 << 30, grain = (int64_t)64 << 20;
+    layout(std::min(s->ckpt_every, kSub));
+    int64_t per_block = A.ws_stride * 8 * wpb;
+    bool have = false;
+    if (s->ckpt_every <= kSub || per_block * grid <= dense_max) {
+      grid = (int)std::min<int64_t>(grid, std::max<int64_t>(1, ws_max / per_block));
+      rc = ensure_buf(c, c->sm_ws, (size_t)((per_block * grid + grain - 1) / grain * grain));
+      if (rc != CTRAJ_OK && s->ckpt_every <= kSub) return rc;
+      have = rc == CTRAJ_OK;
+    }
+    if (!have) {
+      layout(s->ckpt_every);
+      per_block = A.ws_stride * 8 * wpb;
+      // keep the checkpoint/recompute store within 4 GiB
+      grid = (int)std::min<int64_t>(grid, std::max<int64_t>(1, ws_max / per_block));
+      if ((rc = ensure_buf(c, c->sm_ws, (size_t)per_block * grid)) != CTRAJ_OK) return rc;
+    }
     A.ws = (double *)c->sm_ws.p;
   }
-  if ((rc = ensure_buf(c, c->sm_part, (size_t)A.n_items * (np + 1) * sizeof(double))) != CTRAJ_OK) return rc;
-  A.partial = (double *)c->sm_part.p;
+  // the item counter's 256 bytes, then the partial sums
+  if ((rc = ensure_buf(c, c->sm_part, 256 + (size_t)A.n_items * (np + 1) * sizeof(double))) != CTRAJ_OK) return rc;
+  A.next = (unsigned long long *)c->sm_part.p;
+  A.partial = (double *)((char *)c->sm_part.p + 256);
+  if ((rc = ctraj_fill_i64(c, (int64_t *)A.next, 0, 1)) != CTRAJ_OK) return rc;
 
   const KBeam B = make_kbeam(c->d_elems, c->n_elems, c->phys);
   if (grad)
@@ -607,7 +716,7 @@ int32_t ctraj_smooth_objective(ctraj_ctx *c, const ctraj_smooth *s) {
   else
     hipLaunchKernelGGL(k_smooth<false>, dim3(grid), dim3(block), lds, c->stream, B, kt, A);
   HIPCHK(c, hipGetLastError());
-  hipLaunchKernelGGL(k_smooth_reduce, dim3(s->n_cfg), dim3(256), 0, c->stream, (const double *)A.partial,
+  hipLaunchKernelGGL(k_smooth_reduce, dim3(s->n_cfg, np + 1), dim3(256), 0, c->stream, (const double *)A.partial,
                      A.items_per_cfg, np, 1.0 / (double)s->n, s->J, s->grad);
   HIPCHK(c, hipGetLastError());
   return CTRAJ_OK;

@@ -33,7 +33,8 @@ class SmoothFlux:
     """The objective over a fixed molecule sample on one device.
 
     ``x, y, vx, vy, eps`` are host arrays (uploaded once); ``sigma_vz`` scales eps into vz.
-    ``ckpt_every`` is the lens checkpoint interval K; ``max_steps`` bounds the full RK4 steps per lens
+    ``ckpt_every`` bounds the lens checkpoint interval (the library takes checkpoints more often where
+    memory allows; results do not depend on it); ``max_steps`` bounds the full RK4 steps per lens
     (default: what the slowest molecule of the evaluated parameter sets needs).
 
     The molecules are uploaded in order of eps, hence of vz for every parameter set: each wavefront
