@@ -106,20 +106,21 @@ struct PipeArgs {
   uint32_t *wcount;            // PRE: entries queued by each wavefront (a prefix of its region)
   int64_t region;              // queue entries owned by each PRE wavefront, a multiple of 64
   int n_pre_waves;
-  unsigned long long *claim;   // lens kernel: next unclaimed 64-entry chunk of each region group, [8][32]
+  unsigned long long *claim;   // lens kernel: eight claim counters, [8][32] (zeroed by PRE)
   int lens_e;
-  // claim order (all null: the lens kernel claims the regions in order)
+  // claim list (perm null: the lens kernel claims the regions in order)
+  uint32_t *ord_tot;           // [ORD_BUCKETS] entries per bucket, then the list's entry count
+  uint32_t *perm;              // queue slots in claim order
+  // longest-first order (bkt null: the list holds the slots in queue order)
   uint8_t *bkt;                // PRE: lifetime bucket of each queue entry
   uint32_t *ord_hist;          // PRE: bucket counts of each PRE workgroup [block][ORD_BUCKETS]; k_ord_scan turns
                                // each bucket's column into exclusive prefixes over the workgroups
-  uint32_t *ord_tot;           // [ORD_BUCKETS] entries per bucket, then the queue's total entry count
-  uint32_t *perm;              // queue slots in claim order
   float ord_k2[CTRAJ_MAX_STATES];  // per state: the acceleration per unit radius at the W' table's end
   int ord_ref;                 // the lens integrates in the reference's steps of dz (else of dt)
   // lens tallies (null: the lens kernel writes every molecule back and POST reads every slot): the
   // lens kernel counts the molecules stopped in the lens into this block, which POST adds to the run's
   // tallies under the lens's "inside" label, and lists the slots of those that leave the lens, the
-  // only ones POST then walks.  Words (zeroed before the lens kernel): [LT_N] listed slots,
+  // only ones POST then walks.  Words (zeroed by PRE): [LT_N] listed slots,
   // [LT_STOP + s] stopped molecules of state s, [LT_OOT] / [LT_CAP] out-of-table / capped ones among
   // them, [LT_FIRST] ~(slice index) of the first of them (0: none); the list from word LT_LIST.
   uint32_t *lt;
@@ -242,6 +243,12 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
   int lens_hit = 0;
   float ord_bore2 = 0.0f, ord_len = 0.0f, ord_h = 0.0f, ord_cap = 0.0f;  // lifetime prediction (P.bkt)
   if constexpr (PHASE == PHASE_PRE) {
+    // the words that this launch's lens kernel counts in (the previous launch's kernels are done with them)
+    if (blockIdx.x == 0) {
+      for (int k = threadIdx.x; k < 8; k += blockDim.x) P.claim[32 * k] = 0;
+      if (P.lt)
+        for (int k = threadIdx.x; k < LT_LIST; k += blockDim.x) P.lt[k] = 0;
+    }
     const ctraj_elem L = elem_at(B.elems, P.lens_e);
     lens_z0 = L.z0;
     lens_r = L.p[0];
@@ -710,39 +717,43 @@ __global__ void __launch_bounds__(768) k_propagate_lanes(KBeam B, KTab KT, const
 
 // ---------------------------------------------------------------------------------------------
 // k_lens: integration of the lens-entry queue.  Persistent wavefronts keep their lanes busy by
-// lane refill: every iteration advances the lanes that take full steps by one step; when at least
-// `refill_min` lanes do not, or none does, a convergent section finishes the molecules that stopped
-// taking full steps -- those that reached the end of the lens take the final partial step
-// (configuration mode) or the exit hop with the stored a = l1 (reference mode) -- writes each
-// finished molecule's state back into its queue entry with its outcome (queue_put_done), and gives
-// the empty lanes the next queued molecules.  A lane's rem is its full steps left (> 0: it takes
-// steps; 0: it reached the end of the lens), REM_EMPTY when it holds no molecule, and at most
-// REM_STOPPED once the bore stopped it: -2 - k after its k-th full step in configuration mode (the
-// lane forms z and t from k when it finishes, not step by step), REM_STOPPED in reference mode; so
-// one compare per iteration gives both the step's lane mask and the refill count, and a step updates
-// rem with one compare, one select and one subtraction.  Finished molecules are walked
-// through the remaining elements and recorded by POST, so the refill section carries no element
-// walk and no recording.  Wavefronts claim the queue in 64-entry chunks, region by region, from
-// eight counters: counter g serves the regions of the PRE workgroups dispatched to XCD g
-// (workgroup b runs on XCD b mod 8), and a wavefront starts with its own XCD's counter and moves to
-// the next one when it runs dry, which spreads the claim atomics over eight addresses.  Chunk c of
-// group g is entries [64 (c % cpr), +64) of the group's region c / cpr (cpr = region / 64), of
-// which the first wcount are filled, so a claim needs no search and a chunk past a region's count
-// is simply claimed over.  With a claim list (longest-lived first, see ORD_BUCKETS) counter g hands
-// out the list's chunks g, g + 8, g + 16, ... instead.  The per-molecule arithmetic is the one of
-// walk().
+// lane refill.  The lanes that take full steps are a scalar mask; a step loop advances them until at
+// least `refill_min` lanes are idle (or, once nothing is left to claim, until none is busy), then a
+// convergent section finishes the molecules that stopped taking full steps -- those that reached the
+// end of the lens take the final partial step (configuration mode) or the exit hop with the stored
+// a = l1 (reference mode) -- writes each finished molecule's state back into its queue entry with its
+// outcome (queue_put_done), and gives the empty lanes the next queued molecules.  A lane's rem is 1
+// while it takes full steps, 0 at the end of the lens, REM_EMPTY when it holds no molecule, and
+// REM_STOPPED - k once the bore stopped it after its k-th full step (configuration mode forms z and t
+// from k when it finishes, not step by step).  The loop counts its iterations: a lane knows the one that
+// ends its full steps, so a step costs two compares, and the lane's own bookkeeping runs only when a
+// molecule ends.  Finished molecules are walked through the remaining elements and recorded by POST,
+// so the section carries no element walk and no recording.
+//
+// The queue is claimed in chunks of 64 entries, of the claim list (LIST) or of a region.
+// Wavefront w of workgroup b starts with chunk w * gridDim + b, so that few chunks go to as many CUs
+// and SIMDs as there are; the rest come from eight counters (counter g: chunks W + g, W + g + 8, ... of
+// the W wavefronts' launch), which spreads the claim atomics over eight addresses: a wavefront starts
+// with its own XCD's (workgroup b runs on XCD b mod 8) and moves to the next one when it runs dry.
+// The list matters where few molecules reach the lens (the reference's example: 5.3e3 of 10^6, one or two in
+// each region): their wavefronts are full, and so few that each has a SIMD to itself, where claiming the
+// regions put 16 wavefronts of one or two molecules on every CU (2.58 -> 0.83 ms).  Fewer than 64 entries a
+// chunk, so that every SIMD gets a wavefront, measured the same.
+// What bounds the kernel: VALU issue with many molecules (72 instructions a step at eight wavefronts per SIMD,
+// issuing on 95 % of the cycles), the latency of one molecule's steps with few.  The step loop's condition and
+// mask are scalar and its exit is the rare path: 10^4 molecules 188 -> 120 us (430 serial steps), 10^7
+// 2.82 -> 2.75 ms.
+// The per-molecule arithmetic is the one of walk().
 // ---------------------------------------------------------------------------------------------
 
 // The hexapole RK4 instantiations are held to 64 VGPRs (eight wavefronts per SIMD), so the host's
-// 1024-thread workgroups run two per CU beside two copies of one state's 24 KB table.  They fit
-// without spilling vector registers; the two scalar registers they spill are reloaded after the
-// lens loop only.  Unheld, the scheduler spends up to 72 on the lens end's partial step (the step
-// loop itself needs 64), which would leave one workgroup per CU.  The others need more registers
-// than that.
+// 1024-thread workgroups run two per CU beside two copies of one state's 24 KB table.  Unheld, the
+// scheduler spends up to 72 on the lens end's partial step, which would leave one workgroup per CU.
+// The others need more registers than that.
 constexpr int REM_EMPTY = -1, REM_STOPPED = -2;
 
-// ORD: the wavefronts claim the list P.perm (longest-lived first) instead of the regions in order.
-template <int FORCE, int INTEG, bool ORD>
+// LIST: the wavefronts claim the list P.perm instead of the regions in order.
+template <int FORCE, int INTEG, bool LIST>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(
     FORCE == CTRAJ_FORCE_WSPLINE_HEX && INTEG == CTRAJ_INTEG_RK4 ? 8 : 1)))
 k_lens(KBeam B, KTab KT, PipeArgs P, int refill_min, StepK K, unsigned long long *work) {
@@ -756,17 +767,14 @@ k_lens(KBeam B, KTab KT, PipeArgs P, int refill_min, StepK K, unsigned long long
   if (LT && threadIdx.x <= LT_FIRST) s_lt[threadIdx.x] = 0;
   const Tables T = stage_tables(lds, KT);
   __syncthreads();
-  // eight claim counters: counter g serves the regions of one XCD's PRE workgroups (n_chunks over
-  // cpr chunks per region) or, with the claim list, the list's chunks g, g + 8, g + 16, ...
-  const uint32_t cpr = ORD ? 0u : (uint32_t)(P.region >> 6);
-  const uint32_t n_q = ORD ? P.ord_tot[ORD_BUCKETS] : 0u;
-  // chunks: per counter, its group's regions x cpr; with the list, the list's ceil(n_q / 64) (counter
-  // g's claim c is chunk c * 8 + g)
-  const unsigned long long n_chunks =
-      ORD ? (unsigned long long)((n_q + 63u) >> 6) : (unsigned long long)(P.n_pre_waves >> 3) * cpr;
+  const int lane = lane_id();
+  const uint32_t n_waves = gridDim.x * (blockDim.x >> 6);
+  const uint32_t cpr = LIST ? 1u : (uint32_t)(P.region >> 6);  // chunks per region
+  const uint32_t n_q = LIST ? P.ord_tot[ORD_BUCKETS] : 0u;
+  const uint32_t n_chunks = LIST ? (n_q + 63u) >> 6 : (uint32_t)P.n_pre_waves * cpr;
+  uint32_t chunk = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * gridDim.x + blockIdx.x;
   int grp = blockIdx.x & 7, tried = 0;
 
-  const int lane = lane_id();
   const ctraj_elem &L0 = B.elems[P.lens_e];
   const Force<FORCE> F = make_force<FORCE>(L0, B.g);
   // the lens: z1, bore (x^2 + y^2 beyond R2 stops a molecule: (d/2)^2 for RK4, the squared-radius
@@ -776,150 +784,167 @@ k_lens(KBeam B, KTab KT, PipeArgs P, int refill_min, StepK K, unsigned long long
   const double R2 = L0.p[1], z1 = L0.z1, Hs = L0.p[2], Ll = L0.p[3];
   const int n_ref = L0.n_steps;
   uint32_t steps_w = 0, faces_w = 0;  // wave-uniform counts
-  int64_t next = 0, end = 0;
-  bool exhausted = false;
+  uint32_t next = 0, end = 0;         // the claimed chunk's unassigned entries
+  bool claimed = false, exhausted = chunk >= n_chunks;
 
   // lane state: the molecule (configuration mode: z and t stay at their entry values until the lane
   // finishes; reference mode: they advance with the steps; vz is constant in the lens), its queue
-  // entry and key, rem (see above), its full-step count plus 3 (configuration mode) or the step dt
+  // entry and key, rem (see above), its full-step count, the iteration that ends it, the step dt
   // (reference mode), and its state table
   MState m;
   m.x = m.y = m.z = m.vx = m.vy = m.vz = m.t = 0.0;
   m.ax = 0.0; m.ay = -B.g; m.az = 0.0;
   double r2 = 0.0, h = 0.0;
-  int rem = REM_EMPTY, nfull3 = 0;
-  uint32_t status = 0;
-  int64_t slot = 0, key = 0;
+  int rem = REM_EMPTY, nfull = 0;
+  uint32_t ends_at = 0, it = 0;
+  uint32_t status = 0, slot = 0;
+  int64_t key = 0;
   WsRef wsb = ws_of(T, 0);
 
   for (;;) {
-    bool act = rem > 0;
-    uint64_t am = __builtin_amdgcn_ballot_w64(act);
-    if (64 - __popcll(am) >= refill_min) {
-      for (;;) {
-        // finish the molecules that hold a lane but take no more full steps: stopped by the bore, or
-        // at the end of the lens, which takes one more step (configuration mode) or the exit hop
-        // (reference mode)
-        const bool fin = rem == 0 || rem <= REM_STOPPED;
-        const bool dead = rem <= REM_STOPPED;
-        const uint64_t ends = __builtin_amdgcn_ballot_w64(rem == 0);
-        if constexpr (INTEG == CTRAJ_INTEG_RK4) steps_w += (uint32_t)__popcll(ends);
-        else faces_w += (uint32_t)__popcll(ends);
-        if (fin) {
-          int outcome = LENS_STOPPED;
-          if constexpr (INTEG == CTRAJ_INTEG_RK4) {
-            if (!dead) {  // the end of the lens: one partial step of L/vz - n dt, so the lens ends at z1
-              const int nfull = nfull3 - 3;
-              const double hp = Ll / m.vz - (double)nfull * Hs;
-              if constexpr (FORCE == CTRAJ_FORCE_WSPLINE_HEX) {  // the host launches only folding lenses here
-                rk4_step_hex_k(wsb, T.umax, F.cu, K.gk, hex_k(F.ks, hp), m.x, m.y, m.vx, m.vy, r2);
-              } else {
-                rk4_step<FORCE>(F, T, wsb, hp, m.x, m.y, m.vx, m.vy, r2, status);
-              }
-              m.z = z1;
-              m.t = __builtin_fma((double)nfull, Hs, m.t) + hp;
-              r2 = __builtin_fma(m.x, m.x, m.y * m.y);
-              outcome = r2 > R2 ? LENS_STOPPED : LENS_LEFT;
-            } else {  // stopped by the bore after k full steps: z and t from their entry values
-              const double k = (double)(REM_STOPPED - rem);
-              m.z = __builtin_fma(k, m.vz * Hs, m.z);
-              m.t = __builtin_fma(k, Hs, m.t);
+    for (;;) {
+      // finish the molecules that hold a lane but take no more full steps: stopped by the bore, or
+      // at the end of the lens, which takes one more step (configuration mode) or the exit hop
+      // (reference mode)
+      const bool fin = rem == 0 || rem <= REM_STOPPED;
+      const bool dead = rem <= REM_STOPPED;
+      const uint64_t ends = __builtin_amdgcn_ballot_w64(rem == 0);
+      if constexpr (INTEG == CTRAJ_INTEG_RK4) steps_w += (uint32_t)__popcll(ends);
+      else faces_w += (uint32_t)__popcll(ends);
+      if (fin) {
+        int outcome = LENS_STOPPED;
+        if constexpr (INTEG == CTRAJ_INTEG_RK4) {
+          if (!dead) {  // the end of the lens: one partial step of L/vz - n dt, so the lens ends at z1
+            const double hp = Ll / m.vz - (double)nfull * Hs;
+            if constexpr (FORCE == CTRAJ_FORCE_WSPLINE_HEX) {  // the host launches only folding lenses here
+              rk4_step_hex_k(wsb, T.umax, F.cu, K.gk, hex_k(F.ks, hp), m.x, m.y, m.vx, m.vy, r2);
+            } else {
+              rk4_step<FORCE>(F, T, wsb, hp, m.x, m.y, m.vx, m.vy, r2, status);
             }
-          } else {
-            if (!dead) {  // exit hop with the stored a = l1 of the last step (electrostatic_lens.py:74-77)
-              drift_dt(m, time_to(m, z1), B.g);
-              outcome = LENS_LEFT;
-            }
+            m.z = z1;
+            m.t = __builtin_fma((double)nfull, Hs, m.t) + hp;
+            r2 = __builtin_fma(m.x, m.x, m.y * m.y);
+            outcome = r2 > R2 ? LENS_STOPPED : LENS_LEFT;
+          } else {  // stopped by the bore after k full steps: z and t from their entry values
+            const double k = (double)(REM_STOPPED - rem);
+            m.z = __builtin_fma(k, m.vz * Hs, m.z);
+            m.t = __builtin_fma(k, Hs, m.t);
           }
-          if (LT && P.lt && outcome == LENS_STOPPED) {
-            // lens tallies: the molecule is counted here and needs no further walk
-            atomicAdd(&s_lt[LT_STOP + (int)((uint64_t)key >> 56)], 1u);
-            atomicMax(&s_lt[LT_FIRST], ~(uint32_t)key);  // slice index < 2^32
-            if (status) {
-              if (status & CTRAJ_ST_OOT) atomicAdd(&s_lt[LT_OOT], 1u);
-              if (status & CTRAJ_ST_CAPPED) atomicAdd(&s_lt[LT_CAP], 1u);
-            }
-          } else {
-            queue_put_done(P.q, slot, m.x, m.y, m.z, m.vx, m.vy, m.vz, m.t,
-                           key | ((int64_t)status << 40) | ((int64_t)outcome << 48));
-            if (LT && P.lt) {  // list the slot for POST: one atomic per wavefront, by its first lane here
-              const uint64_t lm = __builtin_amdgcn_ballot_w64(true);
-              const int rank = lanes_below(lm);
-              uint32_t base = 0;
-              if (rank == 0) base = atomicAdd(&P.lt[LT_N], (uint32_t)__popcll(lm));
-              base = __builtin_amdgcn_readfirstlane(base);
-              P.lt[LT_LIST + base + (uint32_t)rank] = (uint32_t)slot;
-            }
+        } else {
+          if (!dead) {  // exit hop with the stored a = l1 of the last step (electrostatic_lens.py:74-77)
+            drift_dt(m, time_to(m, z1), B.g);
+            outcome = LENS_LEFT;
           }
-          rem = REM_EMPTY;
         }
-        const uint64_t need = __builtin_amdgcn_ballot_w64(rem == REM_EMPTY);
-        if (!need || exhausted) break;
-        if (next >= end) {
+        if (LT && P.lt && outcome == LENS_STOPPED) {
+          // lens tallies: the molecule is counted here and needs no further walk
+          atomicAdd(&s_lt[LT_STOP + (int)((uint64_t)key >> 56)], 1u);
+          atomicMax(&s_lt[LT_FIRST], ~(uint32_t)key);  // slice index < 2^32
+          if (status) {
+            if (status & CTRAJ_ST_OOT) atomicAdd(&s_lt[LT_OOT], 1u);
+            if (status & CTRAJ_ST_CAPPED) atomicAdd(&s_lt[LT_CAP], 1u);
+          }
+        } else {
+          queue_put_done(P.q, slot, m.x, m.y, m.z, m.vx, m.vy, m.vz, m.t,
+                         key | ((int64_t)status << 40) | ((int64_t)outcome << 48));
+          if (LT && P.lt) {  // list the slot for POST: one atomic per wavefront, by its first lane here
+            const uint64_t lm = __builtin_amdgcn_ballot_w64(true);
+            const int rank = lanes_below(lm);
+            uint32_t base = 0;
+            if (rank == 0) base = atomicAdd(&P.lt[LT_N], (uint32_t)__popcll(lm));
+            base = __builtin_amdgcn_readfirstlane(base);
+            P.lt[LT_LIST + base + (uint32_t)rank] = slot;
+          }
+        }
+        rem = REM_EMPTY;
+      }
+      const uint64_t need = __builtin_amdgcn_ballot_w64(rem == REM_EMPTY);
+      if (!need || exhausted) break;
+      if (next >= end) {
+        if (claimed) {
+          if (n_chunks <= n_waves) {  // every chunk was some wavefront's first
+            exhausted = true;
+            continue;
+          }
           unsigned long long c = 0;
           if (lane == 0) c = atomicAdd(P.claim + 32 * grp, 1ull);
           c = uniform_u64(c);  // every lane is active here, lane 0 first
-          if (ORD ? c * 8 + (unsigned)grp >= n_chunks : c >= n_chunks) {
+          const unsigned long long ch = n_waves + c * 8 + (unsigned)grp;
+          if (ch >= n_chunks) {
             if (++tried == 8) exhausted = true;
             grp = (grp + 1) & 7;
             continue;
           }
-          if constexpr (ORD) {
-            next = (int64_t)(c * 8 + (unsigned)grp) * 64;
-            end = next + 64 < (int64_t)n_q ? next + 64 : (int64_t)n_q;
-          } else {
-            const uint32_t r = (uint32_t)c / cpr;
-            const uint32_t w = ((r >> 2) << 5) | ((uint32_t)grp << 2) | (r & 3u);
-            const int64_t base = (int64_t)((uint32_t)c - r * cpr) * 64;
-            const int64_t filled = (int64_t)P.wcount[w] - base;
-            next = (int64_t)w * P.region + base;
-            end = next + (filled < 64 ? filled : 64);  // next >= end: an empty chunk, claim again
-          }
-          continue;
+          chunk = (uint32_t)ch;
         }
-        const int64_t avail = end - next;
-        if (rem == REM_EMPTY) {
-          const int rank = lanes_below(need);
-          if (rank < avail) {
-            slot = next + rank;
-            if constexpr (ORD) slot = P.perm[slot];
-            queue_get_done(P.q, slot, m, key);
-            m.ax = 0.0;  // the lens entrance row stores (0, -g, 0)
-            m.ay = -B.g;
-            m.az = 0.0;
-            wsb = ws_of(T, (int)((uint64_t)key >> 56));
-            status = 0;
-            if constexpr (INTEG == CTRAJ_INTEG_RK4) {
-              rem = rk4_full_steps(Ll, m.vz, Hs, B.cap, status);
-              nfull3 = rem + 3;
-              r2 = __builtin_fma(m.x, m.x, m.y * m.y);
-            } else {
-              rem = n_ref;
-              h = Hs / m.vz;  // dt = dz / v_z (electrostatic_lens.py:88)
-            }
-          }
+        claimed = true;
+        if constexpr (LIST) {
+          next = chunk * 64u;
+          end = min(next + 64u, n_q);
+        } else {
+          const uint32_t w = chunk / cpr;
+          const uint32_t base = (chunk - w * cpr) * 64u;
+          const uint32_t filled = P.wcount[w];
+          next = (uint32_t)(w * P.region) + base;
+          end = next + (filled > base ? min(filled - base, 64u) : 0u);  // next >= end: an empty chunk, claim again
         }
-        next += avail < (int64_t)__popcll(need) ? avail : (int64_t)__popcll(need);
+        continue;
       }
-      act = rem > 0;
-      am = __builtin_amdgcn_ballot_w64(act);
-      if (!am) break;  // the queue is exhausted and every molecule has been finished
+      const uint32_t avail = end - next;
+      if (rem == REM_EMPTY) {
+        const uint32_t rank = (uint32_t)lanes_below(need);
+        if (rank < avail) {
+          slot = next + rank;
+          if constexpr (LIST) slot = P.perm[slot];
+          queue_get_done(P.q, slot, m, key);
+          m.ax = 0.0;  // the lens entrance row stores (0, -g, 0)
+          m.ay = -B.g;
+          m.az = 0.0;
+          wsb = ws_of(T, (int)((uint64_t)key >> 56));
+          status = 0;
+          if constexpr (INTEG == CTRAJ_INTEG_RK4) {
+            nfull = rk4_full_steps(Ll, m.vz, Hs, B.cap, status);
+            r2 = __builtin_fma(m.x, m.x, m.y * m.y);
+          } else {
+            nfull = n_ref;
+            h = Hs / m.vz;  // dt = dz / v_z (electrostatic_lens.py:88)
+          }
+          rem = nfull > 0 ? 1 : 0;
+          ends_at = it + (uint32_t)nfull;
+        }
+      }
+      next += min(avail, (uint32_t)__popcll(need));
     }
 
-    steps_w += (uint32_t)__popcll(am);
-    if (act) {
+    uint64_t am = __builtin_amdgcn_ballot_w64(rem > 0);  // the lanes that take full steps
+    if (!am) break;  // the queue is exhausted and every molecule has been finished
+    uint32_t cnt = (uint32_t)__popcll(am);
+    // idle lanes wait for a refill only while there is something to claim
+    const uint32_t keep = __builtin_amdgcn_readfirstlane(exhausted ? 0 : 64 - refill_min);
+    do {
+      steps_w += cnt;
+      ++it;
+      bool out;  // beyond the bore (lanes outside am: whatever)
       if constexpr (INTEG == CTRAJ_INTEG_RK4) {
-        if constexpr (FORCE == CTRAJ_FORCE_WSPLINE_HEX)  // the host launches only folding lenses here
-          rk4_step_hex_k(wsb, T.umax, F.cu, K.gk, K.hk, m.x, m.y, m.vx, m.vy, r2);
-        else
-          rk4_step_k<FORCE>(F, T, wsb, K.h1, m.x, m.y, m.vx, m.vy, r2, status);
-        r2 = __builtin_fma(m.x, m.x, m.y * m.y);
-        rem = rem - (r2 > R2 ? nfull3 : 1);  // stopped after its k-th step: -2 - k
+        if (lane_in(am)) {
+          if constexpr (FORCE == CTRAJ_FORCE_WSPLINE_HEX)  // the host launches only folding lenses here
+            rk4_step_hex_k(wsb, T.umax, F.cu, K.gk, K.hk, m.x, m.y, m.vx, m.vy, r2);
+          else
+            rk4_step_k<FORCE>(F, T, wsb, K.h1, m.x, m.y, m.vx, m.vy, r2, status);
+          r2 = __builtin_fma(m.x, m.x, m.y * m.y);
+        }
+        out = r2 > R2;
       } else {
-        ref_step<FORCE>(F, T, wsb, h, m, status);  // the row stores a = l1
-        rem = beyond_r2(m.x, m.y, R2) ? REM_STOPPED : rem - 1;  // R2: the threshold of d/2 (lens_ref)
+        if (lane_in(am)) ref_step<FORCE>(F, T, wsb, h, m, status);  // the row stores a = l1
+        out = beyond_r2(m.x, m.y, R2);  // R2: the threshold of d/2 (lens_ref)
       }
-    }
+      const uint64_t over = am & (__builtin_amdgcn_ballot_w64(out) | __builtin_amdgcn_ballot_w64(ends_at == it));
+      if (over) {
+        if (lane_in(over)) rem = out ? REM_STOPPED - (int)(it - ends_at + (uint32_t)nfull) : 0;
+        am &= ~over;
+        cnt = (uint32_t)__popcll(am);
+      }
+    } while (cnt > keep);
   }
 
   if (work || (LT && P.lt)) {  // kernel arguments: every thread takes the same branch
@@ -1327,14 +1352,9 @@ static PropFn prop_kernel(int f, int i, bool has_lens, int km, bool out, bool mi
   return nullptr;
 }
 
-static LensFn lens_kernel(int f, int i, bool ord) {
-  if (ord) {  // the claim list is built for hexapole lenses only
-    if (f == CTRAJ_FORCE_WSPLINE_HEX && i == CTRAJ_INTEG_RK4) return k_lens<CTRAJ_FORCE_WSPLINE_HEX, CTRAJ_INTEG_RK4, true>;
-    if (f == CTRAJ_FORCE_WSPLINE_HEX && i == CTRAJ_INTEG_REF) return k_lens<CTRAJ_FORCE_WSPLINE_HEX, CTRAJ_INTEG_REF, true>;
-    return nullptr;
-  }
+static LensFn lens_kernel(int f, int i, bool list) {
 #define X(F, I) \
-  if (f == F && i == I) return k_lens<F, I, false>;
+  if (f == F && i == I) return list ? k_lens<F, I, true> : k_lens<F, I, false>;
   CT_FI_LIST(X)
 #undef X
   return nullptr;
@@ -1494,11 +1514,15 @@ static int32_t propagate_impl(ctraj_ctx *c, const ctraj_run *R, char *sdev) {
     pev = c->pt_ev[slot];
   }
   if (pipeline) {
-    // claim order, longest-lived first: hexapole lenses (whose W' table gives the prediction's force
-    // scale), unless the run asks for queue order; the scratch array of the allocation-free entry
-    // point holds no room for it
-    const bool ordered = !sdev && c->force == CTRAJ_FORCE_WSPLINE_HEX && !(R->flags & CTRAJ_RUN_QUEUE_ORDER);
-    LensFn kl = lens_kernel(c->force, c->integ, ordered);
+    // The claim list.  While every SIMD gets at most one wavefront of the queue's regions, the regions are
+    // claimed as they are: no order helps then, and the list kernels would only add their launches.
+    // Beyond that a list packs the molecules into full chunks: longest-lived first for hexapole lenses
+    // (whose W' table gives the prediction's force scale), else, or where the run asks for it, in queue
+    // order.  The scratch array of the allocation-free entry point holds no room for a list.
+    const bool few = R->n <= (int64_t)64 * 4 * c->n_cu;
+    const bool list = !sdev && !few;
+    const bool ordered = list && c->force == CTRAJ_FORCE_WSPLINE_HEX && !(R->flags & CTRAJ_RUN_QUEUE_ORDER);
+    LensFn kl = lens_kernel(c->force, c->integ, list);
     if (!kl) return fail(c, CTRAJ_EINVAL, "no kernel for this force/integrator");
     const bool out = wants_outputs(R);
     // lens tallies: for a hexapole lens in RK4 steps, without per-molecule outputs, and unless the
@@ -1560,16 +1584,20 @@ static int32_t propagate_impl(ctraj_ctx *c, const ctraj_run *R, char *sdev) {
     const int64_t threads = (int64_t)gpre * blk;
     P.n_pre_waves = gpre * (blk / 64);
     P.lens_e = lens_e;
-    if (ordered) {
+    if (list) {
       const size_t cap = (size_t)threads * (size_t)((slice + threads - 1) / threads);
-      const size_t b_bkt = (cap + 255) & ~(size_t)255, b_perm = cap * 4, b_tot = 2048;
-      const size_t b_hist = (size_t)gpre * ORD_BUCKETS * 4;
+      const size_t b_bkt = ordered ? (cap + 255) & ~(size_t)255 : 0, b_perm = cap * 4, b_tot = 2048;
+      const size_t b_hist = ordered ? (size_t)gpre * ORD_BUCKETS * 4 : 0;
       if ((rc = ensure_buf(c, c->ord, b_bkt + b_perm + b_tot + b_hist)) != CTRAJ_OK) return rc;
       char *o = (char *)c->ord.p;
       P.ord_tot = (uint32_t *)o;
-      P.ord_hist = (uint32_t *)(o + b_tot);
       P.perm = (uint32_t *)(o + b_tot + b_hist);
-      P.bkt = (uint8_t *)(o + b_tot + b_hist + b_perm);
+      if (ordered) {
+        P.ord_hist = (uint32_t *)(o + b_tot);
+        P.bkt = (uint8_t *)(o + b_tot + b_hist + b_perm);
+      }
+    }
+    if (ordered) {
       const double ks = c->h_elems[lens_e].p[4];
       for (int st = 0; st < c->ws_states && st < CTRAJ_MAX_STATES; ++st) P.ord_k2[st] = (float)(ks * c->ws_end[st]);
       P.ord_ref = c->integ == CTRAJ_INTEG_REF;
@@ -1577,15 +1605,16 @@ static int32_t propagate_impl(ctraj_ctx *c, const ctraj_run *R, char *sdev) {
     // refill at 10 idle lanes by default (a sweep of 6-16 on the 10^7-molecule ES-lens run: 10 and
     // 12 fastest, 3 % ahead of 8)
     const int refill = R->refill > 0 ? std::min(R->refill, 64) : 10;
-    const int grid = grid_for(c, (const void *)kl, block, lds, (int64_t)1 << 40, 0);
+    // few molecules: one workgroup of four wavefronts per CU at most
+    const int blk_lens = few && !R->block ? 256 : block;
+    int grid = grid_for(c, (const void *)kl, blk_lens, lds, (int64_t)1 << 40, 0);
+    if (few && !R->block) grid = std::min(grid, std::max(1, std::min(c->n_cu, P.n_pre_waves)));
     const StepK K = step_k(c->h_elems[lens_e].p[2], c->h_elems[lens_e].p[4], c->phys.g);
     const bool one_slice = slice >= R->n;
     for (int64_t s0 = 0; s0 < R->n; s0 += slice) {
       const int64_t len = std::min(slice, R->n - s0);
       const ctraj_run S = slice_of(*R, s0, len);
       P.region = (len + threads - 1) / threads * 64;
-      if ((rc = ctraj_fill_i64(c, (int64_t *)P.claim, 0, 8 * 32)) != CTRAJ_OK) return rc;
-      if (P.lt && (rc = ctraj_fill_i64(c, (int64_t *)P.lt, 0, LT_LIST / 2)) != CTRAJ_OK) return rc;
       if (pev && s0 == 0) HIPCHK(c, hipEventRecord(pev[0], c->stream));
       hipLaunchKernelGGL(kpre, dim3(gpre), dim3(blk), lds_aoi, c->stream, B, kt, S, 0, P);
       HIPCHK(c, hipGetLastError());
@@ -1594,9 +1623,13 @@ static int32_t propagate_impl(ctraj_ctx *c, const ctraj_run *R, char *sdev) {
         hipLaunchKernelGGL(k_ord_scatter, dim3(gpre), dim3(256), 0, c->stream,
                            OrdList{P.bkt, P.ord_hist, P.ord_tot, P.perm, P.wcount, P.region});
         HIPCHK(c, hipGetLastError());
+      } else if (list) {
+        hipLaunchKernelGGL(k_list, dim3(gpre), dim3(256), 0, c->stream, (const uint32_t *)P.wcount, P.region,
+                           P.ord_tot, P.perm);
+        HIPCHK(c, hipGetLastError());
       }
       if (pev && one_slice) HIPCHK(c, hipEventRecord(pev[1], c->stream));
-      hipLaunchKernelGGL(kl, dim3(grid), dim3(block), lds, c->stream, B, kt, P, refill, K,
+      hipLaunchKernelGGL(kl, dim3(grid), dim3(blk_lens), lds, c->stream, B, kt, P, refill, K,
                          (unsigned long long *)R->work);
       HIPCHK(c, hipGetLastError());
       if (pev && one_slice) HIPCHK(c, hipEventRecord(pev[2], c->stream));

@@ -1,4 +1,4 @@
-// ctraj_order.hpp -- the lens kernels' claim list: longest predicted lens time first.
+// ctraj_order.hpp -- the lens kernels' claim list: longest predicted lens time first, or queue order.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -191,4 +191,24 @@ static __global__ void __launch_bounds__(256) k_ord_scatter(OrdList P) {
     __syncthreads();
     for (uint32_t k = t; k < m; k += 256) P.perm[s_pos[k]] = s_slot[k];
   }
+}
+
+// The claim list in queue order: the filled slots of the regions without their gaps.  Workgroup b
+// (256 threads) lists its four wavefronts' regions from the position that the counts before them give
+// (at most a few thousand counts, read by every workgroup); the last one leaves the total.
+static __global__ void __launch_bounds__(256) k_list(const uint32_t *wcount, int64_t region, uint32_t *tot,
+                                                     uint32_t *perm) {
+  __shared__ uint32_t s[256];
+  const int t = threadIdx.x;
+  const uint32_t w0 = blockIdx.x * 4u;
+  uint32_t v = 0;
+  for (uint32_t w = t; w < w0; w += 256) v += wcount[w];
+  uint32_t pos;
+  (void)block_excl_scan256(v, s, &pos);
+  for (uint32_t w = w0; w < w0 + 4; ++w) {
+    const uint32_t c = wcount[w];
+    for (uint32_t k = t; k < c; k += 256) perm[pos + k] = (uint32_t)(w * region) + k;
+    pos += c;
+  }
+  if (blockIdx.x == gridDim.x - 1 && t == 0) tot[ORD_BUCKETS] = pos;
 }

@@ -42,6 +42,9 @@ __device__ __forceinline__ int lanes_below(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
+// This lane's bit of a wave-uniform mask, as a condition that costs no vector instruction.
+__device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
 // A lens-entry queue entry is 64 bytes, four 16-byte vectors: (x, y) (z, vx) (vy, vz) (t, key) with
 // key = molecule index within the slice (bits 0-39) | status bits << 40 | lens outcome << 48 | lens state
 // << 56; the walk to the lens queues a molecule with status and outcome 0, and the lens kernel writes
