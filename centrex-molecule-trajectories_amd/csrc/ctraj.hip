@@ -1208,7 +1208,8 @@ double circ_r2_threshold(double d) {
 // so does a reference-mode lens for its bore test (its p[1] has no other use; configuration mode
 // compares x^2 + y^2 with (d/2)^2 itself); an RTABLE lens carries its table's knot offset (table),
 // knot count (reserved), inverse knot spacing (p[6]) and first and last knots (p[4], p[5], which
-// only the spline forces use) instead of the table id.
+// only the spline forces use) instead of the table id, and whether the table allows the fast reference
+// step (p[7], otherwise the electrode voltage, which no table lens uses).
 void resolve_elems(const ctraj_ctx *ctx, const ctraj_elem *e, int n, ctraj_elem *out) {
   for (int i = 0; i < n; ++i) {
     out[i] = e[i];
@@ -1222,6 +1223,11 @@ void resolve_elems(const ctraj_ctx *ctx, const ctraj_elem *e, int n, ctraj_elem 
       const std::vector<double> &tb = ctx->rt_host[id];
       out[i].p[4] = tb.empty() ? 0.0 : tb[0];
       out[i].p[5] = tb.empty() ? 0.0 : tb[tb.size() - 4];
+      // ref_step's fast form: every knot, value, slope and g zero or of moderate size
+      auto moderate = [](double v) { return v == 0.0 || tame_value(v); };
+      bool tame = moderate(ctx->phys.g);
+      for (double v : tb) tame = tame && moderate(v);
+      out[i].p[7] = tame ? 1.0 : 0.0;
     }
   }
 }
