@@ -815,9 +815,9 @@ int32_t ctraj_batch_create(ctraj_ctx *c, const ctraj_elem *elems, int32_t n_elem
     b->region = (slice + threads - 1) / threads * 64;
     // the queue, then the lens kernel's count and list of the molecules that leave their lens
     const size_t qbytes = (size_t)b->n_pre_waves * (size_t)b->region * (64 + 4) + 4 * BLT_LIST;
-    if (hipMalloc((void **)&b->d_lensk, sizeof(BLensC) * n_cfgs) != hipSuccess ||
-        hipMalloc(&b->d_pipe, qbytes) != hipSuccess ||
-        hipMalloc(&b->d_pipe_cnt, 8 * 256 + (size_t)b->n_pre_waves * sizeof(uint32_t)) != hipSuccess) {
+    if (dev_malloc(c, (void **)&b->d_lensk, sizeof(BLensC) * n_cfgs) != hipSuccess ||
+        dev_malloc(c, &b->d_pipe, qbytes) != hipSuccess ||
+        dev_malloc(c, &b->d_pipe_cnt, 8 * 256 + (size_t)b->n_pre_waves * sizeof(uint32_t)) != hipSuccess) {
       // not enough memory for the queue: the single-kernel walker needs none
       (void)hipGetLastError();
       if (b->d_pipe) (void)hipFree(b->d_pipe);

@@ -21,6 +21,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -1288,6 +1289,27 @@ int grid_for(ctraj_ctx *ctx, const void *kern, int block, size_t lds, int64_t n,
   return (int)std::max<int64_t>(1, std::min(need, full));
 }
 
+constexpr size_t POOL_MAX = (size_t)1 << 30;  // bytes of scratch blocks kept per context
+
+// Release every kept block (the caller holds the pool's lock).
+static void pool_trim(ctraj_pool &P) {
+  for (auto &kv : P.kept) (void)hipFree(kv.second);
+  P.kept.clear();
+  P.kept_bytes = 0;
+}
+
+hipError_t dev_malloc(ctraj_ctx *ctx, void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  {
+    std::lock_guard<std::mutex> lock(ctx->pool.mu);
+    if (ctx->pool.kept.empty()) return e;
+    pool_trim(ctx->pool);
+  }
+  (void)hipGetLastError();
+  return hipMalloc(p, bytes);
+}
+
 int ensure_buf(ctraj_ctx *ctx, ctraj_devbuf &b, size_t bytes) {
   if (b.bytes >= bytes && b.p) return CTRAJ_OK;
   if (b.p) {
@@ -1296,7 +1318,7 @@ int ensure_buf(ctraj_ctx *ctx, ctraj_devbuf &b, size_t bytes) {
     b.p = nullptr;
     b.bytes = 0;
   }
-  if (hipMalloc(&b.p, bytes) != hipSuccess) {
+  if (dev_malloc(ctx, &b.p, bytes) != hipSuccess) {
     b.p = nullptr;
     (void)hipGetLastError();
     return fail(ctx, CTRAJ_ENOMEM, "device allocation of " + std::to_string(bytes) + " bytes failed");
@@ -1766,6 +1788,10 @@ int32_t ctraj_ctx_destroy(ctraj_ctx *c) {
   if (!c) return CTRAJ_OK;
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
+  {
+    std::lock_guard<std::mutex> lock(c->pool.mu);
+    pool_trim(c->pool);
+  }
   if (c->d_elems) (void)hipFree(c->d_elems);
   if (c->d_ws) (void)hipFree(c->d_ws);
   if (c->d_rt) (void)hipFree(c->d_rt);
@@ -1803,9 +1829,59 @@ int32_t ctraj_dev_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) {
   if (!c || !ptr) return fail(c, CTRAJ_EINVAL, "null argument");
   HIPCHK(c, hipSetDevice(c->device));
   *ptr = nullptr;
-  hipError_t e = hipMalloc(ptr, bytes ? bytes : 1);
+  hipError_t e = dev_malloc(c, ptr, bytes ? bytes : 1);
   if (e != hipSuccess) return fail(c, CTRAJ_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
   return CTRAJ_OK;
+}
+
+int32_t ctraj_scratch_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) try {
+  if (!c || !ptr) return fail(c, CTRAJ_EINVAL, "null argument");
+  *ptr = nullptr;
+  // sizes in steps of an eighth of their power of two, so that runs of similar sizes share blocks
+  size_t step = 512;
+  while (step * 16 <= bytes) step *= 2;
+  const size_t size = std::max<size_t>(4096, (bytes + step - 1) / step * step);
+  if (size < bytes) return fail(c, CTRAJ_ENOMEM, "size out of range");
+  {
+    std::lock_guard<std::mutex> lock(c->pool.mu);
+    auto it = c->pool.kept.lower_bound(size);
+    if (it != c->pool.kept.end() && it->first <= size + size / 4) {
+      *ptr = it->second;
+      c->pool.out[it->second] = it->first;
+      c->pool.kept_bytes -= it->first;
+      c->pool.kept.erase(it);
+      return CTRAJ_OK;
+    }
+  }
+  HIPCHK(c, hipSetDevice(c->device));
+  const hipError_t e = dev_malloc(c, ptr, size);
+  if (e != hipSuccess) return fail(c, CTRAJ_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+  std::lock_guard<std::mutex> lock(c->pool.mu);
+  c->pool.out[*ptr] = size;
+  return CTRAJ_OK;
+} catch (const std::bad_alloc &) {
+  return fail(c, CTRAJ_ENOMEM, "host allocation failed");
+}
+
+int32_t ctraj_scratch_free(ctraj_ctx *c, void *ptr) try {
+  if (!c) return fail(nullptr, CTRAJ_EINVAL, "ctx is NULL");
+  if (!ptr) return CTRAJ_OK;
+  {
+    std::lock_guard<std::mutex> lock(c->pool.mu);
+    auto it = c->pool.out.find(ptr);
+    if (it == c->pool.out.end()) return fail(c, CTRAJ_EINVAL, "not a scratch block of this context");
+    const size_t size = it->second;
+    c->pool.out.erase(it);
+    if (c->pool.kept_bytes + size <= POOL_MAX) {
+      c->pool.kept.emplace(size, ptr);
+      c->pool.kept_bytes += size;
+      return CTRAJ_OK;
+    }
+  }
+  HIPCHK(c, hipFree(ptr));
+  return CTRAJ_OK;
+} catch (const std::bad_alloc &) {
+  return fail(c, CTRAJ_ENOMEM, "host allocation failed");
 }
 
 int32_t ctraj_dev_free(ctraj_ctx *c, void *ptr) {

@@ -4,7 +4,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <map>
+#include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/ctraj.h"
@@ -13,6 +16,16 @@
 struct ctraj_devbuf {
   void *p = nullptr;
   size_t bytes = 0;
+};
+
+// Blocks of ctraj_scratch_alloc: those handed out, and those given back and kept for the next request (all
+// work on them is queued on the context's one stream, so a block may be handed out while the last holder's
+// kernels still run).
+struct ctraj_pool {
+  std::mutex mu;
+  std::multimap<size_t, void *> kept;
+  std::unordered_map<void *, size_t> out;
+  size_t kept_bytes = 0;
 };
 
 struct ctraj_ctx {
@@ -55,6 +68,7 @@ struct ctraj_ctx {
   ctraj_devbuf pipe, pipe_cnt;
   // lens kernel claim order: per-entry lifetime buckets, per-workgroup bucket counts, slot permutation
   ctraj_devbuf ord;
+  ctraj_pool pool;
   // this device's scratch array of ctraj_propagate_noalloc (device address), or nullptr
   char *scratch = nullptr;
 };
@@ -93,6 +107,8 @@ int lds_limit(ctraj_ctx *ctx, const void *kern, size_t bytes);
 int grid_for(ctraj_ctx *ctx, const void *kern, int block, size_t lds, int64_t n, int req);
 // EINVAL unless `block` threads fit the kernel's launch bounds
 int block_ok(ctraj_ctx *ctx, const void *kern, int block);
+// hipMalloc that releases the context's kept scratch blocks and tries again when memory runs out
+hipError_t dev_malloc(ctraj_ctx *ctx, void **p, size_t bytes);
 // make b hold at least `bytes` (grow-only; the old buffer is released first)
 int ensure_buf(ctraj_ctx *ctx, ctraj_devbuf &b, size_t bytes);
 

@@ -180,6 +180,8 @@ SIGNATURES = [
     ("ctraj_device_info", C.c_int32, [C.c_void_p] + [C.POINTER(C.c_int32)] * 4),
     ("ctraj_dev_alloc", C.c_int32, [C.c_void_p, C.c_uint64, C.POINTER(C.c_void_p)]),
     ("ctraj_dev_free", C.c_int32, [C.c_void_p, C.c_void_p]),
+    ("ctraj_scratch_alloc", C.c_int32, [C.c_void_p, C.c_uint64, C.POINTER(C.c_void_p)]),
+    ("ctraj_scratch_free", C.c_int32, [C.c_void_p, C.c_void_p]),
     ("ctraj_host_alloc", C.c_int32, [C.c_void_p, C.c_uint64, C.POINTER(C.c_void_p)]),
     ("ctraj_host_free", C.c_int32, [C.c_void_p, C.c_void_p]),
     ("ctraj_memcpy", C.c_int32, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_uint64, C.c_int32]),

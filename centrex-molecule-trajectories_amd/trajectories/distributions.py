@@ -51,6 +51,25 @@ class Distribution(ABC):
         raise NotImplementedError(f"{type(self).__name__} has no device sampler")
 
 
+def _plain(*values) -> bool:
+    return all(type(v) in (int, float, np.float64) for v in values)
+
+
+def _normals(loc, scale, n: int) -> np.ndarray:
+    """norm.rvs(loc, scale, n): for plain numbers its own two operations on the same random state, without the
+    argument handling that made up nearly all of a short draw's time (17 us)."""
+    if _plain(loc, scale) and scale > 0 and type(n) is int:
+        return norm.random_state.standard_normal(n) * scale + loc
+    return norm.rvs(loc=loc, scale=scale, size=n)
+
+
+def _uniforms(n: int) -> np.ndarray:
+    """uniform.rvs(size=n) (on [0, 1)), likewise."""
+    if type(n) is int:
+        return uniform.random_state.uniform(0.0, 1.0, n)
+    return uniform.rvs(size=n)
+
+
 @dataclass
 class GaussianDistribution(Distribution):
     mean: float
@@ -60,6 +79,8 @@ class GaussianDistribution(Distribution):
         self.dist = norm
 
     def draw(self, n: int) -> np.ndarray:
+        if self.dist is norm:
+            return _normals(self.mean, self.sigma, n)
         return self.dist.rvs(loc=self.mean, scale=self.sigma, size=n)
 
     def plot(self):
@@ -101,8 +122,8 @@ class CeNTREXPositionDistribution(Distribution):
     z: float = 0.25 * 0.0254
 
     def draw(self, n: int) -> np.ndarray:
-        theta = uniform.rvs(size=n) * 2 * np.pi
-        r = np.sqrt(uniform.rvs(size=n)) * self.d / 2
+        theta = _uniforms(n) * 2 * np.pi
+        r = np.sqrt(_uniforms(n)) * self.d / 2
         return np.array((r * np.cos(theta), r * np.sin(theta), np.full(n, self.z)))
 
     def disc_params(self):
@@ -124,3 +145,42 @@ class GaussianPositionDistribution(Distribution):
 
     def gaussian_params(self):
         return (np.array([0.0, 0.0, self.z], float), np.array([self.sigmax, self.sigmay, 0.0], float))
+
+
+def draw_chunks(xdist: Distribution, vdist: Distribution, n: int, chunks: int) -> tuple[np.ndarray, np.ndarray]:
+    """``chunks`` times vdist.draw(n) then xdist.draw(n) (trajectory_simulator.py:52-60 of the reference), joined:
+    X and V of shape (3, chunks n).
+
+    The reference's distributions draw from one random state, whose normal stream does not depend on how it is cut
+    into calls: with Gaussian velocities and either position distribution, a chunk's normals are one call and
+    its uniforms another, and the arithmetic is done once on all chunks, element for element the same."""
+    total = n * chunks
+    if type(vdist) is CeNTREXVelocityDistribution and norm.random_state is uniform.random_state and n > 0:
+        vp = (vdist.vx, vdist.sigmax, vdist.vy, vdist.sigmay, vdist.vz, vdist.sigmaz)
+        if _plain(*vp) and min(vp[1::2]) > 0:
+            rs = norm.random_state
+            if type(xdist) is GaussianPositionDistribution and _plain(xdist.sigmax, xdist.sigmay, xdist.z) \
+                    and min(xdist.sigmax, xdist.sigmay) > 0:
+                g = rs.standard_normal(5 * total).reshape(chunks, 5, n)
+                X = np.stack([(g[:, 3] * xdist.sigmax + 0).reshape(-1), (g[:, 4] * xdist.sigmay + 0).reshape(-1),
+                              np.full(total, xdist.z, dtype=np.float64)])
+            elif type(xdist) is CeNTREXPositionDistribution and _plain(xdist.d, xdist.z):
+                g, u = np.empty((chunks, 3, n)), np.empty((chunks, 2, n))
+                for c in range(chunks):
+                    g[c] = rs.standard_normal(3 * n).reshape(3, n)
+                    u[c] = rs.uniform(0.0, 1.0, 2 * n).reshape(2, n)
+                theta = u[:, 0].reshape(-1) * 2 * np.pi
+                r = np.sqrt(u[:, 1].reshape(-1)) * xdist.d / 2
+                X = np.stack([r * np.cos(theta), r * np.sin(theta), np.full(total, xdist.z, dtype=np.float64)])
+            else:
+                g = None
+            if g is not None:
+                V = np.stack([(g[:, k] * vp[2 * k + 1] + vp[2 * k]).reshape(-1) for k in range(3)])
+                return X, V
+    vs, xs = [], []
+    for _ in range(chunks):
+        vs.append(np.asarray(vdist.draw(n), dtype=np.float64).reshape(3, n))
+        xs.append(np.asarray(xdist.draw(n), dtype=np.float64).reshape(3, n))
+    if not vs:
+        return np.zeros((3, 0)), np.zeros((3, 0))
+    return np.concatenate(xs, axis=1), np.concatenate(vs, axis=1)

@@ -60,7 +60,7 @@ class Engine:
         call copies its results to the host before it returns, so the next call may reuse it)."""
         b = self._scratch.get(name)
         if b is None or b.n < n or b.dtype != np.dtype(dtype):
-            b = self.ctx.alloc(max(int(n), 1), dtype)
+            b = self.ctx.scratch(max(int(n), 1), dtype)
             self._scratch[name] = b
         return b
 
@@ -110,18 +110,25 @@ class Engine:
     def _upload_inputs(self, x, y, z, vx, vy, vz, t, a0, state):
         ctx = self.ctx
         n = int(np.asarray(x).size)
-        inp = {k: ctx.to_device(np.asarray(v, dtype=np.float64)) for k, v in
-               zip(FIELDS[:6], (x, y, z, vx, vy, vz))}
+        host = []  # the uploads' sources, kept until the one wait below
+
+        def up(a, dtype):
+            a = np.ascontiguousarray(a, dtype=dtype).reshape(-1)
+            host.append(a)
+            return ctx.scratch_from(a)
+
+        inp = {k: up(v, np.float64) for k, v in zip(FIELDS[:6], (x, y, z, vx, vy, vz))}
         if t is not None:
-            inp["t"] = ctx.to_device(np.asarray(t, dtype=np.float64))
+            inp["t"] = up(t, np.float64)
         a0d = None
         if a0 is not None:
-            a0d = [ctx.to_device(np.asarray(a, dtype=np.float64)) for a in a0]
+            a0d = [up(a, np.float64) for a in a0]
         st = None
         if state is not None:
-            st = ctx.to_device(np.asarray(state, dtype=np.uint8))
-            if n and int(np.max(state)) >= self.cb.n_states:
-                raise ValueError("state id >= n_states")
+            st = up(state, np.uint8)
+        ctx.sync()
+        if state is not None and n and int(np.max(state)) >= self.cb.n_states:
+            raise ValueError("state id >= n_states")
         return n, inp, a0d, st
 
     def propagate(self, x, y, z, vx, vy, vz, t=None, a0=None, state=None, *, outputs: bool = True,
@@ -144,9 +151,12 @@ class Engine:
         a0d, st = a0, state
         res = {"n": n, "labels": list(self.cb.labels)}
         nl, ns = self.cb.n_labels, self.cb.n_states
-        tally = self._buf("tally", ns * nl, np.int64).fill(0)
-        first = self._buf("first", nl, np.int64).fill(np.iinfo(np.int64).max)
-        work = self._buf("work", N.WORK_N, np.uint64).fill(0)
+        # tally, work counters and the count of kept molecules, then the first indices: two fills, one copy back
+        nz = ns * nl + N.WORK_N + 1
+        counts = self._buf("counts", nz + nl, np.int64)
+        tally, work, count, first = (counts.ptr + 8 * k for k in (0, ns * nl, nz - 1, nz))
+        for at, k, v in ((tally, nz, 0), (first, nl, np.iinfo(np.int64).max)):
+            N.check("ctraj_fill_i64", N.lib().ctraj_fill_i64(ctx.handle, at, int(v), k), ctx.handle)
         label = self._buf("label", n, np.int32) if per_molecule else None
         status = self._buf("status", n, np.uint8) if per_molecule else None
         out = {k: self._buf("out_" + k, n) for k in FIELDS} if outputs else None
@@ -157,7 +167,7 @@ class Engine:
                 mask |= 1 << self.cb.labels.index(name)
         aoi = {}
         if mask:
-            aoi["count"] = self._buf("aoi_count", 1, np.int64).fill(0)
+            aoi["count"] = count
             aoi["index"] = self._buf("aoi_index", n, np.int64)
             aoi["label"] = self._buf("aoi_label", n, np.int32)
             aoi["out"] = {k: self._buf("aoi_out_" + k, n) for k in FIELDS}
@@ -167,31 +177,38 @@ class Engine:
                         aoi_index=aoi.get("index"), aoi_label=aoi.get("label"), aoi_out=aoi.get("out"),
                         work=work, a0=a0d, state=st,
                         n=n, index_base=index_base, block=block, flags=flags, refill=refill, noalloc=noalloc)
-        ctx.sync()
-        res["tally"] = tally.to_host(count=ns * nl).reshape(ns, nl)
-        res["first_index"] = first.to_host(count=nl)
-        res["work"] = work.to_host(count=N.WORK_N)
+        h = np.empty(nz + nl, np.int64)
+        pairs = [(counts, h)]
+
+        def want(buf, shape=n):
+            pairs.append((buf, np.empty(shape, buf.dtype)))
+            return pairs[-1][1]
+
         if per_molecule:
-            res["label"] = label.to_host(count=n)
-            res["status"] = status.to_host(count=n)
+            res["label"], res["status"] = want(label), want(status)
         if outputs:
-            res["out"] = {k: v.to_host(count=n) for k, v in out.items()}
+            res["out"] = {k: want(v) for k, v in out.items()}
         if want_accel:
-            res["out_a"] = [v.to_host(count=n) for v in out_a]
+            res["out_a"] = [want(v) for v in out_a]
+        ctx.read(*pairs)
+        res["tally"] = h[: ns * nl].reshape(ns, nl).copy()
+        res["work"] = h[ns * nl: nz - 1].view(np.uint64).copy()
+        res["first_index"] = h[nz:].copy()
         if mask:
-            cnt = int(aoi["count"].to_host(count=1)[0])
-            res["aoi_index"] = aoi["index"].to_host(count=cnt)
-            res["aoi_label"] = aoi["label"].to_host(count=cnt)
-            res["aoi_out"] = {k: v.to_host(count=cnt) for k, v in aoi["out"].items()}
+            cnt = int(h[nz - 1])
+            pairs = []
+            res["aoi_index"], res["aoi_label"] = want(aoi["index"], cnt), want(aoi["label"], cnt)
+            res["aoi_out"] = {k: want(v, cnt) for k, v in aoi["out"].items()}
+            ctx.read(*pairs)
         return res
 
     def _record(self, mode, x, y, z, vx, vy, vz, t, a0, state, cap, z_start=0.0, z_step=0.0):
         ctx = self.ctx
         n, inp, a0d, st = self._upload_inputs(x, y, z, vx, vy, vz, t, a0, state)
         nf = 10 if mode == N.REC_ROWS else 6
-        buf = ctx.alloc(max(nf * cap * n, 1))
-        nrows = ctx.alloc(max(n, 1), np.int32)
-        lab = ctx.alloc(max(n, 1), np.int32)
+        buf = ctx.scratch(max(nf * cap * n, 1))
+        nrows = ctx.scratch(max(n, 1), np.int32)
+        lab = ctx.scratch(max(n, 1), np.int32)
         if n:
             bind(ctx, self.cb)
             Rc = N.Record()
@@ -206,12 +223,10 @@ class Engine:
             Rc.buf, Rc.n_rows, Rc.label = buf.ptr, nrows.ptr, lab.ptr
             N.check("ctraj_record_trajectories", N.lib().ctraj_record_trajectories(ctx.handle, C.byref(Rc)),
                     ctx.handle)
-        ctx.sync()
-        if mode == N.REC_ZGRID_MOL:
-            data = buf.to_host()[: nf * cap * n].reshape(n, cap, nf)
-        else:
-            data = buf.to_host()[: nf * cap * n].reshape(nf, cap, n)
-        return data, nrows.to_host()[:n], lab.to_host()[:n]
+        data = np.empty((n, cap, nf) if mode == N.REC_ZGRID_MOL else (nf, cap, n))
+        nr_h, lab_h = np.empty(n, np.int32), np.empty(n, np.int32)
+        ctx.read((buf, data), (nrows, nr_h), (lab, lab_h))
+        return data, nr_h, lab_h
 
     def record_rows(self, x, y, z, vx, vy, vz, t=None, a0=None, state=None, cap: int = 64):
         """Every trajectory row per molecule: (rows [n][cap][10], n_rows [n], labels [n]).

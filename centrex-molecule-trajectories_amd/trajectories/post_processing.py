@@ -54,27 +54,29 @@ def sample_rows(molecules, z: float, ctx=None) -> tuple[np.ndarray, np.ndarray]:
     n = off.size - 1
     if n == 0:
         return np.zeros((6, 0)), np.zeros(0, bool)
-    d_rows = ctx.to_device(rows.reshape(-1) if rows.size else np.zeros(10))
-    d_off = ctx.to_device(off)
-    outs = [ctx.alloc(n) for _ in range(6)]
-    valid = ctx.alloc(n, np.uint8)
+    host = rows.reshape(-1) if rows.size else np.zeros(10)
+    d_rows = ctx.scratch_from(host)
+    d_off = ctx.scratch_from(off)
+    outs = [ctx.scratch(n) for _ in range(6)]
+    valid = ctx.scratch(n, np.uint8)
     S = N.Sample()
     S.n, S.row_off, S.n_rows, S.rows, S.z = n, d_off.ptr, rows.shape[0], d_rows.ptr, float(z)
     for f in range(6):
         S.out[f] = outs[f].ptr
     S.valid = valid.ptr
     N.check("ctraj_sample_rows", N.lib().ctraj_sample_rows(ctx.handle, C.byref(S)), ctx.handle)
-    ctx.sync()
-    return np.array([o.to_host() for o in outs]), valid.to_host().astype(bool)
+    vals, ok = np.empty((6, n)), np.empty(n, np.uint8)
+    ctx.read(*((o, vals[f]) for f, o in enumerate(outs)), (valid, ok))
+    return vals, ok.astype(bool)
 
 
 def sample_at(result, z: float, elements: List[str] = None) -> tuple[np.ndarray, np.ndarray]:
     """The molecules of ``result`` at z: ([6][m] x, y, vx, vy, vz, t of the molecules the reference keeps,
     in result order; their indices into result.molecules)."""
     mols = result.molecules
-    hits = mols.aperture_hits if hasattr(mols, "aperture_hits") else [m.aperture_hit for m in mols]
-    sel = np.arange(len(hits), dtype=np.int64)
+    sel = np.arange(len(mols), dtype=np.int64)
     if elements is not None:
+        hits = mols.aperture_hits if hasattr(mols, "aperture_hits") else [m.aperture_hit for m in mols]
         sel = np.array([i for i, h in enumerate(hits) if h in elements], dtype=np.int64)
     if hasattr(mols, "sample_at"):
         vals, valid = mols.sample_at(z, sel)

@@ -147,15 +147,9 @@ class SmoothFlux:
         dG = self._buf("grad", n_cfg * self.n_params) if grad else None
         self._capped.fill(0)
         self.launch(dP.ptr, n_cfg, dJ.ptr, None if dG is None else dG.ptr, ms)
-        J = np.empty(n_cfg)
-        self.ctx.memcpy(J.ctypes.data, dJ.ptr, J.nbytes, N.D2H)
-        G = None
-        if grad:
-            G = np.empty((n_cfg, self.n_params))
-            self.ctx.memcpy(G.ctypes.data, dG.ptr, G.nbytes, N.D2H)
-        cap = np.empty(1, np.int64)
-        self.ctx.memcpy(cap.ctypes.data, self._capped.ptr, 8, N.D2H)
-        self.ctx.sync()
+        J, cap = np.empty(n_cfg), np.empty(1, np.int64)
+        G = np.empty((n_cfg, self.n_params)) if grad else None
+        self.ctx.read((dJ, J), (self._capped, cap), *(((dG, G),) if grad else ()))
         return SmoothResult(J, G, int(cap[0]))
 
     def central_differences(self, theta, rel_step: float = 1e-6) -> np.ndarray:

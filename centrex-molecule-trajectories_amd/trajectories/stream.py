@@ -61,10 +61,10 @@ class StreamResult:
             raise IndexError("detected molecule out of range")
         e = np.arange(ns * 6)[None, :]
         idx = np.ascontiguousarray((js[:, None] * (ns * 6) + e).reshape(-1))
-        d_idx = ctx.to_device(idx)
-        out = ctx.alloc(max(idx.size, 1))
+        d_idx = ctx.scratch_from(idx)
+        out = ctx.scratch(max(idx.size, 1))
         gather(ctx, idx.size, d_idx, 0, 6 * ns * nd, [self.trajectories], [out])
-        return out.to_host()[: idx.size].reshape(js.size, ns, 6)
+        return out.to_host(count=idx.size).reshape(js.size, ns, 6)
 
 
 class StreamedRun:
@@ -93,14 +93,14 @@ class StreamedRun:
         nl, ns = cb.n_labels, cb.n_states
         det = cb.label_detected
         ch = min(self.chunk, max(self.n, 1))
-        inp = {k: ctx.alloc(ch) for k in FIELDS6}
-        state = ctx.alloc(ch, np.uint8)
-        tally = ctx.alloc(ns * nl, np.int64)
-        work = ctx.alloc(N.WORK_N, np.uint64)
-        aoi_count = ctx.alloc(1, np.int64)
+        inp = {k: ctx.scratch(ch) for k in FIELDS6}
+        state = ctx.scratch(ch, np.uint8)
+        tally = ctx.scratch(ns * nl, np.int64)
+        work = ctx.scratch(N.WORK_N, np.uint64)
+        aoi_count = ctx.scratch(1, np.int64)
         cap = max(4096, int(0.05 * self.n))
         while True:
-            aoi_index = ctx.alloc(cap, np.int64)
+            aoi_index = ctx.scratch(cap, np.int64)
             for a in (tally, work, aoi_count):
                 a.fill(0)
             t0 = time.perf_counter()
@@ -127,11 +127,11 @@ class StreamedRun:
         if count:
             # output buffers first, so that the timed device region holds pass 2's kernels only
             t0 = time.perf_counter()
-            init = [ctx.alloc(count) for _ in FIELDS6]
-            init_state = ctx.alloc(count, np.uint8)
+            init = [ctx.scratch(count) for _ in FIELDS6]
+            init_state = ctx.scratch(count, np.uint8)
             if trajectories:
-                traj = ctx.alloc(6 * self.n_samples * count)
-                written = ctx.alloc(count, np.int32)
+                traj = ctx.alloc(6 * self.n_samples * count)  # the caller's
+                written = ctx.scratch(count, np.int32)
             t_alloc = time.perf_counter() - t0
             ctx.event_record(2)
             sort_i64(ctx, aoi_index, count)
@@ -153,16 +153,15 @@ class StreamedRun:
             ctx.event_record(3)
             ctx.sync()
             t_pass2 = ctx.event_elapsed_ms(2, 3)
-            idx_h = np.empty(count, np.int64)
-            ctx.memcpy(idx_h.ctypes.data, aoi_index.ptr, idx_h.nbytes, N.D2H)
-            st_h = np.empty(count, np.uint8)
-            ctx.memcpy(st_h.ctypes.data, init_state.ptr, st_h.nbytes, N.D2H)
-            ctx.sync()
-        return StreamResult(self.n, list(cb.labels), tally.to_host().reshape(ns, nl), idx_h, st_h, self.n_samples,
-                            self.z_start, self.z_step, traj, None if written is None else written.to_host(),
+            idx_h, st_h = np.empty(count, np.int64), np.empty(count, np.uint8)
+            ctx.read((aoi_index, idx_h), (init_state, st_h))
+        tally_h, work_h = np.empty((ns, nl), np.int64), np.empty(N.WORK_N, np.uint64)
+        written_h = None if written is None else np.empty(count, np.int32)
+        ctx.read((tally, tally_h), (work, work_h), *(() if written is None else ((written, written_h),)))
+        return StreamResult(self.n, list(cb.labels), tally_h, idx_h, st_h, self.n_samples,
+                            self.z_start, self.z_step, traj, written_h,
                             {"pass1_device_ms": t_pass1, "pass1_wall_s": wall1, "pass2_device_ms": t_pass2,
-                             "pass2_alloc_s": t_alloc},
-                            work.to_host())
+                             "pass2_alloc_s": t_alloc}, work_h)
 
     def _grow(self, arr: DeviceArray, used: int, new_n: int) -> DeviceArray:
         out = self.ctx.alloc(new_n, arr.dtype)

@@ -21,7 +21,7 @@ import numpy as np
 
 from . import _native as N
 from .beamline import Beamline
-from .distributions import CeNTREXPositionDistribution, CeNTREXVelocityDistribution, Distribution
+from .distributions import CeNTREXPositionDistribution, CeNTREXVelocityDistribution, Distribution, draw_chunks
 from .engine import Engine
 from .molecule import Molecule, Trajectory
 
@@ -171,12 +171,7 @@ class TrajectorySimulator:
                                   chunk=chunk, block=block, states=states, raise_out_of_table=raise_out_of_table)
             self._store(run_name, beamline, xdist, vdist, res)
             return
-        vs, xs = [], []
-        for _ in range(N_loops):
-            vs.append(np.asarray(vdist.draw(N), dtype=np.float64).reshape(3, N))
-            xs.append(np.asarray(xdist.draw(N), dtype=np.float64).reshape(3, N))
-        V = np.concatenate(vs, axis=1) if vs else np.zeros((3, 0))
-        X = np.concatenate(xs, axis=1) if xs else np.zeros((3, 0))
+        X, V = draw_chunks(xdist, vdist, N, N_loops)
         res = simulate_arrays(beamline, X, V, apertures_of_interest, ctx=ctx, chunk=chunk, block=block,
                               states=states, raise_out_of_table=raise_out_of_table)
         assert res.n == total
@@ -295,7 +290,7 @@ def simulate_device(beamline: Beamline, xdist: Distribution, vdist: Distribution
     work = np.zeros(8, np.uint64)
     aoi_idx, aoi_lab, aoi_fin, inits = [], [], [], []
     n_oot = n_capped = 0
-    bufs = [ctx.alloc(max(1, min(chunk, n))) for _ in range(6)]
+    bufs = [ctx.scratch(max(1, min(chunk, n))) for _ in range(6)]
     for s in range(0, n, chunk):
         m = min(chunk, n - s)
         src = [*xdist.draw_device(m, kx, offset=s, ctx=ctx, out=bufs[:3]),
@@ -320,9 +315,11 @@ def simulate_device(beamline: Beamline, xdist: Distribution, vdist: Distribution
             aoi_lab.append(r["aoi_label"][o])
             aoi_fin.append({k: v[o] for k, v in r["aoi_out"].items()})
             if idx.size:
-                dst = [ctx.alloc(idx.size) for _ in range(6)]
-                gather(ctx, idx.size, ctx.to_device(idx), s, m, src, dst)
-                inits.append(np.array([d.to_host()[: idx.size] for d in dst]))
+                dst = [ctx.scratch(idx.size) for _ in range(6)]
+                gather(ctx, idx.size, ctx.scratch_from(idx), s, m, src, dst)
+                rows = np.empty((6, idx.size))
+                ctx.read(*((d, rows[f]) for f, d in enumerate(dst)))
+                inits.append(rows)
     eng.free_scratch()
     for b in bufs:
         b.free()

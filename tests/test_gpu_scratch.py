@@ -1,0 +1,66 @@
+"""GPU: scratch blocks are exclusive while held, reused after they are given back, and bounded."""
+import threading
+
+import numpy as np
+import pytest
+
+from trajectories import _native as N
+from trajectories import configs
+from trajectories.device import Context
+from trajectories.engine import Engine
+
+pytestmark = pytest.mark.gpu
+
+
+def test_blocks():
+    ctx = Context(0)
+    a = ctx.scratch(1000)
+    p = a.ptr
+    b = ctx.scratch(1000)
+    assert b.ptr != p
+    a.free()
+    assert ctx.scratch(990).ptr == p  # the block given back
+    with pytest.raises(N.NativeError):
+        N.check("ctraj_scratch_free", N.lib().ctraj_scratch_free(ctx.handle, b.ptr + 8), ctx.handle)
+    big = ctx.scratch((3 << 30) // 8)  # larger than everything that is kept: released at once
+    big.free()
+    h = np.arange(300_000.0)  # through page-locked memory and past it
+    d, e = ctx.scratch_from(h), ctx.scratch_from(h[:5])
+    ctx.sync()
+    x, y, z = np.empty_like(h), np.empty(5), np.empty(0)
+    ctx.read((d, x), (e, y), (d, z))
+    assert np.array_equal(x, h) and np.array_equal(y, h[:5])
+    ctx.close()
+
+
+def test_threads_hold_different_blocks():
+    ctx = Context(0)
+    seen, lock, bad = set(), threading.Lock(), []
+
+    def work():
+        for n in (10, 1000, 5000) * 30:
+            a = ctx.scratch(n)
+            with lock:
+                if a.ptr in seen:
+                    bad.append(a.ptr)
+                seen.add(a.ptr)
+            with lock:
+                seen.discard(a.ptr)
+            a.free()
+
+    ts = [threading.Thread(target=work) for _ in range(6)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad
+    ctx.close()
+
+
+def test_results_do_not_depend_on_reused_blocks():
+    eng = Engine(configs.config1())
+    X, V = configs.draw_source(30_000, 3)
+    first = {n: eng.propagate(*X[:, :n], *V[:, :n], aoi_labels=["Detected"]) for n in (30_000, 1, 777)}
+    for n in (777, 30_000, 1):
+        r = eng.propagate(*X[:, :n], *V[:, :n], aoi_labels=["Detected"])
+        assert np.array_equal(r["label"], first[n]["label"]) and np.array_equal(r["tally"], first[n]["tally"])
+        assert all(np.array_equal(r["out"][k], first[n]["out"][k]) for k in r["out"])
+        assert np.array_equal(np.sort(r["aoi_index"]), np.sort(first[n]["aoi_index"]))
