@@ -53,11 +53,9 @@ struct AoiStage {
   double *val;     // [7][AOI_WAVE]
 };
 
-// Copy a wavefront's staged entries [0, cnt) to the output (called by the whole wavefront).
-__device__ __forceinline__ void aoi_flush_wave(const ctraj_run &R, const AoiStage &A, int cnt, int lane) {
-  unsigned long long base = 0;
-  if (lane == 0) base = atomicAdd((unsigned long long *)R.aoi_count, (unsigned long long)cnt);
-  base = __shfl(base, 0);
+// Copy a wavefront's staged entries [0, cnt) to the output from slot `base` on (called by the whole wavefront).
+__device__ __forceinline__ void aoi_write_wave(const ctraj_run &R, const AoiStage &A, int cnt, int lane,
+                                               unsigned long long base) {
   double *outs[7] = {R.aoi_out.x, R.aoi_out.y, R.aoi_out.z, R.aoi_out.vx, R.aoi_out.vy, R.aoi_out.vz, R.aoi_out.t};
   for (int j = lane; j < cnt; j += 64) {
     const int64_t slot = (int64_t)base + j;
@@ -69,6 +67,12 @@ __device__ __forceinline__ void aoi_flush_wave(const ctraj_run &R, const AoiStag
         if (outs[f]) outs[f][slot] = A.val[f * AOI_WAVE + j];
     }
   }
+}
+
+__device__ __forceinline__ void aoi_flush_wave(const ctraj_run &R, const AoiStage &A, int cnt, int lane) {
+  unsigned long long base = 0;
+  if (lane == 0) base = atomicAdd((unsigned long long *)R.aoi_count, (unsigned long long)cnt);
+  aoi_write_wave(R, A, cnt, lane, __shfl(base, 0));
 }
 
 struct InMol {
@@ -207,7 +211,8 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
   extern __shared__ __attribute__((aligned(16))) double lds[];
   __shared__ uint32_t s_hist[CTRAJ_MAX_STATES * CTRAJ_MAX_LABELS];
   __shared__ unsigned long long s_first[CTRAJ_MAX_LABELS];
-  __shared__ unsigned long long s_work[5];
+  __shared__ unsigned long long s_work[5], s_aoi_base;
+  __shared__ uint32_t s_aoi[4];  // kept molecules staged by each wavefront at the end
   __shared__ uint32_t s_ord[PHASE == PHASE_PRE ? ORD_BUCKETS : 1];  // PRE: this workgroup's lifetime buckets
   const int nbins = B.n_states * B.n_labels;
   for (int b = threadIdx.x; b < nbins; b += blockDim.x) s_hist[b] = 0;
@@ -423,7 +428,7 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
     }
     for (int64_t wbase = w0, j = j0; wbase < n_items; wbase += stride, j += stride) body(q, j, wbase);
   }
-  if (R.aoi_mask && aoi_n > 0) aoi_flush_wave(R, A, aoi_n, lane);
+  if (R.aoi_mask && lane == 0) s_aoi[wave] = (uint32_t)aoi_n;
   if constexpr (PHASE == PHASE_PRE) {
     if (lane == 0) P.wcount[gwave] = (uint32_t)qn;
   }
@@ -435,6 +440,15 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
     if (faces_post) atomicAdd(&s_work[4], (unsigned long long)faces_post);
   }
   __syncthreads();
+  // what the wavefronts still hold of kept molecules goes out with one reservation per workgroup: atomics on one
+  // address from all XCDs complete about 15 ns apart, which made one per wavefront 60 us of the 69 us that 10^6
+  // molecules took
+  unsigned long long aoi_base = 0;
+  if (R.aoi_mask && threadIdx.x == 0) {
+    uint32_t total = 0;
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) total += s_aoi[w];
+    if (total) aoi_base = atomicAdd((unsigned long long *)R.aoi_count, (unsigned long long)total);
+  }
   if (R.tally)
     for (int b = threadIdx.x; b < nbins; b += blockDim.x)
       if (s_hist[b]) atomicAdd((unsigned long long *)&R.tally[b], (unsigned long long)s_hist[b]);
@@ -448,6 +462,13 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
     if (P.bkt)  // every workgroup writes its whole row
       for (int b = threadIdx.x; b < ORD_BUCKETS; b += blockDim.x)
         P.ord_hist[(size_t)blockIdx.x * ORD_BUCKETS + b] = s_ord[b];
+  }
+  if (R.aoi_mask) {
+    if (threadIdx.x == 0) s_aoi_base = aoi_base;
+    __syncthreads();
+    unsigned long long base = s_aoi_base;
+    for (int w = 0; w < wave; ++w) base += s_aoi[w];
+    aoi_write_wave(R, A, aoi_n, lane, base);
   }
 }
 
@@ -1724,7 +1745,14 @@ static int32_t propagate_impl(ctraj_ctx *c, const ctraj_run *R, char *sdev) {
     if (rc) return rc;
     rc = block_ok(c, (const void *)k, block);
     if (rc) return rc;
-    const int grid = grid_for(c, (const void *)k, block, lds_all, R->n, R->grid);
+    // Without a lens, up to six times the resident workgroups while each thread keeps a dozen molecules: a SIMD
+    // issues its oldest wavefronts first, so with one share each the youngest ran on alone at the end, and the
+    // dispatcher evens that out.  The workgroups' final atomics, some 15 ns apart on one address, are the price.
+    // 5 10^7 molecules: 755 us with the resident 1024 workgroups, 711, 687, 682 with 2, 4, 6 times as many; 10^7:
+    // 168, 161, 164, 171; 3 10^6: 61, 65, 81, 99.
+    int grid = grid_for(c, (const void *)k, block, lds_all, R->n, R->grid);
+    if (n_lens == 0 && R->grid <= 0)
+      grid = (int)std::max<int64_t>(grid, std::min<int64_t>((int64_t)6 * grid, R->n / ((int64_t)block * 12)));
     if (pev) HIPCHK(c, hipEventRecord(pev[0], c->stream));
     hipLaunchKernelGGL(k, dim3(grid), dim3(block), lds_all, c->stream, B, kt, *R, aoi_off, PipeArgs{});
     if (pev) {
