@@ -710,7 +710,7 @@ int32_t ctraj_smooth_objective(ctraj_ctx *c, const ctraj_smooth *s) {
   A.partial = (double *)((char *)c->sm_part.p + 256);
   if ((rc = ctraj_fill_i64(c, (int64_t *)A.next, 0, 1)) != CTRAJ_OK) return rc;
 
-  const KBeam B = make_kbeam(c->d_elems, c->n_elems, c->phys);
+  const KBeam B = make_kbeam(c->d_elems, c->h_elems.data(), c->n_elems, c->phys);
   if (grad)
     hipLaunchKernelGGL(k_smooth<true>, dim3(grid), dim3(block), lds, c->stream, B, kt, A);
   else

@@ -55,6 +55,7 @@ struct BArgs {
   int64_t total;
   double g;
   int n_cfg, n_labels, label_detected, cap, chunk, refill_min;
+  int tame;                     // every face and g are of moderate size (walk_tame_elems)
   double Hs;                    // the lens dt shared by every configuration (split path's lens kernel, UH)
   int off_begin, off_hist;      // in doubles from the LDS base (off_begin: the lens constants in the lens kernel)
 };
@@ -96,7 +97,7 @@ __device__ __forceinline__ int find_cfg(const int64_t *s_begin, int n_cfg, int64
 // elements `el` before its lens and through the lens entrance.  Returns true if it enters the lens;
 // otherwise it has finished with label `lab`.
 template <int KM>
-__device__ __forceinline__ bool batch_start(const BCfg &C, const ctraj_elem *el, uint64_t j, double g,
+__device__ __forceinline__ bool batch_start(const BCfg &C, const ctraj_elem *el, uint64_t j, double g, bool tame,
                                             int label_detected, MState &m, int &lab, WalkCounters &wc) {
   double z[6];
   gaussian_pair(C.seed, j, 0u, z[0], z[1]);
@@ -113,12 +114,18 @@ __device__ __forceinline__ bool batch_start(const BCfg &C, const ctraj_elem *el,
   m.ay = -g;
   m.az = 0.0;
   lab = label_detected;
-  const bool ok = walk_plain<KM, true>(el, 0, C.lens >= 0 ? C.lens : C.ne, g, m, lab, wc);
-  if (!ok || C.lens < 0) return false;
+  const int e1 = C.lens >= 0 ? C.lens : C.ne;
+  if (KM == KM_CIRC && (tame & walk_tame(m))) {
+    const double iv = recip(m.vz);
+    if (!walk_circ_tame<true>(el, 0, e1, g, m, iv, lab, wc) || C.lens < 0) return false;
+    drift_tame(m, el[C.lens].z0, iv, g);
+  } else {
+    if (!walk_plain<KM, true>(el, 0, e1, g, m, lab, wc) || C.lens < 0) return false;
+    drift_dt(m, time_to(m, el[C.lens].z0), g);
+  }
   const ctraj_elem &L = el[C.lens];
-  drift_dt(m, time_to(m, L.z0), g);
   ++wc.faces;
-  if (rho_of(m.x, m.y) > L.p[0]) {
+  if (beyond_r2(m.x, m.y, L.p[6])) {  // the squared-radius threshold of d/2 (batch elements)
     lab = L.label_hit;
     return false;
   }
@@ -339,7 +346,8 @@ __global__ void __launch_bounds__(256) k_batch_pre(BArgs A, BPipe P) {
     if (active) {
       c = find_cfg(s_begin, A.n_cfg, gi);
       const BCfg &C = opaque(A.cfgs)[c];
-      enq = batch_start<KM>(C, opaque(A.elems) + C.e0, (uint64_t)(gi - C.begin), g, A.label_detected, m, lab, wc);
+      enq = batch_start<KM>(C, opaque(A.elems) + C.e0, (uint64_t)(gi - C.begin), g, A.tame != 0, A.label_detected, m, lab,
+                            wc);
     }
     const uint64_t qm = __ballot(enq);
     if (enq) queue_put(P.q, gwave * P.region + qn + lanes_below(qm), m, c, 0);
@@ -550,12 +558,19 @@ __global__ void __launch_bounds__(256) k_batch_post(BArgs A, BPipe P) {
       queue_get_done(P.q, (int64_t)P.lt[BLT_LIST + j], m, key);
       c = (int)(key & QKEY_INDEX);
       const uint32_t status = (uint32_t)((key >> 40) & 0xff);
+      // x and y in registers of their own: this compiler (ROCm 7.2) keeps them in the 16 bytes they were loaded in and
+      // then overwrites y inside the walk's loop (its own -verify-machineinstrs reports it)
+      asm volatile("" : "+v"(m.x), "+v"(m.y));
       const BLensC &K = A.lensk[c];
       m.ax = 0.0;
       m.ay = -g;
       m.az = 0.0;
       label = A.label_detected;
-      walk_plain<KM>(opaque(A.elems) + K.e0, K.lens + 1, K.ne, g, m, label, wc);
+      const ctraj_elem *el = opaque(A.elems) + K.e0;
+      if (KM == KM_CIRC && ((A.tame != 0) & walk_tame(m)))
+        walk_circ_tame<false>(el, K.lens + 1, K.ne, g, m, recip(m.vz), label, wc);
+      else
+        walk_plain<KM>(el, K.lens + 1, K.ne, g, m, label, wc);
       n_oot += (status & CTRAJ_ST_OOT) ? 1u : 0u;
       n_cap += (status & CTRAJ_ST_CAPPED) ? 1u : 0u;
     }
@@ -595,6 +610,7 @@ struct ctraj_batch {
   bool uniform_dt = false;  // every lens has the same dt and folds its force scale (hex_folds)
   double dt = 0.0;
   int64_t slice = 0;        // molecules per slice of the split path
+  bool tame = false;        // walk_tame_elems over every configuration
   bool circ_only = false;   // only circular apertures (and lenses) in every configuration
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // captured launches by (block, chunk, grid, refill, fused)
@@ -624,6 +640,7 @@ static int batch_launch(ctraj_batch *b, int block, int chunk, int grid, int refi
   A.n_labels = b->n_labels;
   A.label_detected = b->label_detected;
   A.cap = b->cap;
+  A.tame = b->tame;
   A.chunk = chunk;
   A.refill_min = refill;
   const size_t hist_bytes = (size_t)b->n_cfg * b->n_labels * sizeof(uint32_t);
@@ -773,6 +790,7 @@ int32_t ctraj_batch_create(ctraj_ctx *c, const ctraj_elem *elems, int32_t n_elem
   b->uniform_dt = true;
   bool have_dt = false;
   bool all_fold = true;
+  b->tame = walk_tame_elems(elems, n_elems_total, b->g);
   b->circ_only = true;
   for (int e = 0; e < n_elems_total; ++e)
     if (elems[e].kind != CTRAJ_CIRC && elems[e].kind != CTRAJ_LENS) b->circ_only = false;
@@ -824,10 +842,13 @@ int32_t ctraj_batch_create(ctraj_ctx *c, const ctraj_elem *elems, int32_t n_elem
       b->d_pipe = nullptr;
     }
   }
-  // the device copy of the elements: circular apertures carry their squared-radius threshold
+  // the device copy of the elements: circular apertures carry their squared-radius threshold, lenses that of
+  // their entrance (a slot that spline forces do not use)
   std::vector<ctraj_elem> dev_elems(elems, elems + n_elems_total);
-  for (auto &E : dev_elems)
+  for (auto &E : dev_elems) {
     if (E.kind == CTRAJ_CIRC) E.p[1] = circ_r2_threshold(E.p[0]);
+    if (E.kind == CTRAJ_LENS) E.p[6] = circ_r2_threshold(E.p[0]);
+  }
   if (hipStreamSynchronize(c->stream) != hipSuccess ||
       (b->d_lensk && hipMemcpy(b->d_lensk, hl.data(), sizeof(BLensC) * n_cfgs, hipMemcpyHostToDevice) != hipSuccess) ||
       (b->d_ws && hipMemcpy(b->d_ws, c->d_ws, sizeof(double) * 4 * b->ws_nseg, hipMemcpyDeviceToDevice) != hipSuccess) ||

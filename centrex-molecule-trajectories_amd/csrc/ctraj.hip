@@ -113,6 +113,7 @@ struct PipeArgs {
   int n_pre_waves;
   unsigned long long *claim;   // lens kernel: eight claim counters, [8][32] (zeroed by PRE)
   int lens_e;
+  double lens_thr2;            // squared-radius threshold of the lens entrance (beyond_r2)
   // claim list (perm null: the lens kernel claims the regions in order)
   uint32_t *ord_tot;           // [ORD_BUCKETS] entries per bucket, then the list's entry count
   uint32_t *perm;              // queue slots in claim order
@@ -245,7 +246,7 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
   int64_t qn = 0;  // PRE: entries this wavefront has queued
   // PRE: the lens entrance, read once with scalar loads (a vector load of it in the loop would wait
   // for the prefetched molecules and the queue stores in flight)
-  double lens_z0 = 0.0, lens_r = 0.0;
+  double lens_z0 = 0.0;
   int lens_hit = 0;
   float ord_bore2 = 0.0f, ord_len = 0.0f, ord_h = 0.0f, ord_cap = 0.0f;  // lifetime prediction (P.bkt)
   if constexpr (PHASE == PHASE_PRE) {
@@ -257,7 +258,6 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
     }
     const ctraj_elem L = elem_at(B.elems, P.lens_e);
     lens_z0 = L.z0;
-    lens_r = L.p[0];
     lens_hit = L.label_hit;
     ord_bore2 = (float)L.p[1];
     ord_h = (float)L.p[2];
@@ -279,6 +279,8 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
                   (unsigned long long)(R.index_base + (int64_t)~P.lt[LT_FIRST]));
     }
   }
+  // no stored accelerations given: every molecule starts with (0, -g, 0)
+  const bool std_accel = !R.a0[0] && !R.a0[1] && !R.a0[2];
   const int64_t j0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t w0 = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63);
   // one grid-stride iteration: molecule j (inputs in q, loaded earlier), then q is refilled
@@ -316,16 +318,34 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
     bool enq = false;
     if (active) {
       if constexpr (PHASE == PHASE_FULL) {
-        NullSink sk;
-        walk<FORCE, INTEG, NullSink, KM, true>(B.elems, B.n_elems, T, B.g, B.cap, st, B.label_detected, m, label, status,
-                                         wc, sk);
+        if constexpr (INTEG == CTRAJ_INTEG_NONE && KM == KM_CIRC) {
+          label = B.label_detected;
+          if (B.tame & (MIN || std_accel) & walk_tame(m))
+            walk_circ_tame<true>(B.elems, 0, B.n_elems, B.g, m, recip(m.vz), label, wc);
+          else
+            walk_plain<KM, true>(B.elems, 0, B.n_elems, B.g, m, label, wc);
+        } else {
+          NullSink sk;
+          walk<FORCE, INTEG, NullSink, KM, true>(B.elems, B.n_elems, T, B.g, B.cap, st, B.label_detected, m, label,
+                                                 status, wc, sk);
+        }
       } else if constexpr (PHASE == PHASE_PRE) {
         label = B.label_detected;
-        if (walk_plain<KM, true>(B.elems, 0, P.lens_e, B.g, m, label, wc)) {
-          drift_dt(m, time_to(m, lens_z0), B.g);  // lens entrance (electrostatic_lens.py:59-64)
+        // to and through the lens entrance (electrostatic_lens.py:59-64)
+        if (KM == KM_CIRC && (B.tame & (MIN || std_accel) & walk_tame(m))) {
+          const double iv = recip(m.vz);
+          enq = walk_circ_tame<true>(B.elems, 0, P.lens_e, B.g, m, iv, label, wc);
+          if (enq) drift_tame(m, lens_z0, iv, B.g);
+        } else {
+          enq = walk_plain<KM, true>(B.elems, 0, P.lens_e, B.g, m, label, wc);
+          if (enq) drift_dt(m, time_to(m, lens_z0), B.g);
+        }
+        if (enq) {
           ++wc.faces;
-          if (rho_of(m.x, m.y) > lens_r) label = lens_hit;
-          else enq = true;
+          if (beyond_r2(m.x, m.y, P.lens_thr2)) {
+            label = lens_hit;
+            enq = false;
+          }
         }
       } else if constexpr (PHASE == PHASE_POST) {
         if (outcome == LENS_LEFT) {
@@ -334,7 +354,10 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
           m.ax = 0.0; m.ay = -B.g; m.az = 0.0;
           label = B.label_detected;
           const uint32_t f0 = wc.faces;
-          walk_plain<KM, true>(B.elems, P.lens_e + 1, B.n_elems, B.g, m, label, wc);
+          if (KM == KM_CIRC && (B.tame & walk_tame(m)))
+            walk_circ_tame<true>(B.elems, P.lens_e + 1, B.n_elems, B.g, m, recip(m.vz), label, wc);
+          else
+            walk_plain<KM, true>(B.elems, P.lens_e + 1, B.n_elems, B.g, m, label, wc);
           faces_post += wc.faces - f0;
         } else {
           label = lens_inside;
@@ -1274,7 +1297,7 @@ int check_phys(ctraj_ctx *ctx, const ctraj_phys *p) {
   return CTRAJ_OK;
 }
 
-KBeam make_kbeam(const ctraj_elem *d_elems, int n, const ctraj_phys &p) {
+KBeam make_kbeam(const ctraj_elem *d_elems, const ctraj_elem *h_elems, int n, const ctraj_phys &p) {
   KBeam b;
   b.elems = d_elems;
   b.n_elems = n;
@@ -1283,6 +1306,7 @@ KBeam make_kbeam(const ctraj_elem *d_elems, int n, const ctraj_phys &p) {
   b.label_detected = p.label_detected;
   b.n_states = p.n_states;
   b.cap = p.max_lens_steps > 0 ? p.max_lens_steps : (1 << 20);
+  b.tame = walk_tame_elems(h_elems, n, p.g);
   return b;
 }
 
@@ -1527,7 +1551,7 @@ static int32_t propagate_impl(ctraj_ctx *c, const ctraj_run *R, char *sdev) {
   KTab kt = ctx_ktab(c);
   if (c->force == CTRAJ_FORCE_RTABLE) kt.ws_states = 0;
   const size_t lds = ktab_lds_bytes(kt);
-  KBeam B = make_kbeam(c->d_elems, c->n_elems, c->phys);
+  KBeam B = make_kbeam(c->d_elems, c->h_elems.data(), c->n_elems, c->phys);
   int n_lens = 0, lens_e = -1;
   for (int e = 0; e < c->n_elems; ++e)
     if (c->h_elems[e].kind == CTRAJ_LENS) {
@@ -1633,6 +1657,7 @@ static int32_t propagate_impl(ctraj_ctx *c, const ctraj_run *R, char *sdev) {
     const int64_t threads = (int64_t)gpre * blk;
     P.n_pre_waves = gpre * (blk / 64);
     P.lens_e = lens_e;
+    P.lens_thr2 = circ_r2_threshold(c->h_elems[lens_e].p[0]);
     if (list) {
       const size_t cap = (size_t)threads * (size_t)((slice + threads - 1) / threads);
       const size_t b_bkt = ordered ? (cap + 255) & ~(size_t)255 : 0, b_perm = cap * 4, b_tot = 2048;
@@ -2119,7 +2144,7 @@ int32_t ctraj_record_trajectories(ctraj_ctx *c, const ctraj_record *RC) {
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
   const int grid = grid_for(c, (const void *)k, block, lds, RC->n, 0);
-  KBeam B = make_kbeam(c->d_elems, c->n_elems, c->phys);
+  KBeam B = make_kbeam(c->d_elems, c->h_elems.data(), c->n_elems, c->phys);
   hipLaunchKernelGGL(k, dim3(grid), dim3(block), lds, c->stream, B, kt, *RC);
   HIPCHK(c, hipGetLastError());
   return CTRAJ_OK;

@@ -80,6 +80,7 @@ struct KBeam {
   int n_elems;
   double g;
   int n_labels, label_detected, n_states, cap;
+  int tame;  // every face and g are of moderate size (walk_tame_elems)
 };
 
 struct KTab {
@@ -102,7 +103,7 @@ void resolve_elems(const ctraj_ctx *ctx, const ctraj_elem *e, int n, ctraj_elem 
 // when r2 > circ_r2_threshold(d).  Device element tables keep it in a circular aperture's p[1].
 double circ_r2_threshold(double d);
 int check_phys(ctraj_ctx *ctx, const ctraj_phys *p);
-KBeam make_kbeam(const ctraj_elem *d_elems, int n, const ctraj_phys &p);
+KBeam make_kbeam(const ctraj_elem *d_elems, const ctraj_elem *h_elems, int n, const ctraj_phys &p);
 int lds_limit(ctraj_ctx *ctx, const void *kern, size_t bytes);
 int grid_for(ctraj_ctx *ctx, const void *kern, int block, size_t lds, int64_t n, int req);
 // EINVAL unless `block` threads fit the kernel's launch bounds

@@ -34,6 +34,81 @@ struct LaneMol {
   double h, hp, dzs, r2;  // current step, final partial step, z advance per full step, x^2 + y^2
 };
 
+// ---- circular apertures, the common case arranged for few instructions ----
+// A face costs 45 VALU instructions as walk_plain writes it (14 of them the division by vz, 10 the products with
+// the zero components of the acceleration), and a wavefront runs nearly every face of the beamline.  With
+// a = (0, -g, 0) and faces, z, vz and g of moderate size (walk_tame_elems on the host, walk_tame per molecule) the
+// same values come from 22:
+//   * every face's time is the correctly rounded (zf - z) / vz from one reciprocal of vz, by the last two
+//     operations of the hardware's own division sequence (nothing needs its scaling: a face is nonzero, so zf - z
+//     is zero or at least 2^-160);
+//   * 0 dt^2 / 2 and 0 dt add +0, which changes only a -0 (walk_tame sends x or vx = -0 the plain way);
+//   * (a dt^2) / 2 is exact and goes with its sum into one fused operation; dt = 0 changes
+//     nothing (velocities are bounded).
+// 5 10^7 molecules without a lens: 682 -> 581 us (4.1 TB/s of inputs).
+constexpr double kWalkLo = 0x1p-100, kWalkHi = 0x1p100;
+
+__host__ __device__ __forceinline__ bool walk_tame_value(double v) {
+  const double a = __builtin_fabs(v);
+  return a >= kWalkLo && a < kWalkHi;
+}
+
+// The element table's part of the condition: circular apertures (elements in between are not looked at) and lens
+// entrances on faces of moderate size, g moderate or zero.
+inline bool walk_tame_elems(const ctraj_elem *e, int n, double g) {
+  bool ok = g == 0.0 || walk_tame_value(g);
+  for (int i = 0; i < n; ++i) ok = ok && walk_tame_value(e[i].z0) && walk_tame_value(e[i].z1);
+  return ok;
+}
+
+__device__ __forceinline__ uint32_t high_word(double v) { return (uint32_t)((uint64_t)__double_as_longlong(v) >> 32); }
+// false for -0 (and the smallest negative numbers)
+__device__ __forceinline__ bool not_neg_zero(double v) { return high_word(v) != 0x80000000u; }
+// |v| < 2^1000: v dt is 0 where dt is
+__device__ __forceinline__ bool bounded(double v) { return high_word(v) << 1 < (uint32_t)(1023 + 1000) << 21; }
+
+// The molecule's part: its acceleration is (0, -g, 0) (the caller's knowledge).
+__device__ __forceinline__ bool walk_tame(const MState &m) {
+  return walk_tame_value(m.vz) & ((m.z == 0.0) | walk_tame_value(m.z)) & not_neg_zero(m.x) & not_neg_zero(m.vx) &
+         bounded(m.vx) & bounded(m.vy);
+}
+
+// 1 / v to within an ulp (v moderate).
+__device__ __forceinline__ double recip(double v) {
+  double y = __builtin_amdgcn_rcp(v);
+  y = __builtin_fma(__builtin_fma(-v, y, 1.0), y, y);
+  return __builtin_fma(__builtin_fma(-v, y, 1.0), y, y);
+}
+
+// Drift of a tame molecule to the plane zf (iv = recip(vz)); the acceleration stays (0, -g, 0).
+__device__ __forceinline__ void drift_tame(MState &m, double zf, double iv, double g) {
+  const double a = zf - m.z, q = a * iv;
+  const double dt = __builtin_fma(__builtin_fma(-m.vz, q, a), iv, q);
+  m.x = m.x + m.vx * dt;
+  m.y = __builtin_fma(0.5, (-g) * (dt * dt), m.y + m.vy * dt);
+  m.z = m.z + m.vz * dt;
+  m.vy = m.vy + (-g) * dt;
+  m.t = m.t + dt;
+}
+
+// walk_plain over circular apertures for a tame molecule.
+template <bool SE>
+__device__ __forceinline__ bool walk_circ_tame(const ctraj_elem *__restrict__ elems, int e0, int e1, double g, MState &m,
+                                               double iv, int &label, WalkCounters &wc) {
+  for (int e = e0; e < e1; ++e) {
+    const ctraj_elem E = elem_get<SE>(elems, e);
+    const int lhit = SE ? stop_label(E.label_hit) : E.label_hit;
+    const double thr2 = E.p[1];
+    drift_tame(m, E.z0, iv, g);
+    ++wc.faces;
+    if (beyond_r2(m.x, m.y, thr2)) { label = lhit; return false; }
+    drift_tame(m, E.z1, iv, g);
+    ++wc.faces;
+    if (beyond_r2(m.x, m.y, thr2)) { label = lhit; return false; }
+  }
+  return true;
+}
+
 // Walk elements [e0, e1) (no lens among them) from the molecule's current row.  Returns false if
 // the molecule stopped (label set).
 template <int KM = KM_ALL, bool SE = false>
