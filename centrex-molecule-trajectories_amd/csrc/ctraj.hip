@@ -166,12 +166,19 @@ __device__ __forceinline__ void load_entry(const PipeArgs &P, int64_t e, InMol &
   q.st = (int)((uint64_t)key >> 56);
 }
 
-// POST's item j: with lens tallies the j-th listed slot, else queue slot j (entry k of PRE wavefront
-// w's region; slots past the region's count are empty).
+// POST's item j: with lens tallies the j-th listed slot, with a claim list in queue order its j-th slot, else
+// queue slot j (entry k of PRE wavefront w's region; slots past the region's count are empty).  The
+// longest-first list would read the queue's entries in scattered order.
+__device__ __forceinline__ bool post_by_list(const PipeArgs &P) { return P.perm && !P.bkt; }
+
 __device__ __forceinline__ void load_slot(const PipeArgs &P, int64_t j, InMol &q) {
   q.outcome = LENS_QUEUED;
   if (P.lt) {
     load_entry(P, (int64_t)P.lt[LT_LIST + j], q);
+    return;
+  }
+  if (post_by_list(P)) {
+    load_entry(P, (int64_t)P.perm[j], q);
     return;
   }
   const int64_t w = j / P.region;
@@ -194,18 +201,23 @@ __device__ __forceinline__ void load_min(const ctraj_run &R, int64_t i, InMol &q
 // ahead (and the constant time, acceleration and state are not carried per molecule).
 template <int FORCE, int INTEG, int PHASE, int KM, bool OUT, bool MIN = false>
 __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R, int aoi_lds_off, PipeArgs P) {
-  // POST: the listed slots (lens tallies), else every slot of the queue
-  const int64_t n_items =
-      PHASE == PHASE_POST ? (P.lt ? (int64_t)P.lt[LT_N] : (int64_t)P.n_pre_waves * P.region) : R.n;
-  // POST with lens tallies: the grid is sized for every slot of the queue, but the listed slots are
-  // usually a few per cent of them; only as many workgroups as give each thread about POST_ITEMS
-  // slots take part (the others leave at once; the first also merges the lens kernel's tallies
-  // below), which keeps the same-address atomics of the workgroups' final flushes few
+  // POST: the listed slots (lens tallies, or a claim list in queue order), else every slot of the queue
+  const int64_t n_items = PHASE != PHASE_POST ? R.n
+                          : P.lt              ? (int64_t)P.lt[LT_N]
+                          : post_by_list(P)   ? (int64_t)P.ord_tot[ORD_BUCKETS]
+                                              : (int64_t)P.n_pre_waves * P.region;
+  // POST with a list: the grid is sized for every slot of the queue, but the listed slots are
+  // usually a few per cent of them; only as many workgroups as give each thread about POST_ITEMS slots
+  // take part, or one slot while that takes at most 128 workgroups (the others leave at once; the first
+  // also merges the lens kernel's tallies below), which keeps the same-address atomics of the workgroups'
+  // final flushes few (the reference's example, 5.3e3 listed of 10^6: 23 us over all slots, 12 by list)
   int64_t n_wg = gridDim.x;
   if constexpr (PHASE == PHASE_POST) {
-    if (P.lt) {
-      const int64_t per_wg = (int64_t)blockDim.x * POST_ITEMS;
-      n_wg = std::min<int64_t>(gridDim.x, std::max<int64_t>(1, (n_items + per_wg - 1) / per_wg));
+    if (P.lt || post_by_list(P)) {
+      const int64_t one = (n_items + blockDim.x - 1) / blockDim.x;  // workgroups for one slot a thread
+      n_wg = std::min<int64_t>(gridDim.x,
+                               std::max<int64_t>(std::min<int64_t>(std::max<int64_t>(one, 1), 128),
+                                                 (one + POST_ITEMS - 1) / POST_ITEMS));
       if (blockIdx.x >= n_wg) return;
     }
   }

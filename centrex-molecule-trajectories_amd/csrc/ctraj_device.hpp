@@ -332,17 +332,19 @@ __device__ __forceinline__ void ref_step_plain(const Force<FORCE> &F, const Tabl
 // shared pieces:
 //   * sqrt: the compiler's own Goldschmidt sequence without the scaling; its half reciprocal h1, refined
 //     once against r, is the reciprocal that both divisions by r share;
-//   * a quotient n / d from y = 1/d (relative error at most 2^-53): q = n y, then q + (n - q d) y, the
-//     final two operations of the hardware's division sequence, with v_div_fixup for zeros, infinities and
-//     NaN;
+//   * a quotient n / d from y = 1/d (relative error at most 2^-53): q near n y, then q + (n - q d) y, the
+//     final two operations of the hardware's division sequence (q = a_r (x y) is ready one operation after
+//     a_r);
 //   * n / 6 likewise from the constant 1/6 (its error is a quarter of an ulp, so q is within one ulp and the
 //     corrected quotient is the correctly rounded one);
-//   * the table segment is guessed from the square root's first iterate (2^-46) while the rest of it is
-//     computed, and checked against the final r;
+//   * the table segment is guessed from the first estimate of the square root while it is refined, and checked
+//     against the final r;
 //   * 2 a and a / 2 are exact, so each goes with its sum into one fused operation;
 //   * vz does not change and z advances by a step-independent amount.
+// The quotients' zeros may have the wrong sign, which is lost where they are added to a nonzero velocity or
+// coordinate; the first stage's force, which the row stores, takes v_div_fixup and the knot's own value.
 // A lane whose state is not tame (an exactly zero coordinate is not), whose segment was not the guessed
-// one or that leaves the table takes the plain step.  One wavefront per SIMD: 1.5 -> 0.66 us a step.
+// one or that leaves the table takes the plain step.  One wavefront per SIMD: 1.5 -> 0.64 us a step.
 __device__ __forceinline__ uint32_t abs_exponent(double v) {
   return (uint32_t)((uint64_t)__double_as_longlong(v) >> 32) << 1;
 }
@@ -354,36 +356,44 @@ __host__ __device__ __forceinline__ bool tame_value(double v) {
   return a >= 0x1p-200 && a < 0x1p200;
 }
 
-__device__ __forceinline__ double quotient(double n, double d, double y) {
-  const double q = n * y;
-  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d, q, n), y, q), d, n);
+// n / d from y = 1/d and an estimate q of the quotient, zeros' signs aside.
+__device__ __forceinline__ double quotient(double n, double d, double y, double q) {
+  return __builtin_fma(__builtin_fma(-d, q, n), y, q);
 }
 
-__device__ __forceinline__ double sixth(double n) { return quotient(n, 6.0, 1.0 / 6.0); }
+__device__ __forceinline__ double sixth(double n) { return quotient(n, 6.0, 1.0 / 6.0, n * (1.0 / 6.0)); }
 
-// force_rtable where r^2 is a moderate number and r lies in the guessed segment (returned).
+// force_rtable where r^2 is a moderate number and r lies in the guessed segment (returned).  STORED: the force
+// is a row's acceleration.
+template <bool STORED>
 __device__ __forceinline__ bool force_rtable_fast(const Tables &T, const RDesc &D, double g, double x, double y,
                                                   double &ax, double &ay) {
   const double r2 = x * x + y * y;
   const double s = __builtin_amdgcn_rsq(r2);
   const double g0 = r2 * s, h0 = 0.5 * s;
-  const double e0 = __builtin_fma(-h0, g0, 0.5);
-  const double h1 = __builtin_fma(h0, e0, h0), g1 = __builtin_fma(g0, e0, g0);
-  const double u = (g1 - D.r0) * D.invh;
+  const double u = __builtin_fma(g0, D.invh, -D.r0 * D.invh);
   uint32_t j;  // saturating: 0 for a negative or NaN u
   asm("v_cvt_u32_f64 %0, %1" : "=v"(j) : "v"(u));
-  j = min(j, (uint32_t)(D.n - 2));
-  const lds_double *rec = T.rt + 4 * ((uint32_t)D.off + j);
+  const lds_double *rec = (T.rt + 4 * D.off) + 4 * min(j, (uint32_t)(D.n - 2));
   const dbl2_t ra = *(const lds_dbl2 *)rec;
   const double slope = rec[2], rn = rec[4];
+  const double e0 = __builtin_fma(-h0, g0, 0.5);
+  const double h1 = __builtin_fma(h0, e0, h0), g1 = __builtin_fma(g0, e0, g0);
   const double g2 = __builtin_fma(__builtin_fma(-g1, g1, r2), h1, g1);
   const double r = __builtin_fma(__builtin_fma(-g2, g2, r2), h1, g2);
   const double y0 = h1 + h1;
   const double iy = __builtin_fma(__builtin_fma(-r, y0, 1.0), y0, y0);
-  const double t = slope * (r - ra.x) + ra.y;
-  const double ar = r == ra.x ? ra.y : t;
-  ax = quotient(ar * x, r, iy);
-  ay = quotient(ar * y, r, iy) - g;
+  const double xi = x * iy, yi = y * iy;
+  double ar = slope * (r - ra.x) + ra.y;
+  if constexpr (STORED) ar = r == ra.x ? ra.y : ar;
+  const double nx = ar * x, ny = ar * y;
+  ax = quotient(nx, r, iy, ar * xi);
+  ay = quotient(ny, r, iy, ar * yi);
+  if constexpr (STORED) {
+    ax = __builtin_amdgcn_div_fixup(ax, r, nx);
+    ay = __builtin_amdgcn_div_fixup(ay, r, ny);
+  }
+  ay = ay - g;
   return (ra.x <= r) & (r < rn) & (r2 >= 0x1p-700);
 }
 
@@ -397,13 +407,13 @@ __device__ __forceinline__ void ref_step(const Force<FORCE> &F, const Tables &T,
               tame_value(m.vz) & tame_value(dt);
     const double x = m.x, y = m.y, k1x = m.vx, k1y = m.vy;
     double l1x, l1y, l2x, l2y, l3x, l3y, l4x, l4y;
-    ok &= force_rtable_fast(T, F.d, F.g, x, y, l1x, l1y);
+    ok &= force_rtable_fast<true>(T, F.d, F.g, x, y, l1x, l1y);
     const double k2x = __builtin_fma(0.5, dt * l1x, k1x), k2y = __builtin_fma(0.5, dt * l1y, k1y);
-    ok &= force_rtable_fast(T, F.d, F.g, x + dt * k1x, y + dt * k1y, l2x, l2y);
+    ok &= force_rtable_fast<false>(T, F.d, F.g, x + dt * k1x, y + dt * k1y, l2x, l2y);
     const double k3x = __builtin_fma(0.5, dt * l2x, k1x), k3y = __builtin_fma(0.5, dt * l2y, k1y);
-    ok &= force_rtable_fast(T, F.d, F.g, __builtin_fma(0.5, dt * k2x, x), __builtin_fma(0.5, dt * k2y, y), l3x, l3y);
+    ok &= force_rtable_fast<false>(T, F.d, F.g, __builtin_fma(0.5, dt * k2x, x), __builtin_fma(0.5, dt * k2y, y), l3x, l3y);
     const double k4x = k1x + dt * l3x, k4y = k1y + dt * l3y;
-    ok &= force_rtable_fast(T, F.d, F.g, x + dt * k3x, y + dt * k3y, l4x, l4y);
+    ok &= force_rtable_fast<false>(T, F.d, F.g, x + dt * k3x, y + dt * k3y, l4x, l4y);
     if (ok) {
       const double kx = __builtin_fma(2.0, k3x, __builtin_fma(2.0, k2x, k1x)) + k4x;
       const double ky = __builtin_fma(2.0, k3y, __builtin_fma(2.0, k2y, k1y)) + k4y;
