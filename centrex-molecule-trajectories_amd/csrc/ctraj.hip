@@ -210,7 +210,7 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
   // usually a few per cent of them; only as many workgroups as give each thread about POST_ITEMS slots
   // take part, or one slot while that takes at most 128 workgroups (the others leave at once; the first
   // also merges the lens kernel's tallies below), which keeps the same-address atomics of the workgroups'
-  // final flushes few (the reference's example, 5.3e3 listed of 10^6: 23 us over all slots, 12 by list)
+  // final flushes few (the reference's example, 5.3e3 listed of 10^6: 21.8 us over all slots, 12.7 by list)
   int64_t n_wg = gridDim.x;
   if constexpr (PHASE == PHASE_POST) {
     if (P.lt || post_by_list(P)) {
