@@ -365,16 +365,17 @@ __global__ void __launch_bounds__(256) k_batch_pre(BArgs A, BPipe P) {
 
 // Split scan, phase 2: persistent wavefronts integrate the queued molecules through their
 // configuration's lens with lane refill and write each molecule's state where the lens left it back
-// into its queue entry, with its outcome (the single-run lens kernel's scheme, with the lens
+// into its queue entry, with its status (the single-run lens kernel's scheme, with the lens
 // constants per lane: the configuration's lens constants staged in LDS, its field constants and
-// step in the lane's registers).  A lane's rem is its full steps left (> 0), 0 at the lens end (one
-// partial step of L/vz - n dt to go), REM_STOPPED once the bore stopped it, REM_EMPTY when it holds
-// no molecule.  UH: every configuration's lens has the same dt and folds its force scale (the folded
-// step's constants, hex_k of the lens's ks and dt, are formed per molecule); otherwise each step
-// chooses the folded or the plain RK4 step for its molecule's lens (lens_step).  The arithmetic per
-// molecule is the one of k_batch_lanes.
+// step in the lane's registers).  A lane's rem is 1 while it has full steps to take (until the
+// wavefront's step counter reaches ends_at), 0 at the lens end (one partial step of L/vz - n dt to go),
+// BREM_STOPPED once the bore stopped it, BREM_EMPTY when it holds no molecule.  The lanes that step
+// are a scalar mask, so the step loop spends no vector instruction on the count.  (The partial step
+// as one more turn of the loop, with the lane's own step constants, measured 0.4 % slower.)  UH: every
+// configuration's lens has the same dt and folds its force scale (the folded step's constants, hex_k of
+// the lens's ks and dt, are formed per molecule); otherwise each step chooses the folded or the plain
+// RK4 step for its molecule's lens (lens_step).  The arithmetic per molecule is the one of k_batch_lanes.
 constexpr int BREM_EMPTY = -1, BREM_STOPPED = -2;
-enum : int { BLENS_STOPPED = 1, BLENS_LEFT = 2 };
 
 template <bool UH>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(UH ? 6 : 1)))
@@ -399,6 +400,7 @@ k_batch_integ(BArgs A, BPipe P, KTab KT) {
   uint32_t steps_w = 0;  // wave-uniform
   int64_t next = 0, end = 0;
   bool exhausted = false;
+  uint32_t pend = 0, n_pend = 0;  // lanes below n_pend (wave-uniform) hold a slot for the list
 
   MState m;
   m.x = m.y = m.z = m.vx = m.vy = m.vz = m.t = 0.0;
@@ -407,112 +409,146 @@ k_batch_integ(BArgs A, BPipe P, KTab KT) {
   double r2 = 0.0, ks = 0.0, cu = 0.0, gk = 0.0, R2 = 0.0, Hs = A.Hs;
   HexK hk{};  // UH: the folded step's constants of the molecule's lens
   int rem = BREM_EMPTY, nfull = 0, c = 0;
+  uint32_t it = 0, ends_at = 0;  // the wavefront's steps so far, and where this molecule's full steps end
   uint32_t status = 0;
   int64_t slot = 0, key = 0;
 
   for (;;) {
-    bool act = rem > 0;
-    uint64_t am = __builtin_amdgcn_ballot_w64(act);
-    if (64 - __popcll(am) >= A.refill_min) {
-      for (;;) {
-        // finish the molecules that take no more full steps: stopped by the bore, or at the lens end
-        // with its partial step to take
-        const bool fin = rem == 0 || rem == BREM_STOPPED;
-        steps_w += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(rem == 0));
-        if (fin) {
-          int outcome = BLENS_STOPPED;
-          if (rem == 0) {
-            const BLensC &K = s_cfg[c];
-            const double hp = K.Ll / m.vz - (double)nfull * Hs;
-            const Force<CTRAJ_FORCE_WSPLINE_HEX> F{ks, cu, g, gk};
-            lens_step<CTRAJ_FORCE_WSPLINE_HEX>(F, T, wsb, hp, m.x, m.y, m.vx, m.vy, r2, status);
-            m.z = K.z1;
-            m.t = __builtin_fma((double)nfull, Hs, m.t) + hp;
-            r2 = __builtin_fma(m.x, m.x, m.y * m.y);
-            outcome = r2 > R2 ? BLENS_STOPPED : BLENS_LEFT;
-          }
-          if (outcome == BLENS_STOPPED) {  // counted here: the molecule needs no further walk
-            atomicAdd(&s_stop[c], 1u);
-            if (status) {
-              if (status & CTRAJ_ST_OOT) atomicAdd(&s_stop[A.n_cfg], 1u);
-              if (status & CTRAJ_ST_CAPPED) atomicAdd(&s_stop[A.n_cfg + 1], 1u);
-            }
-          } else {
-            queue_put_done(P.q, slot, m.x, m.y, m.z, m.vx, m.vy, m.vz, m.t,
-                           key | ((int64_t)status << 40) | ((int64_t)outcome << 48));
-            // list the slot for phase 3: one atomic per wavefront, by its first lane here
-            const uint64_t lm = __builtin_amdgcn_ballot_w64(true);
-            const int rank = lanes_below(lm);
-            uint32_t base = 0;
-            if (rank == 0) base = atomicAdd(&P.lt[0], (uint32_t)__popcll(lm));
-            base = __builtin_amdgcn_readfirstlane(base);
-            P.lt[BLT_LIST + base + (uint32_t)rank] = (uint32_t)slot;
-          }
-          rem = BREM_EMPTY;
+    for (;;) {
+      // the molecules that take no more full steps: stopped by the bore, or at the lens end with the
+      // partial step to take, which the bore may stop too
+      const bool fin = rem == 0 || rem == BREM_STOPPED;
+      steps_w += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(rem == 0));
+      if (rem == 0) {
+        const BLensC &K = s_cfg[c];
+        const double hp = K.Ll / m.vz - (double)nfull * Hs;
+        const Force<CTRAJ_FORCE_WSPLINE_HEX> F{ks, cu, g, gk};
+        lens_step<CTRAJ_FORCE_WSPLINE_HEX>(F, T, wsb, hp, m.x, m.y, m.vx, m.vy, r2, status);
+        m.z = K.z1;
+        m.t = __builtin_fma((double)nfull, Hs, m.t) + hp;
+        r2 = __builtin_fma(m.x, m.x, m.y * m.y);
+        if (r2 > R2) rem = BREM_STOPPED;
+      }
+      const uint64_t lm = __builtin_amdgcn_ballot_w64(rem == 0);
+      if (lm) {
+        // list the slots of those that leave for phase 3, 64 per reservation: one reservation per section is
+        // an atomic on one address from every XCD, some 15 ns apart, which held up the sections (a scan of
+        // 256 configurations refilling at 12 idle lanes: 72 % of issue cycles, 14.1 ms; now 11.7)
+        const uint32_t n = (uint32_t)__popcll(lm);
+        const bool left = lane_in(lm);
+        // a permutation of the lanes: the leaving ones onto lanes n_pend, n_pend + 1, ... (cyclic)
+        const uint32_t to = n_pend + (left ? (uint32_t)lanes_below(lm) : n + (uint32_t)lanes_below(~lm));
+        const uint32_t got = (uint32_t)__builtin_amdgcn_ds_permute((int)((to & 63u) * 4u), (int)(uint32_t)slot);
+        const uint32_t full = n_pend + n;
+        if ((uint32_t)lane >= n_pend && (uint32_t)lane < full) pend = got;
+        if (full >= 64u) {
+          uint32_t base = 0;
+          if (lane == 0) base = atomicAdd(&P.lt[0], 64u);
+          base = __builtin_amdgcn_readfirstlane(base);
+          P.lt[BLT_LIST + base + (uint32_t)lane] = pend;
+          if ((uint32_t)lane < full - 64u) pend = got;
         }
-        const uint64_t need = __builtin_amdgcn_ballot_w64(rem == BREM_EMPTY);
-        if (!need || exhausted) break;
-        if (next >= end) {
-          unsigned long long cl = 0;
-          if (lane == 0) cl = atomicAdd(P.claim + 32 * grp, 1ull);
-          cl = uniform_u64(cl);  // every lane is active here, lane 0 first
-          if (cl >= n_chunks) {
-            if (++tried == 8) exhausted = true;
-            grp = (grp + 1) & 7;
-            continue;
+        n_pend = full & 63u;
+      }
+      if (fin) {
+        if (rem == BREM_STOPPED) {  // counted here: the molecule needs no further walk
+          atomicAdd(&s_stop[c], 1u);
+          if (status) {
+            if (status & CTRAJ_ST_OOT) atomicAdd(&s_stop[A.n_cfg], 1u);
+            if (status & CTRAJ_ST_CAPPED) atomicAdd(&s_stop[A.n_cfg + 1], 1u);
           }
-          const uint32_t r = (uint32_t)cl / cpr;
-          const uint32_t w = ((r >> 2) << 5) | ((uint32_t)grp << 2) | (r & 3u);
-          const int64_t base = (int64_t)((uint32_t)cl - r * cpr) * 64;
-          const int64_t filled = (int64_t)P.wcount[w] - base;
-          next = (int64_t)w * P.region + base;
-          end = next + (filled < 64 ? filled : 64);  // next >= end: an empty chunk, claim again
+        } else {
+          queue_put_done(P.q, slot, m.x, m.y, m.z, m.vx, m.vy, m.vz, m.t,
+                         key | ((int64_t)status << 40));
+        }
+        rem = BREM_EMPTY;
+      }
+      const uint64_t need = __builtin_amdgcn_ballot_w64(rem == BREM_EMPTY);
+      if (!need || exhausted) break;
+      if (next >= end) {
+        unsigned long long cl = 0;
+        if (lane == 0) cl = atomicAdd(P.claim + 32 * grp, 1ull);
+        cl = uniform_u64(cl);  // every lane is active here, lane 0 first
+        if (cl >= n_chunks) {
+          if (++tried == 8) exhausted = true;
+          grp = (grp + 1) & 7;
           continue;
         }
-        const int64_t avail = end - next;
-        if (rem == BREM_EMPTY) {
-          const int rank = lanes_below(need);
-          if (rank < avail) {
-            slot = next + rank;
-            queue_get_done(P.q, slot, m, key);
-            c = (int)(key & QKEY_INDEX);
-            const BLensC &K = s_cfg[c];
-            ks = K.ks;
-            cu = K.cu;
-            gk = K.gk;
-            R2 = K.R2;
-            if constexpr (!UH) Hs = K.Hs;
-            if constexpr (UH) {
-              hk = hex_k(ks, Hs);
-            }
-            status = 0;
-            nfull = rk4_full_steps(K.Ll, m.vz, Hs, A.cap, status);
-            r2 = __builtin_fma(m.x, m.x, m.y * m.y);
-            rem = nfull;
-          }
-        }
-        next += avail < (int64_t)__popcll(need) ? avail : (int64_t)__popcll(need);
+        const uint32_t r = (uint32_t)cl / cpr;
+        const uint32_t w = ((r >> 2) << 5) | ((uint32_t)grp << 2) | (r & 3u);
+        const int64_t base = (int64_t)((uint32_t)cl - r * cpr) * 64;
+        const int64_t filled = (int64_t)P.wcount[w] - base;
+        next = (int64_t)w * P.region + base;
+        end = next + (filled < 64 ? filled : 64);  // next >= end: an empty chunk, claim again
+        continue;
       }
-      act = rem > 0;
-      am = __builtin_amdgcn_ballot_w64(act);
-      if (!am) break;  // the queue is exhausted and every molecule has been written back
+      const int64_t avail = end - next;
+      if (rem == BREM_EMPTY) {
+        const int rank = lanes_below(need);
+        if (rank < avail) {
+          slot = next + rank;
+          queue_get_done(P.q, slot, m, key);
+          c = (int)(key & QKEY_INDEX);
+          const BLensC &K = s_cfg[c];
+          ks = K.ks;
+          cu = K.cu;
+          gk = K.gk;
+          R2 = K.R2;
+          if constexpr (!UH) Hs = K.Hs;
+          if constexpr (UH) {
+            hk = hex_k(ks, Hs);
+          }
+          status = 0;
+          nfull = rk4_full_steps(K.Ll, m.vz, Hs, A.cap, status);
+          r2 = __builtin_fma(m.x, m.x, m.y * m.y);
+          rem = nfull > 0 ? 1 : 0;
+          ends_at = it + (uint32_t)nfull;
+        }
+      }
+      next += avail < (int64_t)__popcll(need) ? avail : (int64_t)__popcll(need);
     }
 
-    steps_w += (uint32_t)__popcll(am);
-    if (act) {
-      if constexpr (UH) {
-        rk4_step_hex_k(wsb, T.umax, cu, gk, hk, m.x, m.y, m.vx, m.vy, r2);
-      } else {
-        const Force<CTRAJ_FORCE_WSPLINE_HEX> F{ks, cu, g, gk};
-        lens_step<CTRAJ_FORCE_WSPLINE_HEX>(F, T, wsb, Hs, m.x, m.y, m.vx, m.vy, r2, status);
+    uint64_t am = __builtin_amdgcn_ballot_w64(rem > 0);  // the lanes that take full steps
+    if (!am) break;  // the queue is exhausted and every molecule has been written back
+    uint32_t cnt = (uint32_t)__popcll(am);
+    // idle lanes wait for a refill only while there is something to claim
+    const uint32_t keep = __builtin_amdgcn_readfirstlane(exhausted ? 0 : 64 - A.refill_min);
+    do {
+      steps_w += cnt;
+      ++it;
+      if (lane_in(am)) {
+        if constexpr (UH) {
+          rk4_step_hex_k(wsb, T.umax, cu, gk, hk, m.x, m.y, m.vx, m.vy, r2);
+        } else {
+          const Force<CTRAJ_FORCE_WSPLINE_HEX> F{ks, cu, g, gk};
+          lens_step<CTRAJ_FORCE_WSPLINE_HEX>(F, T, wsb, Hs, m.x, m.y, m.vx, m.vy, r2, status);
+        }
+        r2 = __builtin_fma(m.x, m.x, m.y * m.y);
       }
-      r2 = __builtin_fma(m.x, m.x, m.y * m.y);
-      rem = r2 > R2 ? BREM_STOPPED : rem - 1;
-    }
+      const bool out = r2 > R2;  // beyond the bore (lanes outside am: whatever)
+      const uint64_t over = am & (__builtin_amdgcn_ballot_w64(out) | __builtin_amdgcn_ballot_w64(ends_at == it));
+      if (over) {
+        if (lane_in(over)) rem = out ? BREM_STOPPED : 0;
+        am &= ~over;
+        cnt = (uint32_t)__popcll(am);
+      }
+    } while (cnt > keep);
   }
 
   if (lane == 0 && steps_w) atomicAdd(&s_steps, (unsigned long long)steps_w);
+  // the wavefronts' last, partly filled entries of the list: one reservation per workgroup, in the place
+  // of the tables, which no wavefront reads any more
   __syncthreads();
+  uint32_t *s_list = reinterpret_cast<uint32_t *>(lds);
+  if (threadIdx.x == 0) s_list[0] = 0;
+  __syncthreads();
+  uint32_t off = 0;
+  if (lane == 0 && n_pend) off = atomicAdd(&s_list[0], n_pend);
+  off = __builtin_amdgcn_readfirstlane(off);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_list[0]) s_list[1] = atomicAdd(&P.lt[0], s_list[0]);
+  __syncthreads();
+  if ((uint32_t)lane < n_pend) P.lt[BLT_LIST + s_list[1] + off + (uint32_t)lane] = pend;
   if (threadIdx.x == 0 && s_steps) atomicAdd(&A.work[1], s_steps);
   for (int i = threadIdx.x; i < A.n_cfg; i += blockDim.x)
     if (s_stop[i])
@@ -680,6 +716,10 @@ static int batch_launch(ctraj_batch *b, int block, int chunk, int grid, int refi
   const void *kl = b->uniform_dt ? (const void *)k_batch_integ<true> : (const void *)k_batch_integ<false>;
   A.Hs = b->dt;
   if ((rc = lds_limit(c, kl, lds_lens)) != CTRAJ_OK) return rc;
+  // untuned: the registers allow six wavefronts per SIMD, two workgroups of 768 threads per CU, or one of
+  // 1024 (four per SIMD) where the LDS holds one workgroup's tables only.  The 256-configuration scan at
+  // refill 8: 11.5 ms with 768, 11.7 with 1024
+  if (!block) block = 2 * lds_lens <= (size_t)c->lds_max ? 768 : 1024;
   if ((rc = block_ok(c, kl, block)) != CTRAJ_OK) return rc;
   if (grid <= 0) grid = grid_for(c, kl, block, lds_lens, (int64_t)1 << 40, 0);
   // phase 3: LDS = histogram
@@ -868,12 +908,14 @@ int32_t ctraj_batch_run(ctraj_batch *b, const ctraj_batch_tune *tune, int64_t *t
   ctraj_ctx *c = b->ctx;
   HIPCHK(c, hipSetDevice(c->device));
   const bool fused = (tune && tune->fused) || !b->d_pipe;
-  const int block = tune && tune->block ? tune->block : (fused ? 256 : 1024);
+  const int block = tune && tune->block ? tune->block : (fused ? 256 : 0);  // 0: batch_launch's choice
   const int chunk = tune && tune->chunk ? tune->chunk : 128;
   const int grid = tune ? tune->grid : 0;
-  const int refill = tune && tune->refill ? tune->refill : 16;  // the tuner's usual pick on either path
+  // untuned: the split lens kernel's refill sections are cheap (256 configurations at 4, 8, 12, 16, 20 idle
+  // lanes: 11.6, 11.5, 11.7, 11.9, 12.1 ms), the single kernel's hold the draws and walks
+  const int refill = tune && tune->refill ? tune->refill : (fused ? 16 : 8);
   const bool use_graph = tune && tune->use_graph;
-  if (block % 64 || block < 64 || block > (fused ? 256 : 1024))
+  if (block && (block % 64 || block < 64 || block > (fused ? 256 : 1024)))
     return fail(c, CTRAJ_EINVAL, fused ? "block must be 64, 128, 192 or 256" : "block must be a multiple of 64 up to 1024");
   if (chunk < 1 || chunk > (1 << 20)) return fail(c, CTRAJ_EINVAL, "chunk must be 1..2^20");
   if (refill < 1 || refill > 64) return fail(c, CTRAJ_EINVAL, "refill must be 1..64");
