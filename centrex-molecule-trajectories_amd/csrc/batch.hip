@@ -56,6 +56,7 @@ struct BArgs {
   double g;
   int n_cfg, n_labels, label_detected, cap, chunk, refill_min;
   int tame;                     // every face and g are of moderate size (walk_tame_elems)
+  ClampBound cb;                // the smallest bound of every configuration's lens (split path's lens kernel, UH)
   double Hs;                    // the lens dt shared by every configuration (split path's lens kernel, UH)
   int off_begin, off_hist;      // in doubles from the LDS base (off_begin: the lens constants in the lens kernel)
 };
@@ -407,6 +408,7 @@ k_batch_integ(BArgs A, BPipe P, KTab KT) {
   // z and t stay at their entry values while the molecule steps: a stopped one is only counted, and
   // one that leaves takes z1 and t_in + n dt + hp (the walker's definition)
   double r2 = 0.0, ks = 0.0, cu = 0.0, gk = 0.0, R2 = 0.0, Hs = A.Hs;
+  bool in_table = true;  // UH: the molecule's full steps need no clamp (ClampBound)
   HexK hk{};  // UH: the folded step's constants of the molecule's lens
   int rem = BREM_EMPTY, nfull = 0, c = 0;
   uint32_t it = 0, ends_at = 0;  // the wavefront's steps so far, and where this molecule's full steps end
@@ -503,6 +505,7 @@ k_batch_integ(BArgs A, BPipe P, KTab KT) {
           r2 = __builtin_fma(m.x, m.x, m.y * m.y);
           rem = nfull > 0 ? 1 : 0;
           ends_at = it + (uint32_t)nfull;
+          if constexpr (UH) in_table = within_table(A.cb, R2, r2, m.vx, m.vy, nfull);
         }
       }
       next += avail < (int64_t)__popcll(need) ? avail : (int64_t)__popcll(need);
@@ -513,26 +516,31 @@ k_batch_integ(BArgs A, BPipe P, KTab KT) {
     uint32_t cnt = (uint32_t)__popcll(am);
     // idle lanes wait for a refill only while there is something to claim
     const uint32_t keep = __builtin_amdgcn_readfirstlane(exhausted ? 0 : 64 - A.refill_min);
-    do {
-      steps_w += cnt;
-      ++it;
-      if (lane_in(am)) {
-        if constexpr (UH) {
-          rk4_step_hex_k(wsb, T.umax, cu, gk, hk, m.x, m.y, m.vx, m.vy, r2);
-        } else {
-          const Force<CTRAJ_FORCE_WSPLINE_HEX> F{ks, cu, g, gk};
-          lens_step<CTRAJ_FORCE_WSPLINE_HEX>(F, T, wsb, Hs, m.x, m.y, m.vx, m.vy, r2, status);
+    const auto steps = [&](auto clamp) {
+      do {
+        steps_w += cnt;
+        ++it;
+        if (lane_in(am)) {
+          if constexpr (UH) {
+            rk4_step_hex_k<decltype(clamp)::value>(wsb, T.umax, cu, gk, hk, m.x, m.y, m.vx, m.vy, r2);
+          } else {
+            const Force<CTRAJ_FORCE_WSPLINE_HEX> F{ks, cu, g, gk};
+            lens_step<CTRAJ_FORCE_WSPLINE_HEX>(F, T, wsb, Hs, m.x, m.y, m.vx, m.vy, r2, status);
+          }
+          r2 = __builtin_fma(m.x, m.x, m.y * m.y);
         }
-        r2 = __builtin_fma(m.x, m.x, m.y * m.y);
-      }
-      const bool out = r2 > R2;  // beyond the bore (lanes outside am: whatever)
-      const uint64_t over = am & (__builtin_amdgcn_ballot_w64(out) | __builtin_amdgcn_ballot_w64(ends_at == it));
-      if (over) {
-        if (lane_in(over)) rem = out ? BREM_STOPPED : 0;
-        am &= ~over;
-        cnt = (uint32_t)__popcll(am);
-      }
-    } while (cnt > keep);
+        const bool out = r2 > R2;  // beyond the bore (lanes outside am: whatever)
+        const uint64_t over = am & (__builtin_amdgcn_ballot_w64(out) | __builtin_amdgcn_ballot_w64(ends_at == it));
+        if (over) {
+          if (lane_in(over)) rem = out ? BREM_STOPPED : 0;
+          am &= ~over;
+          cnt = (uint32_t)__popcll(am);
+        }
+      } while (cnt > keep);
+    };
+    // nearly every wavefront's: no molecule of it can leave the table
+    if (UH && !(am & __builtin_amdgcn_ballot_w64(!in_table))) steps(std::false_type{});
+    else steps(std::true_type{});
   }
 
   if (lane == 0 && steps_w) atomicAdd(&s_steps, (unsigned long long)steps_w);
@@ -645,6 +653,7 @@ struct ctraj_batch {
   int64_t region = 0;
   bool uniform_dt = false;  // every lens has the same dt and folds its force scale (hex_folds)
   double dt = 0.0;
+  ClampBound cb{-1.0, 0.0};  // uniform_dt: the smallest of the lenses' bounds
   int64_t slice = 0;        // molecules per slice of the split path
   bool tame = false;        // walk_tame_elems over every configuration
   bool circ_only = false;   // only circular apertures (and lenses) in every configuration
@@ -715,6 +724,7 @@ static int batch_launch(ctraj_batch *b, int block, int chunk, int grid, int refi
   const size_t lds_lens = (tab + cfg_dbl) * sizeof(double) + (size_t)(b->n_cfg + 2) * sizeof(uint32_t);
   const void *kl = b->uniform_dt ? (const void *)k_batch_integ<true> : (const void *)k_batch_integ<false>;
   A.Hs = b->dt;
+  A.cb = b->cb;
   if ((rc = lds_limit(c, kl, lds_lens)) != CTRAJ_OK) return rc;
   // untuned: the registers allow six wavefronts per SIMD, two workgroups of 768 threads per CU, or one of
   // 1024 (four per SIMD) where the LDS holds one workgroup's tables only.  The 256-configuration scan at
@@ -851,6 +861,8 @@ int32_t ctraj_batch_create(ctraj_ctx *c, const ctraj_elem *elems, int32_t n_elem
       K.gk = hex_folds(K.ks) ? -b->g / K.ks : 0.0;
       all_fold = all_fold && hex_folds(K.ks);
       K.label_inside = L.label_inside;
+      const ClampBound cb = clamp_bound(K.ks, K.cu, K.R2, K.Hs, b->g, c->ws_max, c->ws_nseg);
+      b->cb = have_dt ? ClampBound{std::min(b->cb.vlim, cb.vlim), std::max(b->cb.hamax, cb.hamax)} : cb;
       if (!have_dt) {
         b->dt = K.Hs;
         have_dt = true;

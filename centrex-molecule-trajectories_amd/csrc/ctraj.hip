@@ -100,10 +100,11 @@ struct StepK {
   double gk;
   HexK hk;  // the folded hexapole step's constants, hex_k(ks, h)
   HexK h1;  // the plain step's, hex_k(1, h)
+  ClampBound cb;  // the molecules whose full steps need no clamp to the table's end (hexapole)
 };
 
 __host__ __device__ inline StepK step_k(double h, double ks, double g) {
-  return StepK{hex_folds(ks) ? -g / ks : 0.0, hex_k(ks, h), hex_k(1.0, h)};
+  return StepK{hex_folds(ks) ? -g / ks : 0.0, hex_k(ks, h), hex_k(1.0, h), ClampBound{-1.0, 0.0}};
 }
 
 struct PipeArgs {
@@ -796,7 +797,8 @@ __global__ void __launch_bounds__(768) k_propagate_lanes(KBeam B, KTab KT, const
 // each region): their wavefronts are full, and so few that each has a SIMD to itself, where claiming the
 // regions put 16 wavefronts of one or two molecules on every CU (2.58 -> 0.83 ms).  Fewer than 64 entries a
 // chunk, so that every SIMD gets a wavefront, measured the same.
-// What bounds the kernel: VALU issue with many molecules (72 instructions a step at eight wavefronts per SIMD,
+// What bounds the kernel: VALU issue with many molecules (72 instructions a step, 68 without clamps, at eight
+// wavefronts per SIMD,
 // issuing on 95 % of the cycles), the latency of one molecule's steps with few.  The step loop's condition and
 // mask are scalar and its exit is the rare path: 10^4 molecules 188 -> 120 us (430 serial steps), 10^7
 // 2.82 -> 2.75 ms.
@@ -857,6 +859,8 @@ k_lens(KBeam B, KTab KT, PipeArgs P, int refill_min, StepK K, unsigned long long
   uint32_t status = 0, slot = 0;
   int64_t key = 0;
   WsRef wsb = ws_of(T, 0);
+  constexpr bool BOUND = FORCE == CTRAJ_FORCE_WSPLINE_HEX && INTEG == CTRAJ_INTEG_RK4;
+  bool in_table = true;  // the molecule's full steps need no clamp (ClampBound)
 
   for (;;) {
     for (;;) {
@@ -968,6 +972,7 @@ k_lens(KBeam B, KTab KT, PipeArgs P, int refill_min, StepK K, unsigned long long
           }
           rem = nfull > 0 ? 1 : 0;
           ends_at = it + (uint32_t)nfull;
+          if constexpr (BOUND) in_table = within_table(K.cb, R2, r2, m.vx, m.vy, nfull);
         }
       }
       next += min(avail, (uint32_t)__popcll(need));
@@ -978,30 +983,35 @@ k_lens(KBeam B, KTab KT, PipeArgs P, int refill_min, StepK K, unsigned long long
     uint32_t cnt = (uint32_t)__popcll(am);
     // idle lanes wait for a refill only while there is something to claim
     const uint32_t keep = __builtin_amdgcn_readfirstlane(exhausted ? 0 : 64 - refill_min);
-    do {
-      steps_w += cnt;
-      ++it;
-      bool out;  // beyond the bore (lanes outside am: whatever)
-      if constexpr (INTEG == CTRAJ_INTEG_RK4) {
-        if (lane_in(am)) {
-          if constexpr (FORCE == CTRAJ_FORCE_WSPLINE_HEX)  // the host launches only folding lenses here
-            rk4_step_hex_k(wsb, T.umax, F.cu, K.gk, K.hk, m.x, m.y, m.vx, m.vy, r2);
-          else
-            rk4_step_k<FORCE>(F, T, wsb, K.h1, m.x, m.y, m.vx, m.vy, r2, status);
-          r2 = __builtin_fma(m.x, m.x, m.y * m.y);
+    const auto steps = [&](auto clamp) {
+      do {
+        steps_w += cnt;
+        ++it;
+        bool out;  // beyond the bore (lanes outside am: whatever)
+        if constexpr (INTEG == CTRAJ_INTEG_RK4) {
+          if (lane_in(am)) {
+            if constexpr (FORCE == CTRAJ_FORCE_WSPLINE_HEX)  // the host launches only folding lenses here
+              rk4_step_hex_k<decltype(clamp)::value>(wsb, T.umax, F.cu, K.gk, K.hk, m.x, m.y, m.vx, m.vy, r2);
+            else
+              rk4_step_k<FORCE>(F, T, wsb, K.h1, m.x, m.y, m.vx, m.vy, r2, status);
+            r2 = __builtin_fma(m.x, m.x, m.y * m.y);
+          }
+          out = r2 > R2;
+        } else {
+          if (lane_in(am)) ref_step<FORCE>(F, T, wsb, h, m, status);  // the row stores a = l1
+          out = beyond_r2(m.x, m.y, R2);  // R2: the threshold of d/2 (lens_ref)
         }
-        out = r2 > R2;
-      } else {
-        if (lane_in(am)) ref_step<FORCE>(F, T, wsb, h, m, status);  // the row stores a = l1
-        out = beyond_r2(m.x, m.y, R2);  // R2: the threshold of d/2 (lens_ref)
-      }
-      const uint64_t over = am & (__builtin_amdgcn_ballot_w64(out) | __builtin_amdgcn_ballot_w64(ends_at == it));
-      if (over) {
-        if (lane_in(over)) rem = out ? REM_STOPPED - (int)(it - ends_at + (uint32_t)nfull) : 0;
-        am &= ~over;
-        cnt = (uint32_t)__popcll(am);
-      }
-    } while (cnt > keep);
+        const uint64_t over = am & (__builtin_amdgcn_ballot_w64(out) | __builtin_amdgcn_ballot_w64(ends_at == it));
+        if (over) {
+          if (lane_in(over)) rem = out ? REM_STOPPED - (int)(it - ends_at + (uint32_t)nfull) : 0;
+          am &= ~over;
+          cnt = (uint32_t)__popcll(am);
+        }
+      } while (cnt > keep);
+    };
+    // nearly every wavefront's: no molecule of it can leave the table
+    if (BOUND && !(am & __builtin_amdgcn_ballot_w64(!in_table))) steps(std::false_type{});
+    else steps(std::true_type{});
   }
 
   if (work || (LT && P.lt)) {  // kernel arguments: every thread takes the same branch
@@ -1695,7 +1705,11 @@ static int32_t propagate_impl(ctraj_ctx *c, const ctraj_run *R, char *sdev) {
     const int blk_lens = few && !R->block ? 256 : block;
     int grid = grid_for(c, (const void *)kl, blk_lens, lds, (int64_t)1 << 40, 0);
     if (few && !R->block) grid = std::min(grid, std::max(1, std::min(c->n_cu, P.n_pre_waves)));
-    const StepK K = step_k(c->h_elems[lens_e].p[2], c->h_elems[lens_e].p[4], c->phys.g);
+    StepK K = step_k(c->h_elems[lens_e].p[2], c->h_elems[lens_e].p[4], c->phys.g);
+    if (c->force == CTRAJ_FORCE_WSPLINE_HEX && c->integ == CTRAJ_INTEG_RK4) {
+      const ctraj_elem &L = c->h_elems[lens_e];
+      K.cb = clamp_bound(L.p[4], L.p[5], L.p[1], L.p[2], c->phys.g, c->ws_max, c->ws_nseg);
+    }
     const bool one_slice = slice >= R->n;
     for (int64_t s0 = 0; s0 < R->n; s0 += slice) {
       const int64_t len = std::min(slice, R->n - s0);
@@ -2095,6 +2109,9 @@ int32_t ctraj_set_wspline(ctraj_ctx *c, int32_t n_states, int32_t n_seg, const d
     const double *last = coef + ((size_t)st * n_seg + n_seg - 1) * 4;
     c->ws_end[st] = (last[0] + last[1]) + last[2];
   }
+  c->ws_max = 0.0;  // a bound of |W'|: a segment's A s^2 + B s + C with 0 <= s < 1
+  for (size_t k = 0; k < cnt; k += 4)
+    c->ws_max = std::max(c->ws_max, std::fabs(coef[k]) + std::fabs(coef[k + 1]) + std::fabs(coef[k + 2]));
   return CTRAJ_OK;
 }
 

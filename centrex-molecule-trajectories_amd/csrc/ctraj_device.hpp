@@ -12,6 +12,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
+#include <type_traits>
+
 #include "../../include/ctraj.h"
 
 namespace ctraj {
@@ -175,8 +178,10 @@ __device__ __forceinline__ double clamp_to(double u, double umax) {
   return r;
 }
 
+// CLAMP false: the caller has shown u < umax (ClampBound), so the minimum would return u.
+template <bool CLAMP = true>
 __device__ __forceinline__ double wspline_eval(const WsRef &w, double umax, double u) {
-  u = clamp_to(u, umax);
+  if constexpr (CLAMP) u = clamp_to(u, umax);
   const unsigned k = (unsigned)(int)u;
   const double s = __builtin_amdgcn_fract(u);
   const dbl2_t ab = w.ab[k];
@@ -259,6 +264,32 @@ struct WalkCounters {
   uint32_t faces;
   uint32_t steps;
 };
+
+// When a hexapole lens's full steps cannot leave the W' table, so that the clamp of u = cu r^2 to its end
+// (4 of a step's 72 instructions) is the identity.  A stage lies within h |v| + h^2 amax / 2 of the step's
+// start, which lies in the bore (r^2 <= R2: the loop ends a molecule beyond it), and |v| grows by at most
+// h amax a step, where amax = |ks| max|W'| Rs + |g| bounds the acceleration inside the table's radius Rs
+// (cu Rs^2 = n segments).  So a molecule with r^2 <= R2 and |vx| + |vy| + n h amax <= vlim, vlim =
+// (Rs - R) / h - h amax / 2, stays in the table for its n steps.  A relative 10^-6 covers the rounding of
+// the bound and of the stages (the positions and velocities accumulate a few 10^-16 a step).  vlim < 0:
+// never (also for parameters that are not of moderate size).  Runs with and without, in turn: 10^4
+// molecules 146.4 -> 140.9 us, 10^7 3.18 -> 3.10 ms, a scan of 256 configurations 11.64 -> 11.41 ms.
+struct ClampBound {
+  double vlim, hamax;
+};
+
+__host__ inline ClampBound clamp_bound(double ks, double cu, double R2, double h, double g, double wmax, int nseg) {
+  const double Rs = std::sqrt((double)nseg / cu) * (1.0 - 1e-6), R = std::sqrt(R2) * (1.0 + 1e-6);
+  const double amax = (std::fabs(ks) * wmax * Rs + std::fabs(g)) * (1.0 + 1e-6);
+  const double vlim = ((Rs - R) / h - 0.5 * h * amax) * (1.0 - 1e-6);
+  const bool ok = cu > 0.0 && h > 1e-200 && R2 > 1e-200 && Rs < 1e100 && amax < 1e100 && vlim > 0.0 && vlim < 1e100;
+  return ok ? ClampBound{vlim, h * amax} : ClampBound{-1.0, 0.0};
+}
+
+// A NaN or infinite velocity, or a start beyond the bore, is not within the bound.
+__device__ __forceinline__ bool within_table(const ClampBound &b, double R2, double r2, double vx, double vy, int n) {
+  return r2 <= R2 && __builtin_fma((double)n, b.hamax, __builtin_fabs(vx) + __builtin_fabs(vy)) <= b.vlim;
+}
 
 // A hexapole lens with ks = -2 cE/m folds ks into its RK4 step constants (rk4_step_hex_k) when
 // |ks| lies in [2^-500, 2^500]: then -g/ks and ks times any step size the lens uses are finite
@@ -524,17 +555,19 @@ __device__ __forceinline__ void rk4_step(const Force<FORCE> &F, const Tables &T,
 // The hexapole step with the force scale folded into the step constants.  The acceleration is
 // a = ks W'(cu r^2) (x, y) - g y_hat = ks s with the slope s = W' (x, y) + (0, gk), gk = -g/ks, so
 // the step takes K = hex_k(ks, h): one multiplication fewer per slope than the plain step.
+template <bool CLAMP = true>
 __device__ __forceinline__ void slope_hex_k(const WsRef &wsb, double umax, double cu, double gk, double x, double y,
                                             double r2, double &sx, double &sy) {
-  const double w = wspline_eval(wsb, umax, r2 * cu);
+  const double w = wspline_eval<CLAMP>(wsb, umax, r2 * cu);
   sx = w * x;
   sy = __builtin_fma(w, y, gk);
 }
 
+template <bool CLAMP = true>
 __device__ __forceinline__ void rk4_step_hex_k(const WsRef &wsb, double umax, double cu, double gk, const HexK &K,
                                                double &x, double &y, double &vx, double &vy, double r2) {
   rk4_expanded(
-      K, [&](double px, double py, double pr2, double &sx, double &sy) { slope_hex_k(wsb, umax, cu, gk, px, py, pr2, sx, sy); },
+      K, [&](double px, double py, double pr2, double &sx, double &sy) { slope_hex_k<CLAMP>(wsb, umax, cu, gk, px, py, pr2, sx, sy); },
       x, y, vx, vy, r2);
 }
 

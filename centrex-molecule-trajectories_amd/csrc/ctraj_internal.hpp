@@ -44,6 +44,7 @@ struct ctraj_ctx {
   double *d_ws = nullptr;
   int ws_nseg = 0, ws_states = 0;
   double ws_end[CTRAJ_MAX_STATES] = {};  // W' at each state table's end (A + B + C of its last segment)
+  double ws_max = 0.0;                    // a bound of |W'| over every state's table
   // r tables, concatenated [knot][4]
   double *d_rt = nullptr;
   int rt_total = 0;
