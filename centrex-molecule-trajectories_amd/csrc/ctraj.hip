@@ -29,6 +29,7 @@
 #include "ctraj_internal.hpp"
 #include "ctraj_lanes.hpp"
 #include "ctraj_order.hpp"
+#include "ctraj_record.hpp"
 #include "ctraj_sinks.hpp"
 #include "ctraj_wave.hpp"
 
@@ -798,9 +799,8 @@ __global__ void __launch_bounds__(768) k_propagate_lanes(KBeam B, KTab KT, const
 // regions put 16 wavefronts of one or two molecules on every CU (2.58 -> 0.83 ms).  Fewer than 64 entries a
 // chunk, so that every SIMD gets a wavefront, measured the same.
 // What bounds the kernel: VALU issue with many molecules (72 instructions a step, 68 without clamps, at eight
-// wavefronts per SIMD,
-// issuing on 95 % of the cycles), the latency of one molecule's steps with few.  The step loop's condition and
-// mask are scalar and its exit is the rare path: 10^4 molecules 188 -> 120 us (430 serial steps), 10^7
+// wavefronts per SIMD, issuing on 95 % of the cycles), the latency of one molecule's steps with few.  The step
+// loop's condition and mask are scalar and its exit is the rare path: 10^4 molecules 188 -> 120 us (430 serial steps), 10^7
 // 2.82 -> 2.75 ms.
 // The per-molecule arithmetic is the one of walk().
 // ---------------------------------------------------------------------------------------------
@@ -1035,12 +1035,16 @@ k_lens(KBeam B, KTab KT, PipeArgs P, int refill_min, StepK K, unsigned long long
 // SIMD fit their registers, and one workgroup per CU is all that several lens-state tables leave
 // room for in LDS); 256 for the general ones, whose z-grid form needs more registers.
 template <int FORCE, int INTEG, int MODE, int KM>
-__global__ void __launch_bounds__(KM == KM_CIRC ? 512 : 256) k_record(KBeam B, KTab KT, ctraj_record RC) {
+__global__ void __launch_bounds__(KM == KM_CIRC ? 512 : 256) k_record(KBeam B, KTab KT, ctraj_record RC,
+                                                                              const uint32_t *slots) {
   extern __shared__ __attribute__((aligned(16))) double lds[];
+  if (slots && slots[0] == 0) return;  // a list that is nearly always empty
   const Tables T = stage_tables(lds, KT);
   __syncthreads();
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; s < RC.n; s += stride) {
+  const int64_t n_slots = slots ? (int64_t)slots[0] : RC.n;
+  for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n_slots; j += stride) {
+    const int64_t s = slots ? (int64_t)slots[1 + j] : j;
     const int64_t i = RC.index ? RC.index[s] : s;
     MState m;
     m.x = RC.in.x[i];
@@ -1408,7 +1412,7 @@ int ensure_buf(ctraj_ctx *ctx, ctraj_devbuf &b, size_t bytes) {
 using PropFn = void (*)(KBeam, KTab, ctraj_run, int, PipeArgs);
 using LensFn = void (*)(KBeam, KTab, PipeArgs, int, StepK, unsigned long long *);
 using LaneFn = void (*)(KBeam, KTab, const ctraj_run *, LaneArgs);
-using RecFn = void (*)(KBeam, KTab, ctraj_record);
+using RecFn = void (*)(KBeam, KTab, ctraj_record, const uint32_t *);
 
 // KM_CIRC when every element in [e0, e1) is a circular aperture, else KM_ALL
 static int kinds_mask(const std::vector<ctraj_elem> &el, int e0, int e1) {
@@ -2147,6 +2151,20 @@ int32_t ctraj_phase_times(ctraj_ctx *c, int32_t max, float *walk_ms, float *lens
   return CTRAJ_OK;
 }
 
+// Whether the rows and the samples of n molecules take kernels of their own (record.hip).  The walk of a slice
+// takes some 0.2 ms whatever the samples, the one-kernel form some 0.7 us per sample of a molecule while the
+// wavefronts are few, and the bytes at 2.2 TB/s once they are many (field-major 0.6).  One kernel -> two, us:
+//   molecule-major  1 x 64: 146 -> 162, 100 x 64: 320 -> 341, 1000 x 64: 231 -> 176, 16384 x 64: 345 -> 256,
+//     16384 x 2501: 1902 -> 747, 37000 x 64: 349 -> 380, 32768 x 251: 501 -> 444, 37000 x 2501: 2041 -> 1494,
+//     10^5 x 1001 (slices): 2037 -> 2232, 2 10^5 x 1501: 6752 -> 6170, x 2501: 10113 -> 7974
+//   field-major  100 x 64: 373 -> 362, 1000 x 64: 218 -> 178, 16384 x 2501: 2672 -> 965, 37000 x 128 (before the
+//     lens): 294 -> 430, 32768 x 251: 636 -> 453, 10^5 x 1001: 6290 -> 2902, 2 10^5 x 2501: 36438 -> 9270
+static bool zgrid_in_two(int64_t n, int cap, bool mol, int n_cu) {
+  if (n < 512 || n >= ((int64_t)1 << 31)) return false;
+  if (n <= (int64_t)64 * n_cu) return cap >= 64;
+  return cap >= (mol && n > ZGRID_SLICE_MOL ? 1500 : 256);
+}
+
 int32_t ctraj_record_trajectories(ctraj_ctx *c, const ctraj_record *RC) {
   if (!c || !RC) return fail(c, CTRAJ_EINVAL, "null argument");
   if (!c->have_beamline) return fail(c, CTRAJ_ESTATE, "no beamline set");
@@ -2174,8 +2192,24 @@ int32_t ctraj_record_trajectories(ctraj_ctx *c, const ctraj_record *RC) {
   HIPCHK(c, hipSetDevice(c->device));
   const int grid = grid_for(c, (const void *)k, block, lds, RC->n, 0);
   KBeam B = make_kbeam(c->d_elems, c->h_elems.data(), c->n_elems, c->phys);
-  hipLaunchKernelGGL(k, dim3(grid), dim3(block), lds, c->stream, B, kt, *RC);
-  HIPCHK(c, hipGetLastError());
+  // many samples of a one-lens beamline: rows first, then the samples (record.hip).  It takes a workspace, so
+  // not under capture; the molecules it leaves out, and all where it finds no memory, take the walk below
+  ZGridPlan plan;
+  int lens_e = -1, n_lens = 0;
+  for (int e = 0; e < c->n_elems; ++e)
+    if (c->h_elems[e].kind == CTRAJ_LENS) lens_e = e, ++n_lens;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (RC->mode != CTRAJ_REC_ROWS && n_lens == 1 && c->integ == CTRAJ_INTEG_RK4 && c->force != CTRAJ_FORCE_RTABLE &&
+      zgrid_in_two(RC->n, RC->cap, RC->mode == CTRAJ_REC_ZGRID_MOL, c->n_cu)) {
+    HIPCHK(c, hipStreamIsCapturing(c->stream, &cap));
+    if (cap == hipStreamCaptureStatusNone &&
+        (rc = record_zgrid(c, *RC, lens_e, km == KM_CIRC, B, kt, lds, plan)) != CTRAJ_OK)
+      return rc;
+  }
+  hipLaunchKernelGGL(k, dim3(grid), dim3(block), lds, c->stream, B, kt, *RC, plan.odd);
+  const hipError_t launched = hipGetLastError();
+  if (plan.ws && (rc = ctraj_scratch_free(c, plan.ws)) != CTRAJ_OK) return rc;  // reused in stream order
+  HIPCHK(c, launched);
   return CTRAJ_OK;
 }
 

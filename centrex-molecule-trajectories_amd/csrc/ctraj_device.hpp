@@ -179,8 +179,8 @@ __device__ __forceinline__ double clamp_to(double u, double umax) {
 }
 
 // CLAMP false: the caller has shown u < umax (ClampBound), so the minimum would return u.
-template <bool CLAMP = true>
-__device__ __forceinline__ double wspline_eval(const WsRef &w, double umax, double u) {
+template <bool CLAMP = true, class W = WsRef>
+__device__ __forceinline__ double wspline_eval(const W &w, double umax, double u) {
   if constexpr (CLAMP) u = clamp_to(u, umax);
   const unsigned k = (unsigned)(int)u;
   const double s = __builtin_amdgcn_fract(u);
@@ -191,7 +191,8 @@ __device__ __forceinline__ double wspline_eval(const WsRef &w, double umax, doub
 
 // Hexapole: |E| = cE r^2, a = -W'(|E|) 2 cE (x, y) / m - g y_hat.  r2 = x^2 + y^2 is passed in
 // so that the bore test of the previous step can share it.
-__device__ __forceinline__ void force_hex_r2(const WsRef &wsb, double umax, double ks, double cu, double g, double x,
+template <class W>
+__device__ __forceinline__ void force_hex_r2(const W &wsb, double umax, double ks, double cu, double g, double x,
                                              double y, double r2, double &ax, double &ay) {
   const double f = wspline_eval(wsb, umax, r2 * cu) * ks;
   ax = f * x;
@@ -200,7 +201,8 @@ __device__ __forceinline__ void force_hex_r2(const WsRef &wsb, double umax, doub
 
 // Linear-field model |E| = cE r (the reference's field assumption, electrostatic_lens.py:199-200):
 // a = -W'(|E|) cE (x, y) / (m r) - g y_hat, and (0, -g) on axis.
-__device__ __forceinline__ void force_lin(const WsRef &wsb, double umax, double ks, double cu, double g, double x,
+template <class W>
+__device__ __forceinline__ void force_lin(const W &wsb, double umax, double ks, double cu, double g, double x,
                                           double y, double &ax, double &ay) {
   const double r = rho_of(x, y);
   double fx = 0.0, fy = 0.0;
@@ -252,7 +254,7 @@ struct Force<CTRAJ_FORCE_WSPLINE_LIN> {
 // arrays (molecule.py:133-144, electrostatic_lens.py:106-111).  NullSink compiles to nothing.
 // ---------------------------------------------------------------------------------------------
 struct NullSink {
-  static constexpr bool kRows = false;
+  static constexpr bool kRows = false, kLensRows = false;
   __device__ __forceinline__ void row(const MState &) {}
 };
 
@@ -612,6 +614,9 @@ __device__ __forceinline__ bool lens_rk4(const ctraj_elem &E, const Tables &T, i
   const double L = E.p[3];
   const double dzs = m.vz * h;
   const int nfull = rk4_full_steps(L, m.vz, h, cap, status);
+  if constexpr (Sink::kLensRows) {
+    if (!sink.lens_begin(m, nfull, dzs)) return false;  // no room: the sink gives the molecule up
+  }
   double x = m.x, y = m.y, vx = m.vx, vy = m.vy;
   const double z_in = m.z, t_in = m.t;
   double z = z_in, t = t_in;
@@ -630,7 +635,9 @@ __device__ __forceinline__ bool lens_rk4(const ctraj_elem &E, const Tables &T, i
     }
     ++wc.steps;
     r2 = __builtin_fma(x, x, y * y);
-    if constexpr (Sink::kRows) {
+    if constexpr (Sink::kLensRows) {
+      sink.lens_row(i + 1, x, y, vx, vy);
+    } else if constexpr (Sink::kRows) {
       MState r = m;
       r.x = x; r.y = y; r.z = z; r.vx = vx; r.vy = vy; r.t = t;
       if (i < nfull || r2 > R2) {
@@ -649,6 +656,7 @@ __device__ __forceinline__ bool lens_rk4(const ctraj_elem &E, const Tables &T, i
   m.x = x; m.y = y; m.vx = vx; m.vy = vy; m.z = z; m.t = t;
   if (alive) {
     m.ax = 0.0; m.ay = -g; m.az = 0.0;
+    if constexpr (Sink::kLensRows) sink.lens_end(m);
   } else {
     uint32_t st = 0;
     F(T, wsb, x, y, m.ax, m.ay, st);

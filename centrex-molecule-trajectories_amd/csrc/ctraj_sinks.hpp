@@ -11,7 +11,7 @@ __device__ __forceinline__ double nan64() { return __builtin_nan(""); }
 // fields x, y, z, vx, vy, vz, ax, ay, az, t.  Rows past `cap` are counted but not stored; rows after
 // the molecule's last row are NaN.
 struct RowSink {
-  static constexpr bool kRows = true;
+  static constexpr bool kRows = true, kLensRows = false;
   double *buf;
   int64_t n, slot;
   int cap;
@@ -46,7 +46,7 @@ struct RowSink {
 // by the same lane's next samples however far the lanes of a wavefront drift apart in z.
 template <bool MOL>
 struct ZGridSinkT {
-  static constexpr bool kRows = true;
+  static constexpr bool kRows = true, kLensRows = false;
   double *buf;
   int64_t n, slot;
   int cap;
