@@ -23,7 +23,12 @@ struct ctraj_devbuf {
 // kernels still run).
 struct ctraj_pool {
   std::mutex mu;
-  std::multimap<size_t, void *> kept;
+  struct Kept {
+    void *p;
+    uint64_t at;  // when it was given back: the block unused longest leaves first
+  };
+  std::multimap<size_t, Kept> kept;
+  uint64_t now = 0;
   std::unordered_map<void *, size_t> out;
   size_t kept_bytes = 0;
 };

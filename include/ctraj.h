@@ -109,7 +109,7 @@ const char *ctraj_last_error(const ctraj_ctx *ctx);
 int32_t ctraj_device_info(ctraj_ctx *ctx, int32_t *n_cu, int32_t *lds_per_block, int32_t *wave, int32_t *arch);
 int32_t ctraj_dev_alloc(ctraj_ctx *ctx, uint64_t bytes, void **ptr);
 int32_t ctraj_dev_free(ctraj_ctx *ctx, void *ptr);
-/* device memory for work queued on the context's stream only: blocks given back are kept (at most 1 GiB of them) and
+/* device memory for work queued on the context's stream only: blocks given back are kept (1 GiB of them, the latest) and
  * handed out again without waiting for the device, so neither the host nor another stream may still use a block when
  * it is given back.  Kept blocks are released when an allocation of the context fails and when it is destroyed.
  * Safe to call from several threads. */

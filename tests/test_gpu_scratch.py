@@ -1,4 +1,5 @@
 """GPU: scratch blocks are exclusive while held, reused after they are given back, and bounded."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -64,3 +65,28 @@ def test_results_do_not_depend_on_reused_blocks():
         assert np.array_equal(r["label"], first[n]["label"]) and np.array_equal(r["tally"], first[n]["tally"])
         assert all(np.array_equal(r["out"][k], first[n]["out"][k]) for k in r["out"])
         assert np.array_equal(np.sort(r["aoi_index"]), np.sort(first[n]["aoi_index"]))
+
+
+@pytest.mark.parametrize("old", [1, 3, 4])
+def test_a_full_pool_keeps_the_blocks_in_use(old):
+    """Blocks of sizes no longer asked for make room: a block given back last is there for the next request,
+    however many older ones the pool (1 GiB) holds."""
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert N.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0  # of the runtime the library uses
+        return free.value
+
+    ctx = Context(0)
+    mib = (1 << 20) // 8
+    for b in [ctx.scratch(n * mib) for n in (240, 200, 220, 260)[:old]]:
+        b.free()
+    for _ in range(3):
+        big = ctx.scratch(640 * mib)
+        big.free()
+        free = free_bytes()
+        big = ctx.scratch(640 * mib)
+        assert free - free_bytes() < 64 << 20  # it was kept
+        big.free()
+    held = free_bytes()
+    ctx.close()
+    assert free_bytes() - held < (1 << 30) + (64 << 20)  # what the pool held is bounded
