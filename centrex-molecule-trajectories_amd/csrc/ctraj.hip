@@ -1361,6 +1361,10 @@ int grid_for(ctraj_ctx *ctx, const void *kern, int block, size_t lds, int64_t n,
 }
 
 constexpr size_t POOL_MAX = (size_t)1 << 30;  // bytes of scratch blocks kept per context
+// Bytes of result blocks kept per context.  A result allocated and released on every call costs 0.07 + 0.26 ms, and
+// where calls follow each other fast the driver falls behind with recycling the memory: runs of 194 173 streamed
+// molecules (216 MB of samples each) took 0.98 ms and 1.1 to 7.7 ms more in hipMalloc.
+constexpr size_t RESULTS_MAX = (size_t)8 << 30;
 
 // Release every kept block (the caller holds the pool's lock).
 static void pool_trim(ctraj_pool &P) {
@@ -1372,13 +1376,84 @@ static void pool_trim(ctraj_pool &P) {
 hipError_t dev_malloc(ctraj_ctx *ctx, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e == hipSuccess) return e;
-  {
-    std::lock_guard<std::mutex> lock(ctx->pool.mu);
-    if (ctx->pool.kept.empty()) return e;
-    pool_trim(ctx->pool);
+  bool any = false;
+  for (ctraj_pool *P : {&ctx->pool, &ctx->results}) {
+    std::lock_guard<std::mutex> lock(P->mu);
+    any = any || !P->kept.empty();
+    pool_trim(*P);
   }
+  if (!any) return e;
   (void)hipGetLastError();
   return hipMalloc(p, bytes);
+}
+
+// A kept block, or a new one.
+static int pool_take(ctraj_ctx *c, ctraj_pool &P, uint64_t bytes, void **ptr) try {
+  *ptr = nullptr;
+  // sizes in steps of an eighth of their power of two, so that runs of similar sizes share blocks
+  size_t step = 512;
+  while (step * 16 <= bytes) step *= 2;
+  const size_t size = std::max<size_t>(4096, (bytes + step - 1) / step * step);
+  if (size < bytes) return fail(c, CTRAJ_ENOMEM, "size out of range");
+  {
+    std::lock_guard<std::mutex> lock(P.mu);
+    auto it = P.kept.lower_bound(size);
+    if (it != P.kept.end() && it->first <= size + size / 4) {
+      *ptr = it->second.p;
+      P.out[it->second.p] = it->first;
+      P.kept_bytes -= it->first;
+      P.kept.erase(it);
+      return CTRAJ_OK;
+    }
+  }
+  HIPCHK(c, hipSetDevice(c->device));
+  const hipError_t e = dev_malloc(c, ptr, size);
+  if (e != hipSuccess) return fail(c, CTRAJ_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+  std::lock_guard<std::mutex> lock(P.mu);
+  P.out[*ptr] = size;
+  return CTRAJ_OK;
+} catch (const std::bad_alloc &) {
+  return fail(c, CTRAJ_ENOMEM, "host allocation failed");
+}
+
+// Keep a block, at most `most` bytes of them.
+static int pool_give(ctraj_ctx *c, ctraj_pool &P, void *ptr, size_t most) try {
+  if (!ptr) return CTRAJ_OK;
+  // Where the pool is full, the blocks unused longest make room.  (Releasing the block given back instead left the
+  // pool to sizes no longer asked for: every call then allocated and released its own, 0.3 ms.)
+  for (;;) {
+    void *release = nullptr;
+    bool last = false;
+    {
+      std::lock_guard<std::mutex> lock(P.mu);
+      auto &kept = P.kept;
+      auto it = P.out.find(ptr);
+      if (it == P.out.end()) return fail(c, CTRAJ_EINVAL, "not such a block of this context");
+      const size_t size = it->second;
+      if (P.kept_bytes + size <= most) {
+        kept.emplace(size, ctraj_pool::Kept{ptr, P.now++});
+        P.kept_bytes += size;
+        P.out.erase(it);
+        return CTRAJ_OK;
+      }
+      if (size > most) {
+        release = ptr;
+        last = true;
+        P.out.erase(it);
+      } else {  // kept is not empty: it is what leaves no room
+        auto old = kept.begin();
+        for (auto k = kept.begin(); k != kept.end(); ++k)
+          if (k->second.at < old->second.at) old = k;
+        release = old->second.p;
+        P.kept_bytes -= old->first;
+        kept.erase(old);
+      }
+    }
+    HIPCHK(c, hipFree(release));
+    if (last) return CTRAJ_OK;
+  }
+} catch (const std::bad_alloc &) {
+  return fail(c, CTRAJ_ENOMEM, "host allocation failed");
 }
 
 int ensure_buf(ctraj_ctx *ctx, ctraj_devbuf &b, size_t bytes) {
@@ -1871,9 +1946,9 @@ int32_t ctraj_ctx_destroy(ctraj_ctx *c) {
   if (!c) return CTRAJ_OK;
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
-  {
-    std::lock_guard<std::mutex> lock(c->pool.mu);
-    pool_trim(c->pool);
+  for (ctraj_pool *P : {&c->pool, &c->results}) {
+    std::lock_guard<std::mutex> lock(P->mu);
+    pool_trim(*P);
   }
   if (c->d_elems) (void)hipFree(c->d_elems);
   if (c->d_ws) (void)hipFree(c->d_ws);
@@ -1917,73 +1992,27 @@ int32_t ctraj_dev_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) {
   return CTRAJ_OK;
 }
 
-int32_t ctraj_scratch_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) try {
+int32_t ctraj_scratch_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) {
   if (!c || !ptr) return fail(c, CTRAJ_EINVAL, "null argument");
-  *ptr = nullptr;
-  // sizes in steps of an eighth of their power of two, so that runs of similar sizes share blocks
-  size_t step = 512;
-  while (step * 16 <= bytes) step *= 2;
-  const size_t size = std::max<size_t>(4096, (bytes + step - 1) / step * step);
-  if (size < bytes) return fail(c, CTRAJ_ENOMEM, "size out of range");
-  {
-    std::lock_guard<std::mutex> lock(c->pool.mu);
-    auto it = c->pool.kept.lower_bound(size);
-    if (it != c->pool.kept.end() && it->first <= size + size / 4) {
-      *ptr = it->second.p;
-      c->pool.out[it->second.p] = it->first;
-      c->pool.kept_bytes -= it->first;
-      c->pool.kept.erase(it);
-      return CTRAJ_OK;
-    }
-  }
-  HIPCHK(c, hipSetDevice(c->device));
-  const hipError_t e = dev_malloc(c, ptr, size);
-  if (e != hipSuccess) return fail(c, CTRAJ_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-  std::lock_guard<std::mutex> lock(c->pool.mu);
-  c->pool.out[*ptr] = size;
-  return CTRAJ_OK;
-} catch (const std::bad_alloc &) {
-  return fail(c, CTRAJ_ENOMEM, "host allocation failed");
+  return pool_take(c, c->pool, bytes, ptr);
 }
 
-int32_t ctraj_scratch_free(ctraj_ctx *c, void *ptr) try {
+int32_t ctraj_scratch_free(ctraj_ctx *c, void *ptr) {
+  if (!c) return fail(nullptr, CTRAJ_EINVAL, "ctx is NULL");
+  return pool_give(c, c->pool, ptr, POOL_MAX);
+}
+
+int32_t ctraj_result_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) {
+  if (!c || !ptr) return fail(c, CTRAJ_EINVAL, "null argument");
+  return pool_take(c, c->results, bytes, ptr);
+}
+
+int32_t ctraj_result_free(ctraj_ctx *c, void *ptr) {
   if (!c) return fail(nullptr, CTRAJ_EINVAL, "ctx is NULL");
   if (!ptr) return CTRAJ_OK;
-  // Where the pool is full, the blocks unused longest make room.  (Releasing the block given back instead left the
-  // pool to sizes no longer asked for: every call then allocated and released its own, 0.3 ms.)
-  for (;;) {
-    void *release = nullptr;
-    bool last = false;
-    {
-      std::lock_guard<std::mutex> lock(c->pool.mu);
-      auto &kept = c->pool.kept;
-      auto it = c->pool.out.find(ptr);
-      if (it == c->pool.out.end()) return fail(c, CTRAJ_EINVAL, "not a scratch block of this context");
-      const size_t size = it->second;
-      if (c->pool.kept_bytes + size <= POOL_MAX) {
-        kept.emplace(size, ctraj_pool::Kept{ptr, c->pool.now++});
-        c->pool.kept_bytes += size;
-        c->pool.out.erase(it);
-        return CTRAJ_OK;
-      }
-      if (size > POOL_MAX) {
-        release = ptr;
-        last = true;
-        c->pool.out.erase(it);
-      } else {  // kept is not empty: it is what leaves no room
-        auto old = kept.begin();
-        for (auto k = kept.begin(); k != kept.end(); ++k)
-          if (k->second.at < old->second.at) old = k;
-        release = old->second.p;
-        c->pool.kept_bytes -= old->first;
-        kept.erase(old);
-      }
-    }
-    HIPCHK(c, hipFree(release));
-    if (last) return CTRAJ_OK;
-  }
-} catch (const std::bad_alloc &) {
-  return fail(c, CTRAJ_ENOMEM, "host allocation failed");
+  HIPCHK(c, hipSetDevice(c->device));
+  HIPCHK(c, hipDeviceSynchronize());  // any stream may have used it; hipFree waits as well
+  return pool_give(c, c->results, ptr, RESULTS_MAX);
 }
 
 int32_t ctraj_dev_free(ctraj_ctx *c, void *ptr) {

@@ -74,7 +74,7 @@ struct ctraj_ctx {
   ctraj_devbuf pipe, pipe_cnt;
   // lens kernel claim order: per-entry lifetime buckets, per-workgroup bucket counts, slot permutation
   ctraj_devbuf ord;
-  ctraj_pool pool;
+  ctraj_pool pool, results;  // of ctraj_scratch_alloc and of ctraj_result_alloc
   // this device's scratch array of ctraj_propagate_noalloc (device address), or nullptr
   char *scratch = nullptr;
 };

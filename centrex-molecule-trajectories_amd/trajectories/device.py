@@ -81,6 +81,7 @@ class ScratchArray(DeviceArray):
     waiting for the device; hipMalloc and hipFree took 3 ms of a 7 ms run_simulation)."""
 
     __slots__ = ()
+    _pool = "scratch"
 
     def __init__(self, ctx: "Context", n: int, dtype=np.float64):
         self.ctx = ctx
@@ -88,13 +89,21 @@ class ScratchArray(DeviceArray):
         self.dtype = np.dtype(dtype)
         self.nbytes = self.n * self.dtype.itemsize
         p = C.c_void_p()
-        N.check("ctraj_scratch_alloc", N.lib().ctraj_scratch_alloc(ctx.handle, self.nbytes, C.byref(p)), ctx.handle)
+        name = f"ctraj_{self._pool}_alloc"
+        N.check(name, getattr(N.lib(), name)(ctx.handle, self.nbytes, C.byref(p)), ctx.handle)
         self.ptr = p.value
 
     def free(self):
         if self.ptr and self.ctx.handle:
-            N.lib().ctraj_scratch_free(self.ctx.handle, self.ptr)
+            getattr(N.lib(), f"ctraj_{self._pool}_free")(self.ctx.handle, self.ptr)
         self.ptr = None
+
+
+class ResultArray(ScratchArray):
+    """A DeviceArray for the caller, on any stream: given back, its block waits for the device and is kept."""
+
+    __slots__ = ()
+    _pool = "result"
 
 
 class Context:
@@ -130,6 +139,9 @@ class Context:
 
     def scratch(self, n, dtype=np.float64) -> ScratchArray:
         return ScratchArray(self, n, dtype)
+
+    def result(self, n, dtype=np.float64) -> ResultArray:
+        return ResultArray(self, n, dtype)
 
     def scratch_from(self, host, dtype=None) -> ScratchArray:
         """Queue the upload of a host array into a scratch buffer; the caller keeps ``host`` (an array that is

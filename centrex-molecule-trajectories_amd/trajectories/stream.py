@@ -130,7 +130,7 @@ class StreamedRun:
             init = [ctx.scratch(count) for _ in FIELDS6]
             init_state = ctx.scratch(count, np.uint8)
             if trajectories:
-                traj = ctx.alloc(6 * self.n_samples * count)  # the caller's
+                traj = ctx.result(6 * self.n_samples * count)  # the caller's
                 written = ctx.scratch(count, np.int32)
             t_alloc = time.perf_counter() - t0
             ctx.event_record(2)

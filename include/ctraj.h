@@ -115,6 +115,11 @@ int32_t ctraj_dev_free(ctraj_ctx *ctx, void *ptr);
  * Safe to call from several threads. */
 int32_t ctraj_scratch_alloc(ctraj_ctx *ctx, uint64_t bytes, void **ptr);
 int32_t ctraj_scratch_free(ctraj_ctx *ctx, void *ptr);
+/* device memory for a result that the caller holds as long as it likes and may use on any stream.  Giving it back
+ * waits for the device, as hipFree does, and keeps the block (8 GiB of them, the latest); kept blocks are released
+ * like those of ctraj_scratch_alloc.  Contents are undefined.  Safe to call from several threads. */
+int32_t ctraj_result_alloc(ctraj_ctx *ctx, uint64_t bytes, void **ptr);
+int32_t ctraj_result_free(ctraj_ctx *ctx, void *ptr);
 int32_t ctraj_host_alloc(ctraj_ctx *ctx, uint64_t bytes, void **ptr); /* pinned host memory */
 int32_t ctraj_host_free(ctraj_ctx *ctx, void *ptr);
 #define CTRAJ_H2D 1

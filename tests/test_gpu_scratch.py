@@ -9,6 +9,7 @@ from trajectories import _native as N
 from trajectories import configs
 from trajectories.device import Context
 from trajectories.engine import Engine
+from trajectories.stream import StreamedRun
 
 pytestmark = pytest.mark.gpu
 
@@ -90,3 +91,24 @@ def test_a_full_pool_keeps_the_blocks_in_use(old):
     held = free_bytes()
     ctx.close()
     assert free_bytes() - held < (1 << 30) + (64 << 20)  # what the pool held is bounded
+
+
+def test_results_outlive_their_run_and_are_kept():
+    """A result held by the caller is not handed out again, its dropped block is (also after use on another
+    stream: giving it back waits for the device), and blocks beyond what is kept are released."""
+    run = StreamedRun(configs.config4(), 60_000, chunk=1 << 20, seed=3, n_states=4)
+    a = run.run()
+    want = a.trajectories.to_host()
+    b = run.run()
+    assert b.trajectories.ptr != a.trajectories.ptr
+    assert np.array_equal(a.trajectories.to_host(), want, equal_nan=True)
+    p, ctx = a.trajectories.ptr, a.trajectories.ctx
+    del a
+    c = run.run()
+    assert c.trajectories.ptr == p
+    assert np.array_equal(c.trajectories.to_host(), want, equal_nan=True)
+    with pytest.raises(N.NativeError):  # of the other kind
+        N.check("ctraj_scratch_free", N.lib().ctraj_scratch_free(ctx.handle, p), ctx.handle)
+    big = ctx.result((9 << 30) // 8)
+    big.free()
+    ctx.result((9 << 30) // 8).free()
