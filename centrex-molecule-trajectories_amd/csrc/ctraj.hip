@@ -2207,10 +2207,14 @@ int32_t ctraj_phase_times(ctraj_ctx *c, int32_t max, float *walk_ms, float *lens
 //     10^5 x 1001 (slices): 2037 -> 2232, 2 10^5 x 1501: 6752 -> 6170, x 2501: 10113 -> 7974
 //   field-major  100 x 64: 373 -> 362, 1000 x 64: 218 -> 178, 16384 x 2501: 2672 -> 965, 37000 x 128 (before the
 //     lens): 294 -> 430, 32768 x 251: 636 -> 453, 10^5 x 1001: 6290 -> 2902, 2 10^5 x 2501: 36438 -> 9270
-static bool zgrid_in_two(int64_t n, int cap, bool mol, int n_cu) {
+//   four states (one workgroup's tables a CU, whose few write streams reach 3.2 TB/s molecule-major): 40960 x 2501
+//     1914 -> 1633, 10^5 x 2501 4403 -> 4046, 3 10^5 x 1501 7224 -> 9527, x 2501 11541 -> 12017; field-major
+//     3 10^5 x 1501 25591 -> 10151
+static bool zgrid_in_two(int64_t n, int cap, bool mol, bool few_streams, int n_cu) {
   if (n < 512 || n >= ((int64_t)1 << 31)) return false;
   if (n <= (int64_t)64 * n_cu) return cap >= 64;
-  return cap >= (mol && n > ZGRID_SLICE_MOL ? 1500 : 256);
+  if (mol && n > ZGRID_SLICE_MOL) return cap >= 1500 && !few_streams;
+  return cap >= 256;
 }
 
 int32_t ctraj_record_trajectories(ctraj_ctx *c, const ctraj_record *RC) {
@@ -2248,7 +2252,7 @@ int32_t ctraj_record_trajectories(ctraj_ctx *c, const ctraj_record *RC) {
     if (c->h_elems[e].kind == CTRAJ_LENS) lens_e = e, ++n_lens;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (RC->mode != CTRAJ_REC_ROWS && n_lens == 1 && c->integ == CTRAJ_INTEG_RK4 && c->force != CTRAJ_FORCE_RTABLE &&
-      zgrid_in_two(RC->n, RC->cap, RC->mode == CTRAJ_REC_ZGRID_MOL, c->n_cu)) {
+      zgrid_in_two(RC->n, RC->cap, RC->mode == CTRAJ_REC_ZGRID_MOL, 2 * lds > (size_t)c->lds_max, c->n_cu)) {
     HIPCHK(c, hipStreamIsCapturing(c->stream, &cap));
     if (cap == hipStreamCaptureStatusNone &&
         (rc = record_zgrid(c, *RC, lens_e, km == KM_CIRC, B, kt, lds, plan)) != CTRAJ_OK)
