@@ -1373,9 +1373,12 @@ static void pool_trim(ctraj_pool &P) {
   P.kept_bytes = 0;
 }
 
+// A failed allocation is the caller's to report: it must not stay the runtime's last error, which the next launch
+// would take for its own.
 hipError_t dev_malloc(ctraj_ctx *ctx, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e == hipSuccess) return e;
+  (void)hipGetLastError();
   bool any = false;
   for (ctraj_pool *P : {&ctx->pool, &ctx->results}) {
     std::lock_guard<std::mutex> lock(P->mu);
@@ -1383,8 +1386,9 @@ hipError_t dev_malloc(ctraj_ctx *ctx, void **p, size_t bytes) {
     pool_trim(*P);
   }
   if (!any) return e;
-  (void)hipGetLastError();
-  return hipMalloc(p, bytes);
+  e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
 }
 
 // A kept block, or a new one.
