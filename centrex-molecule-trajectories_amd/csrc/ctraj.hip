@@ -1391,15 +1391,18 @@ hipError_t dev_malloc(ctraj_ctx *ctx, void **p, size_t bytes) {
   return e;
 }
 
-// A kept block, or a new one.
-static int pool_take(ctraj_ctx *c, ctraj_pool &P, uint64_t bytes, void **ptr) try {
+// A kept block, or a new one; blocks larger than `most` are not kept.
+static int pool_take(ctraj_ctx *c, ctraj_pool &P, uint64_t bytes, size_t most, void **ptr) try {
   *ptr = nullptr;
-  // sizes in steps of an eighth of their power of two, so that runs of similar sizes share blocks
-  size_t step = 512;
-  while (step * 16 <= bytes) step *= 2;
-  const size_t size = std::max<size_t>(4096, (bytes + step - 1) / step * step);
-  if (size < bytes) return fail(c, CTRAJ_ENOMEM, "size out of range");
-  {
+  // sizes in steps of an eighth of their power of two, so that runs of similar sizes share blocks; what is not
+  // kept takes no more than it asks for
+  size_t size = bytes;
+  if (bytes <= most) {
+    size_t step = 512;
+    while (step * 16 <= bytes) step *= 2;
+    size = std::max<size_t>(4096, (bytes + step - 1) / step * step);
+  }
+  if (size <= most) {
     std::lock_guard<std::mutex> lock(P.mu);
     auto it = P.kept.lower_bound(size);
     if (it != P.kept.end() && it->first <= size + size / 4) {
@@ -1411,7 +1414,11 @@ static int pool_take(ctraj_ctx *c, ctraj_pool &P, uint64_t bytes, void **ptr) tr
     }
   }
   HIPCHK(c, hipSetDevice(c->device));
-  const hipError_t e = dev_malloc(c, ptr, size);
+  hipError_t e = dev_malloc(c, ptr, size);
+  if (e != hipSuccess && size > bytes) {  // room for the request, not for the step
+    size = std::max<size_t>(bytes, 1);
+    e = dev_malloc(c, ptr, size);
+  }
   if (e != hipSuccess) return fail(c, CTRAJ_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
   std::lock_guard<std::mutex> lock(P.mu);
   P.out[*ptr] = size;
@@ -1998,7 +2005,7 @@ int32_t ctraj_dev_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) {
 
 int32_t ctraj_scratch_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) {
   if (!c || !ptr) return fail(c, CTRAJ_EINVAL, "null argument");
-  return pool_take(c, c->pool, bytes, ptr);
+  return pool_take(c, c->pool, bytes, POOL_MAX, ptr);
 }
 
 int32_t ctraj_scratch_free(ctraj_ctx *c, void *ptr) {
@@ -2008,7 +2015,7 @@ int32_t ctraj_scratch_free(ctraj_ctx *c, void *ptr) {
 
 int32_t ctraj_result_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) {
   if (!c || !ptr) return fail(c, CTRAJ_EINVAL, "null argument");
-  return pool_take(c, c->results, bytes, ptr);
+  return pool_take(c, c->results, bytes, RESULTS_MAX, ptr);
 }
 
 int32_t ctraj_result_free(ctraj_ctx *c, void *ptr) {

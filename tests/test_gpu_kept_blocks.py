@@ -1,0 +1,43 @@
+"""GPU: what the kept blocks of a context take from the device's memory, and when they give it back."""
+import ctypes as C
+
+import pytest
+
+from trajectories import _native as N
+from trajectories.device import Context
+
+pytestmark = pytest.mark.gpu
+
+GIB = 1 << 30
+
+
+def free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert N.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0  # of the runtime the library uses
+    return free.value
+
+
+@pytest.fixture
+def ctx():
+    c = Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("kind,nbytes", [("scratch", 3 * GIB // 2 + 80 * (1 << 20)), ("result", 35 * GIB // 2)])
+def test_a_block_that_is_not_kept_takes_what_it_asks_for(ctx, kind, nbytes):
+    before = free_bytes()
+    b = getattr(ctx, kind)(nbytes // 8)
+    assert before - free_bytes() <= nbytes + (4 << 20)  # the driver's own granularity
+    b.free()
+    assert free_bytes() >= before - (4 << 20)
+
+
+@pytest.mark.parametrize("nbytes", [1 << 50, 1 << 63, (1 << 64) - 8])
+def test_a_size_out_of_range_is_refused(ctx, nbytes):
+    p = C.c_void_p()
+    for kind in ("scratch", "result"):
+        assert getattr(N.lib(), f"ctraj_{kind}_alloc")(ctx.handle, nbytes, C.byref(p)) == N.ENOMEM
+        assert not p.value
+        with pytest.raises(N.NativeError):
+            getattr(ctx, kind)(-1)
