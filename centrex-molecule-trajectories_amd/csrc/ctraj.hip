@@ -1366,11 +1366,40 @@ constexpr size_t POOL_MAX = (size_t)1 << 30;  // bytes of scratch blocks kept pe
 // molecules (216 MB of samples each) took 0.98 ms and 1.1 to 7.7 ms more in hipMalloc.
 constexpr size_t RESULTS_MAX = (size_t)8 << 30;
 
-// Release every kept block (the caller holds the pool's lock).
-static void pool_trim(ctraj_pool &P) {
-  for (auto &kv : P.kept) (void)hipFree(kv.second.p);
-  P.kept.clear();
-  P.kept_bytes = 0;
+// Release every kept block (the caller holds the pool's lock); whether there was any.
+static bool pool_trim(ctraj_pool &P) {
+  bool any = false;
+  for (auto it = P.kept.begin(); it != P.kept.end();) {
+    if (hipFree(it->second.p) != hipSuccess) {  // not now (a stream is capturing): it stays
+      (void)hipGetLastError();
+      ++it;
+      continue;
+    }
+    any = true;
+    P.kept_bytes -= it->first;
+    it = P.kept.erase(it);
+  }
+  return any;
+}
+
+static bool ctx_trim(ctraj_ctx *c) {
+  bool any = false;
+  for (ctraj_pool *P : {&c->pool, &c->results}) {
+    std::lock_guard<std::mutex> lock(P->mu);
+    any = pool_trim(*P) || any;
+  }
+  return any;
+}
+
+// The contexts that keep blocks: memory that one keeps is there for an allocation of any other on its device.
+struct CtxList {
+  std::mutex mu;
+  std::vector<ctraj_ctx *> all;
+};
+
+static CtxList &ctx_list() {
+  static CtxList &list = *new CtxList;  // contexts may outlive the library's static objects
+  return list;
 }
 
 // A failed allocation is the caller's to report: it must not stay the runtime's last error, which the next launch
@@ -1379,11 +1408,13 @@ hipError_t dev_malloc(ctraj_ctx *ctx, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e == hipSuccess) return e;
   (void)hipGetLastError();
+  if (e != hipErrorOutOfMemory) return e;
   bool any = false;
-  for (ctraj_pool *P : {&ctx->pool, &ctx->results}) {
-    std::lock_guard<std::mutex> lock(P->mu);
-    any = any || !P->kept.empty();
-    pool_trim(*P);
+  {
+    CtxList &L = ctx_list();
+    std::lock_guard<std::mutex> lock(L.mu);
+    for (ctraj_ctx *c : L.all)
+      if (c->device == ctx->device) any = ctx_trim(c) || any;
   }
   if (!any) return e;
   e = hipMalloc(p, bytes);
@@ -1949,6 +1980,14 @@ int32_t ctraj_ctx_create(int32_t device, ctraj_ctx **out) {
     c->scratch = nullptr;
     (void)hipGetLastError();
   }
+  try {
+    CtxList &L = ctx_list();
+    std::lock_guard<std::mutex> lock(L.mu);
+    L.all.push_back(c);
+  } catch (const std::bad_alloc &) {
+    (void)ctraj_ctx_destroy(c);
+    return fail(nullptr, CTRAJ_ENOMEM, "host allocation failed");
+  }
   *out = c;
   return CTRAJ_OK;
 }
@@ -1957,10 +1996,12 @@ int32_t ctraj_ctx_destroy(ctraj_ctx *c) {
   if (!c) return CTRAJ_OK;
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
-  for (ctraj_pool *P : {&c->pool, &c->results}) {
-    std::lock_guard<std::mutex> lock(P->mu);
-    pool_trim(*P);
+  {
+    CtxList &L = ctx_list();
+    std::lock_guard<std::mutex> lock(L.mu);
+    L.all.erase(std::remove(L.all.begin(), L.all.end(), c), L.all.end());
   }
+  (void)ctx_trim(c);
   if (c->d_elems) (void)hipFree(c->d_elems);
   if (c->d_ws) (void)hipFree(c->d_ws);
   if (c->d_rt) (void)hipFree(c->d_rt);
@@ -2000,6 +2041,12 @@ int32_t ctraj_dev_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) {
   *ptr = nullptr;
   hipError_t e = dev_malloc(c, ptr, bytes ? bytes : 1);
   if (e != hipSuccess) return fail(c, CTRAJ_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+  return CTRAJ_OK;
+}
+
+int32_t ctraj_trim(ctraj_ctx *c) {
+  if (!c) return fail(nullptr, CTRAJ_EINVAL, "ctx is NULL");
+  (void)ctx_trim(c);
   return CTRAJ_OK;
 }
 

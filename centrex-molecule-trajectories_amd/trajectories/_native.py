@@ -184,6 +184,7 @@ SIGNATURES = [
     ("ctraj_scratch_free", C.c_int32, [C.c_void_p, C.c_void_p]),
     ("ctraj_result_alloc", C.c_int32, [C.c_void_p, C.c_uint64, C.POINTER(C.c_void_p)]),
     ("ctraj_result_free", C.c_int32, [C.c_void_p, C.c_void_p]),
+    ("ctraj_trim", C.c_int32, [C.c_void_p]),
     ("ctraj_host_alloc", C.c_int32, [C.c_void_p, C.c_uint64, C.POINTER(C.c_void_p)]),
     ("ctraj_host_free", C.c_int32, [C.c_void_p, C.c_void_p]),
     ("ctraj_memcpy", C.c_int32, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_uint64, C.c_int32]),

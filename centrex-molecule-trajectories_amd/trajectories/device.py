@@ -143,6 +143,11 @@ class Context:
     def result(self, n, dtype=np.float64) -> ResultArray:
         return ResultArray(self, n, dtype)
 
+    def trim(self) -> None:
+        """Release the kept blocks of scratch and results (at most 1 and 8 GiB), for another allocator's use; the
+        library's own allocations on this device do so by themselves where memory runs out."""
+        N.check("ctraj_trim", N.lib().ctraj_trim(self.handle), self.handle)
+
     def scratch_from(self, host, dtype=None) -> ScratchArray:
         """Queue the upload of a host array into a scratch buffer; the caller keeps ``host`` (an array that is
         already contiguous and of this dtype) until it has synchronised."""

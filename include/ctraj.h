@@ -111,8 +111,8 @@ int32_t ctraj_dev_alloc(ctraj_ctx *ctx, uint64_t bytes, void **ptr);
 int32_t ctraj_dev_free(ctraj_ctx *ctx, void *ptr);
 /* device memory for work queued on the context's stream only: blocks given back are kept (1 GiB of them, the latest) and
  * handed out again without waiting for the device, so neither the host nor another stream may still use a block when
- * it is given back.  Kept blocks are released when an allocation of the context fails and when it is destroyed.
- * Safe to call from several threads. */
+ * it is given back.  Kept blocks are released by ctraj_trim, when an allocation of any context on the device fails
+ * and when their context is destroyed.  Safe to call from several threads. */
 int32_t ctraj_scratch_alloc(ctraj_ctx *ctx, uint64_t bytes, void **ptr);
 int32_t ctraj_scratch_free(ctraj_ctx *ctx, void *ptr);
 /* device memory for a result that the caller holds as long as it likes and may use on any stream.  Giving it back
@@ -120,6 +120,8 @@ int32_t ctraj_scratch_free(ctraj_ctx *ctx, void *ptr);
  * like those of ctraj_scratch_alloc.  Contents are undefined.  Safe to call from several threads. */
 int32_t ctraj_result_alloc(ctraj_ctx *ctx, uint64_t bytes, void **ptr);
 int32_t ctraj_result_free(ctraj_ctx *ctx, void *ptr);
+/* release the context's kept blocks (of both kinds), for another user of the device's memory */
+int32_t ctraj_trim(ctraj_ctx *ctx);
 int32_t ctraj_host_alloc(ctraj_ctx *ctx, uint64_t bytes, void **ptr); /* pinned host memory */
 int32_t ctraj_host_free(ctraj_ctx *ctx, void *ptr);
 #define CTRAJ_H2D 1

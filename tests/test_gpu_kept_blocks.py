@@ -41,3 +41,17 @@ def test_a_size_out_of_range_is_refused(ctx, nbytes):
         assert not p.value
         with pytest.raises(N.NativeError):
             getattr(ctx, kind)(-1)
+
+
+@pytest.mark.parametrize("kind", ["scratch", "result"])
+def test_kept_memory_is_there_for_others(ctx, kind):
+    """A call releases what a context keeps, and so does an allocation of another context that finds no room."""
+    nbytes, margin = 7 * GIB // 8, 8 << 20  # what else of the process comes and goes meanwhile
+    other = Context(0)
+    before = free_bytes()
+    for release in (ctx.trim, lambda: pytest.raises(N.NativeError, other.alloc, 1 << 47)):
+        getattr(ctx, kind)(nbytes // 8).free()
+        assert free_bytes() <= before - nbytes + margin  # kept
+        release()
+        assert free_bytes() >= before - margin
+    other.close()
