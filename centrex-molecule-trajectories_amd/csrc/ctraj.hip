@@ -1422,78 +1422,93 @@ hipError_t dev_malloc(ctraj_ctx *ctx, void **p, size_t bytes) {
   return e;
 }
 
-// A kept block, or a new one; blocks larger than `most` are not kept.
-static int pool_take(ctraj_ctx *c, ctraj_pool &P, uint64_t bytes, size_t most, void **ptr) try {
-  *ptr = nullptr;
-  // sizes in steps of an eighth of their power of two, so that runs of similar sizes share blocks; what is not
-  // kept takes no more than it asks for
-  size_t size = bytes;
-  if (bytes <= most) {
-    size_t step = 512;
-    while (step * 16 <= bytes) step *= 2;
-    size = std::max<size_t>(4096, (bytes + step - 1) / step * step);
-  }
-  if (size <= most) {
-    std::lock_guard<std::mutex> lock(P.mu);
-    auto it = P.kept.lower_bound(size);
-    if (it != P.kept.end() && it->first <= size + size / 4) {
-      *ptr = it->second.p;
-      P.out[it->second.p] = it->first;
-      P.kept_bytes -= it->first;
-      P.kept.erase(it);
-      return CTRAJ_OK;
-    }
-  }
-  HIPCHK(c, hipSetDevice(c->device));
-  hipError_t e = dev_malloc(c, ptr, size);
-  if (e != hipSuccess && size > bytes) {  // room for the request, not for the step
-    size = std::max<size_t>(bytes, 1);
-    e = dev_malloc(c, ptr, size);
-  }
-  if (e != hipSuccess) return fail(c, CTRAJ_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-  std::lock_guard<std::mutex> lock(P.mu);
-  P.out[*ptr] = size;
-  return CTRAJ_OK;
-} catch (const std::bad_alloc &) {
-  return fail(c, CTRAJ_ENOMEM, "host allocation failed");
+// The smallest kept block for a request of this size that was given back before `before` (the caller holds the lock).
+static std::multimap<size_t, ctraj_pool::Kept>::iterator pool_find(ctraj_pool &P, size_t size, uint64_t before) {
+  auto it = P.kept.lower_bound(size);
+  while (it != P.kept.end() && it->first <= size + size / 4 && it->second.at >= before) ++it;
+  return it != P.kept.end() && it->first <= size + size / 4 ? it : P.kept.end();
 }
 
-// Keep a block, at most `most` bytes of them.
-static int pool_give(ctraj_ctx *c, ctraj_pool &P, void *ptr, size_t most) try {
-  if (!ptr) return CTRAJ_OK;
-  // Where the pool is full, the blocks unused longest make room.  (Releasing the block given back instead left the
-  // pool to sizes no longer asked for: every call then allocated and released its own, 0.3 ms.)
-  for (;;) {
-    void *release = nullptr;
-    bool last = false;
-    {
-      std::lock_guard<std::mutex> lock(P.mu);
-      auto &kept = P.kept;
-      auto it = P.out.find(ptr);
-      if (it == P.out.end()) return fail(c, CTRAJ_EINVAL, "not such a block of this context");
-      const size_t size = it->second;
-      if (P.kept_bytes + size <= most) {
-        kept.emplace(size, ctraj_pool::Kept{ptr, P.now++});
-        P.kept_bytes += size;
-        P.out.erase(it);
+// A kept block, or a new one; blocks larger than `most` are not kept.  wait: any stream may still use a kept block,
+// so the device is waited for first; where it cannot be (a stream is capturing), the memory is new.
+static int pool_take(ctraj_ctx *c, ctraj_pool &P, uint64_t bytes, size_t most, bool wait, void **ptr) {
+  *ptr = nullptr;
+  void *p = nullptr;
+  try {
+    // sizes in steps of an eighth of their power of two, so that runs of similar sizes share blocks; what is not
+    // kept takes no more than it asks for
+    size_t size = bytes;
+    HIPCHK(c, hipSetDevice(c->device));
+    if (bytes <= most) {
+      size_t step = 512;
+      while (step * 16 <= bytes) step *= 2;
+      size = std::max<size_t>(4096, (bytes + step - 1) / step * step);
+      std::unique_lock<std::mutex> lock(P.mu);
+      const uint64_t before = P.now;
+      auto it = pool_find(P, size, before);
+      if (it != P.kept.end() && wait) {
+        lock.unlock();
+        const bool idle = hipDeviceSynchronize() == hipSuccess;
+        if (!idle) (void)hipGetLastError();
+        lock.lock();
+        it = idle ? pool_find(P, size, before) : P.kept.end();
+      }
+      if (it != P.kept.end()) {
+        P.out[it->second.p] = it->first;
+        *ptr = it->second.p;
+        P.kept_bytes -= it->first;
+        P.kept.erase(it);
         return CTRAJ_OK;
       }
-      if (size > most) {
-        release = ptr;
-        last = true;
-        P.out.erase(it);
-      } else {  // kept is not empty: it is what leaves no room
-        auto old = kept.begin();
-        for (auto k = kept.begin(); k != kept.end(); ++k)
-          if (k->second.at < old->second.at) old = k;
-        release = old->second.p;
-        P.kept_bytes -= old->first;
-        kept.erase(old);
-      }
     }
-    HIPCHK(c, hipFree(release));
-    if (last) return CTRAJ_OK;
+    hipError_t e = dev_malloc(c, &p, size);
+    if (e != hipSuccess && size > bytes) {  // room for the request, not for the step
+      size = std::max<size_t>(bytes, 1);
+      e = dev_malloc(c, &p, size);
+    }
+    if (e != hipSuccess) return fail(c, CTRAJ_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    std::lock_guard<std::mutex> lock(P.mu);
+    P.out[p] = size;
+    *ptr = p;
+    return CTRAJ_OK;
+  } catch (const std::bad_alloc &) {
+    if (p) (void)hipFree(p);
+    return fail(c, CTRAJ_ENOMEM, "host allocation failed");
   }
+}
+
+// Keep a block, at most `most` bytes of them: the blocks unused longest make room, and one larger than `most` leaves
+// at once.  (Releasing the block given back instead left the pool to sizes no longer asked for: every call then
+// allocated and released its own, 0.3 ms.)  It may be called from whatever thread collects the holder: it touches
+// neither that thread's current device nor a stream, and a block that cannot be released now stays.
+static int pool_give(ctraj_ctx *c, ctraj_pool &P, void *ptr, size_t most) try {
+  if (!ptr) return CTRAJ_OK;
+  std::unique_lock<std::mutex> lock(P.mu);
+  const auto own = P.out.find(ptr);
+  if (own == P.out.end()) return fail(c, CTRAJ_EINVAL, "not such a block of this context");
+  const size_t size = own->second;
+  P.kept.emplace(size, ctraj_pool::Kept{ptr, P.now++});
+  P.kept_bytes += size;
+  P.out.erase(own);
+  while (P.kept_bytes > most) {
+    auto leave = P.kept.end();
+    for (auto k = P.kept.begin(); k != P.kept.end(); ++k)
+      if (size > most ? k->second.p == ptr : leave == P.kept.end() || k->second.at < leave->second.at) leave = k;
+    if (leave == P.kept.end()) break;
+    const auto node = P.kept.extract(leave);
+    P.kept_bytes -= node.key();
+    lock.unlock();
+    const bool released = hipFree(node.mapped().p) == hipSuccess;
+    if (!released) (void)hipGetLastError();
+    lock.lock();
+    if (!released) {
+      P.kept.emplace(node.key(), node.mapped());
+      P.kept_bytes += node.key();
+      break;
+    }
+    if (size > most) break;
+  }
+  return CTRAJ_OK;
 } catch (const std::bad_alloc &) {
   return fail(c, CTRAJ_ENOMEM, "host allocation failed");
 }
@@ -2052,7 +2067,7 @@ int32_t ctraj_trim(ctraj_ctx *c) {
 
 int32_t ctraj_scratch_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) {
   if (!c || !ptr) return fail(c, CTRAJ_EINVAL, "null argument");
-  return pool_take(c, c->pool, bytes, POOL_MAX, ptr);
+  return pool_take(c, c->pool, bytes, POOL_MAX, false, ptr);
 }
 
 int32_t ctraj_scratch_free(ctraj_ctx *c, void *ptr) {
@@ -2062,14 +2077,11 @@ int32_t ctraj_scratch_free(ctraj_ctx *c, void *ptr) {
 
 int32_t ctraj_result_alloc(ctraj_ctx *c, uint64_t bytes, void **ptr) {
   if (!c || !ptr) return fail(c, CTRAJ_EINVAL, "null argument");
-  return pool_take(c, c->results, bytes, RESULTS_MAX, ptr);
+  return pool_take(c, c->results, bytes, RESULTS_MAX, true, ptr);
 }
 
 int32_t ctraj_result_free(ctraj_ctx *c, void *ptr) {
   if (!c) return fail(nullptr, CTRAJ_EINVAL, "ctx is NULL");
-  if (!ptr) return CTRAJ_OK;
-  HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipDeviceSynchronize());  // any stream may have used it; hipFree waits as well
   return pool_give(c, c->results, ptr, RESULTS_MAX);
 }
 

@@ -18,9 +18,9 @@ struct ctraj_devbuf {
   size_t bytes = 0;
 };
 
-// Blocks of ctraj_scratch_alloc: those handed out, and those given back and kept for the next request (all
-// work on them is queued on the context's one stream, so a block may be handed out while the last holder's
-// kernels still run).
+// Blocks of ctraj_scratch_alloc (all work on them is queued on the context's one stream, so a block may be handed
+// out while the last holder's kernels still run) or of ctraj_result_alloc (any stream's): those handed out, and
+// those given back and kept for the next request.
 struct ctraj_pool {
   std::mutex mu;
   struct Kept {

@@ -100,7 +100,8 @@ class ScratchArray(DeviceArray):
 
 
 class ResultArray(ScratchArray):
-    """A DeviceArray for the caller, on any stream: given back, its block waits for the device and is kept."""
+    """A DeviceArray for the caller, on any stream: given back, its block is kept, and handed out again only after the
+    device has been waited for."""
 
     __slots__ = ()
     _pool = "result"

@@ -115,9 +115,10 @@ int32_t ctraj_dev_free(ctraj_ctx *ctx, void *ptr);
  * and when their context is destroyed.  Safe to call from several threads. */
 int32_t ctraj_scratch_alloc(ctraj_ctx *ctx, uint64_t bytes, void **ptr);
 int32_t ctraj_scratch_free(ctraj_ctx *ctx, void *ptr);
-/* device memory for a result that the caller holds as long as it likes and may use on any stream.  Giving it back
- * waits for the device, as hipFree does, and keeps the block (8 GiB of them, the latest); kept blocks are released
- * like those of ctraj_scratch_alloc.  Contents are undefined.  Safe to call from several threads. */
+/* device memory for a result that the caller holds as long as it likes and may use on any stream.  Blocks given back
+ * are kept (8 GiB of them, the latest), and the device is waited for before one is handed out again; kept blocks are
+ * released like those of ctraj_scratch_alloc.  Contents are undefined.  Safe to call from several threads; giving a
+ * block back changes neither the calling thread's device nor waits for a stream, unless it is too large to be kept. */
 int32_t ctraj_result_alloc(ctraj_ctx *ctx, uint64_t bytes, void **ptr);
 int32_t ctraj_result_free(ctraj_ctx *ctx, void *ptr);
 /* release the context's kept blocks (of both kinds), for another user of the device's memory */

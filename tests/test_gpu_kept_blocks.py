@@ -55,3 +55,18 @@ def test_kept_memory_is_there_for_others(ctx, kind):
         release()
         assert free_bytes() >= before - margin
     other.close()
+
+
+def test_a_result_given_back_while_a_stream_is_captured(ctx):
+    """As a garbage collection may: the capture goes on, and the block is there for the next request."""
+    hip = N.lib()  # the runtime's own entry points, of the runtime the library uses
+    stream, graph = C.c_void_p(), C.c_void_p()
+    n = (64 << 20) // 8
+    a = ctx.result(n)
+    p = a.ptr
+    assert hip.hipStreamCreateWithFlags(C.byref(stream), 1) == 0
+    assert hip.hipStreamBeginCapture(stream, 0) == 0  # of any thread's calls
+    a.free()
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(stream) == 0
+    assert ctx.result(n).ptr == p
