@@ -290,7 +290,12 @@ def simulate_device(beamline: Beamline, xdist: Distribution, vdist: Distribution
     work = np.zeros(8, np.uint64)
     aoi_idx, aoi_lab, aoi_fin, inits = [], [], [], []
     n_oot = n_capped = 0
-    bufs = [ctx.scratch(max(1, min(chunk, n))) for _ in range(6)]
+    # kept blocks only for the library's own draws, which stay on the context's stream: a distribution that
+    # overrides draw_device may fill its buffers on any
+    bufs = []
+    for d in (xdist, vdist):
+        own = getattr(d.draw_device, "__func__", None) is Distribution.draw_device
+        bufs += [(ctx.scratch if own else ctx.alloc)(max(1, min(chunk, n))) for _ in range(3)]
     for s in range(0, n, chunk):
         m = min(chunk, n - s)
         src = [*xdist.draw_device(m, kx, offset=s, ctx=ctx, out=bufs[:3]),
