@@ -128,6 +128,7 @@ class Context:
         self.bound = None  # the CompiledBeamline currently set on the device
         self.lock = threading.RLock()
         self._pinned = None  # (address, uint8 view), made on first use
+        self._uploads, self._uploads_lock = [], threading.Lock()  # host arrays whose copies are queued
 
     # --- memory ---
     def alloc(self, n, dtype=np.float64) -> DeviceArray:
@@ -150,10 +151,15 @@ class Context:
         N.check("ctraj_trim", N.lib().ctraj_trim(self.handle), self.handle)
 
     def scratch_from(self, host, dtype=None) -> ScratchArray:
-        """Queue the upload of a host array into a scratch buffer; the caller keeps ``host`` (an array that is
-        already contiguous and of this dtype) until it has synchronised."""
-        host = np.asarray(host)
-        return ScratchArray(self, host.size, dtype or host.dtype).upload(host, sync=False)
+        """Queue the upload of a host array into a scratch buffer.  The context holds the array until it has waited
+        for the stream, whatever becomes of the caller (an error between this upload and the wait included)."""
+        host = np.ascontiguousarray(host, dtype=dtype)
+        d = ScratchArray(self, host.size, host.dtype)
+        try:
+            return d.upload(host, sync=False)
+        finally:
+            with self._uploads_lock:
+                self._uploads.append(host)
 
     def read(self, *pairs) -> None:
         """Fill host arrays from device memory, pairs of (buffer or address, contiguous array), with one wait: small
@@ -165,17 +171,19 @@ class Context:
                 self._pinned = (p.value, np.frombuffer((C.c_char * self.PINNED).from_address(p.value), np.uint8))
             base, view = self._pinned
             off, staged = 0, []
-            for src, out in pairs:
-                src, nbytes = N.addr(src), out.nbytes
-                if not nbytes:
-                    continue
-                if off + nbytes <= self.PINNED:
-                    self.memcpy(base + off, src, nbytes, N.D2H)
-                    staged.append((off, nbytes, out))
-                    off += (nbytes + 63) & ~63
-                else:
-                    self.memcpy(out.ctypes.data, src, nbytes, N.D2H)
-            self.sync()
+            try:
+                for src, out in pairs:
+                    src, nbytes = N.addr(src), out.nbytes
+                    if not nbytes:
+                        continue
+                    if off + nbytes <= self.PINNED:
+                        self.memcpy(base + off, src, nbytes, N.D2H)
+                        staged.append((off, nbytes, out))
+                        off += (nbytes + 63) & ~63
+                    else:
+                        self.memcpy(out.ctypes.data, src, nbytes, N.D2H)
+            finally:  # no copy into the caller's arrays is left queued
+                self.sync()
             for o, nbytes, out in staged:
                 out.reshape(-1).view(np.uint8)[:] = view[o:o + nbytes]
 
@@ -183,7 +191,14 @@ class Context:
         N.check("ctraj_memcpy", N.lib().ctraj_memcpy(self.handle, dst, src, int(nbytes), int(kind)), self.handle)
 
     def sync(self):
-        N.check("ctraj_sync", N.lib().ctraj_sync(self.handle), self.handle)
+        with self._uploads_lock:
+            uploads, self._uploads = self._uploads, []
+        try:
+            N.check("ctraj_sync", N.lib().ctraj_sync(self.handle), self.handle)
+        except BaseException:
+            with self._uploads_lock:
+                self._uploads += uploads
+            raise
 
     # --- timing on the context stream ---
     def event_record(self, slot: int):

@@ -110,12 +110,9 @@ class Engine:
     def _upload_inputs(self, x, y, z, vx, vy, vz, t, a0, state):
         ctx = self.ctx
         n = int(np.asarray(x).size)
-        host = []  # the uploads' sources, kept until the one wait below
 
-        def up(a, dtype):
-            a = np.ascontiguousarray(a, dtype=dtype).reshape(-1)
-            host.append(a)
-            return ctx.scratch_from(a)
+        def up(a, dtype):  # waited for once, below
+            return ctx.scratch_from(np.ascontiguousarray(a, dtype=dtype).reshape(-1))
 
         inp = {k: up(v, np.float64) for k, v in zip(FIELDS[:6], (x, y, z, vx, vy, vz))}
         if t is not None:
