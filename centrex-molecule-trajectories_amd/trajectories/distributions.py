@@ -155,12 +155,12 @@ def draw_chunks(xdist: Distribution, vdist: Distribution, n: int, chunks: int) -
     into calls: with Gaussian velocities and either position distribution, a chunk's normals are one call and
     its uniforms another, and the arithmetic is done once on all chunks, element for element the same."""
     total = n * chunks
-    if type(vdist) is CeNTREXVelocityDistribution and norm.random_state is uniform.random_state and n > 0:
+    if type(vdist) is CeNTREXVelocityDistribution and norm.random_state is uniform.random_state and min(n, chunks) > 0:
         vp = (vdist.vx, vdist.sigmax, vdist.vy, vdist.sigmay, vdist.vz, vdist.sigmaz)
-        if _plain(*vp) and min(vp[1::2]) > 0:
+        if _plain(*vp) and all(s > 0 for s in vp[1::2]):  # NaN is refused by the plain draws below
             rs = norm.random_state
             if type(xdist) is GaussianPositionDistribution and _plain(xdist.sigmax, xdist.sigmay, xdist.z) \
-                    and min(xdist.sigmax, xdist.sigmay) > 0:
+                    and xdist.sigmax > 0 and xdist.sigmay > 0:
                 g = rs.standard_normal(5 * total).reshape(chunks, 5, n)
                 X = np.stack([(g[:, 3] * xdist.sigmax + 0).reshape(-1), (g[:, 4] * xdist.sigmay + 0).reshape(-1),
                               np.full(total, xdist.z, dtype=np.float64)])

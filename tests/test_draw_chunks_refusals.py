@@ -1,0 +1,41 @@
+"""Chunked host draws refuse what the distributions' own draws refuse, and draw nothing for no chunks."""
+import numpy as np
+import pytest
+
+from trajectories.distributions import (CeNTREXPositionDistribution, CeNTREXVelocityDistribution,
+                                        GaussianPositionDistribution, draw_chunks)
+
+NAN = float("nan")
+X = [GaussianPositionDistribution(), CeNTREXPositionDistribution()]
+
+
+@pytest.mark.parametrize("bad", [NAN, -1.0])
+@pytest.mark.parametrize("which", ["sigmax", "sigmay", "sigmaz"])
+@pytest.mark.parametrize("xd", X, ids=["gaussian", "disc"])
+def test_widths_of_the_velocity(xd, which, bad):
+    vd = CeNTREXVelocityDistribution(**{which: bad})
+    with pytest.raises(ValueError):
+        vd.draw(5)
+    with pytest.raises(ValueError):
+        draw_chunks(xd, vd, 5, 3)
+
+
+@pytest.mark.parametrize("bad", [NAN, -1.0])
+@pytest.mark.parametrize("which", [0, 1])
+def test_widths_of_the_position(which, bad):
+    widths = [1e-3, 1e-3]
+    widths[which] = bad
+    xd = GaussianPositionDistribution(*widths)
+    with pytest.raises(ValueError):
+        xd.draw(5)
+    with pytest.raises(ValueError):
+        draw_chunks(xd, CeNTREXVelocityDistribution(), 5, 3)
+
+
+@pytest.mark.parametrize("xd", X, ids=["gaussian", "disc"])
+@pytest.mark.parametrize("chunks", [0, -1])
+def test_no_chunks(xd, chunks):
+    state = np.random.get_state()
+    A, B = draw_chunks(xd, CeNTREXVelocityDistribution(), 5, chunks)
+    assert A.shape == B.shape == (3, 0)
+    assert all(np.array_equal(a, b) for a, b in zip(state, np.random.get_state()))
