@@ -155,7 +155,9 @@ def draw_chunks(xdist: Distribution, vdist: Distribution, n: int, chunks: int) -
     into calls: with Gaussian velocities and either position distribution, a chunk's normals are one call and
     its uniforms another, and the arithmetic is done once on all chunks, element for element the same."""
     total = n * chunks
-    if type(vdist) is CeNTREXVelocityDistribution and norm.random_state is uniform.random_state and min(n, chunks) > 0:
+    replaced = any("draw" in getattr(d, "__dict__", ()) for d in (xdist, vdist))  # on the instance
+    if not replaced and min(n, chunks) > 0 and type(vdist) is CeNTREXVelocityDistribution \
+            and norm.random_state is uniform.random_state:
         vp = (vdist.vx, vdist.sigmax, vdist.vy, vdist.sigmay, vdist.vz, vdist.sigmaz)
         if _plain(*vp) and all(s > 0 for s in vp[1::2]):  # NaN is refused by the plain draws below
             rs = norm.random_state

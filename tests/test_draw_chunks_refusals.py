@@ -1,4 +1,5 @@
-"""Chunked host draws refuse what the distributions' own draws refuse, and draw nothing for no chunks."""
+"""Chunked host draws refuse what the distributions' own draws refuse, draw nothing for no chunks, and go through a
+draw method that an instance was given."""
 import numpy as np
 import pytest
 
@@ -39,3 +40,13 @@ def test_no_chunks(xd, chunks):
     A, B = draw_chunks(xd, CeNTREXVelocityDistribution(), 5, chunks)
     assert A.shape == B.shape == (3, 0)
     assert all(np.array_equal(a, b) for a, b in zip(state, np.random.get_state()))
+
+
+@pytest.mark.parametrize("xd", X, ids=["gaussian", "disc"])
+def test_a_draw_method_of_the_instance(xd):
+    vd = CeNTREXVelocityDistribution()
+    vd.draw = lambda n: np.full((3, n), 7.0)
+    assert np.array_equal(draw_chunks(xd, vd, 5, 3)[1], np.full((3, 15), 7.0))
+    own = type(xd)()
+    own.draw = lambda n: np.full((3, n), 8.0)
+    assert np.array_equal(draw_chunks(own, CeNTREXVelocityDistribution(), 5, 3)[0], np.full((3, 15), 8.0))
