@@ -643,12 +643,16 @@ int32_t ctraj_smooth_objective(ctraj_ctx *c, const ctraj_smooth *s) {
   kt.ws_states = nl > 0 ? 1 : 0;  // state 0 only
   kt.rt_total = 0;
   const size_t lds_tab = ktab_lds_bytes(kt);
-  // with gradients each wavefront keeps a recompute window in LDS beside the tables: 16 wavefronts fit with
-  // one state's 24 KB table, fewer with a longer one
+  // with gradients each wavefront keeps a recompute window in LDS beside the tables
   const size_t lds_wave = grad ? (size_t)kSub * 256 * sizeof(double) : 0;
   int block = block_req ? block_req : 256;
   if (grad && !block_req) {
-    block = 1024;
+    // 16 wavefronts fit beside one state's 24 KB table, fewer beside a longer one.  Where there are fewer work items
+    // than that for every CU, a workgroup has one CU's share of them: a wavefront's time is then its serial steps,
+    // which take twice as long where four share a SIMD and the other CUs are idle.  One set, K = 8, workgroups of 16
+    // wavefronts -> here, us: 1000 molecules 766 -> 452, 16 384 902 -> 499, 65 536 963 -> 550, 131 072 1036 -> 709
+    const int64_t items = (s->n + 63) / 64 * s->n_cfg;
+    block = 64 * (int)std::min<int64_t>(16, (items + c->n_cu - 1) / c->n_cu);
     while (block > 64 && lds_tab + (size_t)(block / 64) * lds_wave > (size_t)c->lds_max) block -= 64;
   }
   const size_t lds = lds_tab + (size_t)(block / 64) * lds_wave;

@@ -365,7 +365,7 @@ typedef struct ctraj_smooth {
   int32_t ckpt_every;                   /* K >= 1: at most K steps between checkpoints */
   int32_t max_steps;                    /* full RK4 steps per lens at most (>= 1); bounds the checkpoint store */
   int32_t block;                        /* threads per block, multiple of 64 up to 512 (0 = 256, or with gradients
-                                         * as many up to 1024 as the LDS of one CU holds) */
+                                         * by the molecules, as many up to 1024 as the LDS of one CU holds) */
   int32_t reserved;
 } ctraj_smooth;
 /* number of parameters of the current beamline (CIRC: 1, LENS: 2, plus mu) and, when theta is not NULL,
