@@ -606,6 +606,26 @@ static int smooth_layout(ctraj_ctx *c, int *np, int *n_faces, int *n_lens, doubl
   return CTRAJ_OK;
 }
 
+// Whether b holds `bytes`, or could be replaced by a buffer that does.  Where memory is short it stays as it is: a
+// caller that can do with less does not give up what it has, nor other contexts their kept blocks, call after call.
+static bool extra_buf(ctraj_ctx *c, ctraj_devbuf &b, size_t bytes) {
+  if (b.p && b.bytes >= bytes) return true;
+  size_t free_b = 0, total = 0;
+  void *p = nullptr;
+  if (hipMemGetInfo(&free_b, &total) != hipSuccess || free_b < bytes || hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (b.p && (hipStreamSynchronize(c->stream) != hipSuccess || hipFree(b.p) != hipSuccess)) {
+    (void)hipGetLastError();
+    (void)hipFree(p);
+    return false;
+  }
+  b.p = p;
+  b.bytes = bytes;
+  return true;
+}
+
 extern "C" {
 
 int32_t ctraj_smooth_params(ctraj_ctx *c, int32_t *n_params, double *theta) {
@@ -690,21 +710,21 @@ int32_t ctraj_smooth_objective(ctraj_ctx *c, const ctraj_smooth *s) {
     // store then grows with the steps of the lens (1.1 GB for 4096 wavefronts and 520 steps), so it is
     // taken while it stays within 2 GiB and can be had, and the caller's interval otherwise
     const int64_t dense_max = (int64_t)2 << 30, ws_max = (int64_t)4 << 30, grain = (int64_t)64 << 20;
-    layout(std::min(s->ckpt_every, kSub));
-    int64_t per_block = A.ws_stride * 8 * wpb;
-    bool have = false;
-    if (s->ckpt_every <= kSub || per_block * grid <= dense_max) {
-      grid = (int)std::min<int64_t>(grid, std::max<int64_t>(1, ws_max / per_block));
-      rc = ensure_buf(c, c->sm_ws, (size_t)((per_block * grid + grain - 1) / grain * grain));
-      if (rc != CTRAJ_OK && s->ckpt_every <= kSub) return rc;
-      have = rc == CTRAJ_OK;
+    const auto per_block = [&] { return A.ws_stride * 8 * wpb; };
+    // keep the checkpoint/recompute store within 4 GiB
+    const auto bound = [&] { grid = (int)std::min<int64_t>(grid, std::max<int64_t>(1, ws_max / per_block())); };
+    bool dense = false;
+    if (s->ckpt_every > kSub) {
+      layout(kSub);
+      dense = per_block() * grid <= dense_max &&
+              extra_buf(c, c->sm_ws, (size_t)((per_block() * grid + grain - 1) / grain * grain));
     }
-    if (!have) {
+    if (!dense) {
       layout(s->ckpt_every);
-      per_block = A.ws_stride * 8 * wpb;
-      // keep the checkpoint/recompute store within 4 GiB
-      grid = (int)std::min<int64_t>(grid, std::max<int64_t>(1, ws_max / per_block));
-      if ((rc = ensure_buf(c, c->sm_ws, (size_t)per_block * grid)) != CTRAJ_OK) return rc;
+      bound();
+      const int64_t most = per_block() * grid;
+      const int64_t bytes = s->ckpt_every > kSub ? most : (most + grain - 1) / grain * grain;
+      if ((rc = ensure_buf(c, c->sm_ws, (size_t)bytes)) != CTRAJ_OK) return rc;
     }
     A.ws = (double *)c->sm_ws.p;
   }
