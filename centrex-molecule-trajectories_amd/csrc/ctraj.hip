@@ -1039,6 +1039,7 @@ __global__ void __launch_bounds__(KM == KM_CIRC ? 512 : 256) k_record(KBeam B, K
                                                                               const uint32_t *slots) {
   extern __shared__ __attribute__((aligned(16))) double lds[];
   if (slots && slots[0] == 0) return;  // a list that is nearly always empty
+  if (slots && slots[0] == ZGRID_ALL) slots = nullptr;
   const Tables T = stage_tables(lds, KT);
   __syncthreads();
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -2269,22 +2270,43 @@ int32_t ctraj_phase_times(ctraj_ctx *c, int32_t max, float *walk_ms, float *lens
   return CTRAJ_OK;
 }
 
-// Whether the rows and the samples of n molecules take kernels of their own (record.hip).  The walk of a slice
-// takes some 0.2 ms whatever the samples, the one-kernel form some 0.7 us per sample of a molecule while the
-// wavefronts are few, and the bytes at 2.2 TB/s once they are many (field-major 0.6).  One kernel -> two, us:
-//   molecule-major  1 x 64: 146 -> 162, 100 x 64: 320 -> 341, 1000 x 64: 231 -> 176, 16384 x 64: 345 -> 256,
-//     16384 x 2501: 1902 -> 747, 37000 x 64: 349 -> 380, 32768 x 251: 501 -> 444, 37000 x 2501: 2041 -> 1494,
-//     10^5 x 1001 (slices): 2037 -> 2232, 2 10^5 x 1501: 6752 -> 6170, x 2501: 10113 -> 7974
-//   field-major  100 x 64: 373 -> 362, 1000 x 64: 218 -> 178, 16384 x 2501: 2672 -> 965, 37000 x 128 (before the
-//     lens): 294 -> 430, 32768 x 251: 636 -> 453, 10^5 x 1001: 6290 -> 2902, 2 10^5 x 2501: 36438 -> 9270
+// Whether the rows and the samples of n molecules take kernels of their own (record.hip), and for which lens steps S
+// of a molecule.  One kernel -> those, us, by size at S = 326 (a 0.6 m lens in steps of 10 us):
+//   molecule-major  1 x 64: 146 -> 162, 100 x 64: 320 -> 341, 600 x 64: 429 -> 210, 16384 x 64: 463 -> 302,
+//     16384 x 2501: 1903 -> 761, 37000 x 256: 577 -> 554, 37000 x 2501: 2116 -> 1435, 10^5 x 1001 (slices): 2037 ->
+//     2232, 2 10^5 x 1501: 6752 -> 6170, x 2501: 10113 -> 7974
+//   field-major  100 x 64: 373 -> 362, 600 x 64: 479 -> 223, 16384 x 2501: 2852 -> 983, 37000 x 2501: 8251 -> 2256,
+//     10^5 x 512: 2931 -> 2737, x 1001: 6290 -> 2902, 2 10^5 x 2501: 36438 -> 9270
 //   four states (one workgroup's tables a CU, whose few write streams reach 3.2 TB/s molecule-major): 40960 x 2501
-//     1914 -> 1633, 10^5 x 2501 4403 -> 4046, 3 10^5 x 1501 7224 -> 9527, x 2501 11541 -> 12017; field-major
-//     3 10^5 x 1501 25591 -> 10151
-static bool zgrid_in_two(int64_t n, int cap, bool mol, bool few_streams, int n_cu) {
+//     1914 -> 1633, 3 10^5 x 1501 7224 -> 9527, x 2501 11541 -> 12017; field-major 3 10^5 x 1501 25591 -> 10151, but
+//     x 512 7444 -> 7892
+// By the steps: in one slice the kernels of their own gain 0.7 us a step (their walk takes 0.6 us, the one-kernel
+// form's 1.3) and molecule-major 0.38 us a sample, and lose some 5 ns a molecule (k_zfaces takes a run's samples at a time,
+// most of them fewer than a wavefront has lanes): molecule-major 16384 x 64 at S = 3, 65, 326: 61 -> 120, 141 -> 160,
+// 463 -> 302; 40960 x 256: 219 -> 322, 281 -> 364, 580 -> 580; 40960 x 512: 449 -> 462, 503 -> 520, 771 -> 708;
+// field-major 16384 x 64 52 -> 67, 150 -> 114, 516 -> 266.  In several slices their walks follow each other:
+// field-major 10^5 x 256 at S = 65, 163, 326: 1172 -> 948, 1207 -> 1300, 1270 -> 1727.  And more rows than a slice has
+// room for leave everything to the one-kernel form (37000 x 2501 in steps of 5 us, two kernels for what fits and one for the rest: 2395 -> 3563).
+// The steps follow from vz, which only the device has: the host goes by 200 m/s, to spare a clear case the plan and
+// the launches that return at once (20 to 60 us), and the plan has the last word.
+static bool zgrid_in_two(const ctraj_elem &lens, int64_t n, int cap, bool mol, bool few_streams, int n_cu,
+                         ZGridSteps &rows) {
+  const int64_t slice = std::min(n, mol ? ZGRID_SLICE_MOL : ZGRID_SLICE_FIELD);
   if (n < 512 || n >= ((int64_t)1 << 31)) return false;
-  if (n <= (int64_t)64 * n_cu) return cap >= 64;
-  if (mol && n > ZGRID_SLICE_MOL) return cap >= 1500 && !few_streams;
-  return cap >= 256;
+  if (n <= (int64_t)64 * n_cu ? cap < 64 : cap < 256) return false;
+  if (mol) {
+    if (n > slice) {
+      if (cap < 1500 || few_streams) return false;
+    } else {
+      rows.lo = (8.5e-3 * (double)n + 30.0 - 0.38 * cap) / 0.7;
+    }
+  } else {
+    if (cap < 192) rows.lo = 33.0;
+    if (n > slice && cap < 768) rows.hi = cap < 384 || (few_streams && n > 4 * slice) ? 130.0 : 420.0;
+  }
+  const double steps = lens.p[3] / (lens.p[2] * 200.0), each = mol ? steps : 1.25 * steps;
+  return each >= 0.8 * rows.lo && each <= 1.25 * rows.hi && each <= 1.25 * ZGRID_ROWS_EACH &&
+         each * (double)slice <= 1.25 * ZGRID_ROWS;
 }
 
 int32_t ctraj_record_trajectories(ctraj_ctx *c, const ctraj_record *RC) {
@@ -2317,15 +2339,17 @@ int32_t ctraj_record_trajectories(ctraj_ctx *c, const ctraj_record *RC) {
   // many samples of a one-lens beamline: rows first, then the samples (record.hip).  It takes a workspace, so
   // not under capture; the molecules it leaves out, and all where it finds no memory, take the walk below
   ZGridPlan plan;
+  ZGridSteps steps;
   int lens_e = -1, n_lens = 0;
   for (int e = 0; e < c->n_elems; ++e)
     if (c->h_elems[e].kind == CTRAJ_LENS) lens_e = e, ++n_lens;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (RC->mode != CTRAJ_REC_ROWS && n_lens == 1 && c->integ == CTRAJ_INTEG_RK4 && c->force != CTRAJ_FORCE_RTABLE &&
-      zgrid_in_two(RC->n, RC->cap, RC->mode == CTRAJ_REC_ZGRID_MOL, 2 * lds > (size_t)c->lds_max, c->n_cu)) {
+      zgrid_in_two(c->h_elems[lens_e], RC->n, RC->cap, RC->mode == CTRAJ_REC_ZGRID_MOL, 2 * lds > (size_t)c->lds_max,
+                   c->n_cu, steps)) {
     HIPCHK(c, hipStreamIsCapturing(c->stream, &cap));
     if (cap == hipStreamCaptureStatusNone &&
-        (rc = record_zgrid(c, *RC, lens_e, km == KM_CIRC, B, kt, lds, plan)) != CTRAJ_OK)
+        (rc = record_zgrid(c, *RC, lens_e, km == KM_CIRC, B, kt, lds, steps, plan)) != CTRAJ_OK)
       return rc;
   }
   hipLaunchKernelGGL(k, dim3(grid), dim3(block), lds, c->stream, B, kt, *RC, plan.odd);

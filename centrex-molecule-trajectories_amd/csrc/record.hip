@@ -1,4 +1,4 @@
-// record.hip -- z-grid samples of many molecules (post_processing.py:20-140), in three kernels.
+// record.hip -- z-grid samples of many molecules (post_processing.py:20-140), in three kernels and a plan.
 //
 // A sample needs the rows of the molecule's trajectory next to its z and nothing of the other samples, so the
 // walk and the sampling are separate: k_zrows walks one molecule per lane and stores its rows, k_zfaces and k_zlens
@@ -8,6 +8,8 @@
 // 1.94 ms; here 0.24 + 0.87 + 0.45 (a fill of the same buffer takes 0.87).  Sampling in one kernel took 1.6 to 2.8 ms:
 // with the force tables in LDS, or the lens's rows and force in the same loop (150 registers a lane), too few
 // wavefronts are in flight for the loads, which wait behind the wavefront's own stores.
+// k_zplan decides on the device whether they are the form for these molecules; if not, they return at once and the
+// one-kernel form, which is launched last in any case, takes all of them.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -34,11 +36,17 @@ struct ZRows {
   double *face;              // [n / 64][n_face][10][64]; the last row at the number of face rows
   double2 *lens;             // [cap_rows][2]: molecule-major (a molecule's rows contiguous) or interleaved
   unsigned long long *used;  // lens rows given out
-  uint32_t *odd;             // [0] count, [1 ...] slots left to the one-kernel form
+  const uint32_t *go;        // 0: every slot is left to the one-kernel form (k_zplan)
+  uint32_t *odd;             // [0] count or ZGRID_ALL, [1 ...] slots left to the one-kernel form
   int n_face;
   int64_t cap_rows;
   int64_t s0, n;             // this slice's slots
 };
+
+// Whether a lens step of dz takes a molecule at z forward, at a step that its z resolves.
+__device__ __forceinline__ bool moves_on(double dz, double z) {
+  return dz > 1e-9 * __builtin_fabs(z) && dz > 1e-100 && dz < 1e100;
+}
 
 template <bool MOL>
 struct RowStore {
@@ -61,11 +69,12 @@ struct RowStore {
   }
   // Room for the lens rows of the wavefront's lanes that are here: each its own number (molecule-major), or as
   // many each as the longest (interleaved).  A molecule that is not moving forward at a step that its z
-  // resolves, that alone wants a large part of the room, or that finds none left is odd.
+  // resolves or that finds no room left is odd: k_zplan has seen to it that there is room and that there are no such
+  // molecules, except where an axial acceleration changes vz before the lens.
   __device__ __forceinline__ bool lens_begin(const MState &m, int n_full, double dz) {
     nb = nf;
     nfull = n_full;
-    odd = !(dz > 1e-9 * __builtin_fabs(m.z) && dz > 1e-100 && dz < 1e100) || (int64_t)n_full >= Z->cap_rows / 1024;
+    odd = !moves_on(dz, m.z) || (int64_t)n_full >= Z->cap_rows;
     const uint32_t rows = odd ? 0u : (uint32_t)n_full + 1u;
     // over the lanes here, bit by bit: the sum of rows (below this lane, and of all), or the largest
     uint64_t among = __builtin_amdgcn_ballot_w64(true);
@@ -99,12 +108,24 @@ struct RowStore {
   __device__ __forceinline__ void lens_end(const MState &m) { row(m); }
 };
 
+// A value that the whole wavefront reads: through the constant address space it is a scalar load, which does not
+// wait behind the wavefront's stores (vector memory operations complete in order) and takes no vector registers.
+// What it reads was written by an earlier kernel.
+template <bool UNIFORM, class T>
+__device__ __forceinline__ T load(const T *p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (UNIFORM) return *(const __attribute__((address_space(4))) T *)p;
+#endif
+  return *p;
+}
+
 template <int FORCE, bool MOL, int KM>
 __global__ void __launch_bounds__(KM == KM_CIRC ? 512 : 256) k_zrows(KBeam B, KTab KT, ctraj_record RC, ZRows Z) {
   extern __shared__ __attribute__((aligned(16))) double lds[];
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  if (load<true>(Z.go) == 0) return;
   const Tables T = stage_tables(lds, KT);
   __syncthreads();
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < Z.n; k += stride) {
     const int64_t s = Z.s0 + k;
     const int64_t i = RC.index ? RC.index[s] : s;
@@ -132,7 +153,7 @@ __global__ void __launch_bounds__(KM == KM_CIRC ? 512 : 256) k_zrows(KBeam B, KT
     if (sk.odd) Z.odd[1 + atomicAdd(&Z.odd[0], 1u)] = (uint32_t)s;
     Z.hdr[k] = make_int4(sk.nb < 0 ? sk.nf : sk.nb, sk.nl, sk.nfull, sk.odd ? -1 : sk.nf | st << 16);
     Z.lens_at[k] = sk.at;
-    if (RC.n_rows) RC.n_rows[s] = 0;  // k_zsamples counts
+    if (RC.n_rows) RC.n_rows[s] = 0;  // k_zfaces and k_zlens count
     if (RC.label) RC.label[s] = label;
   }
 }
@@ -157,17 +178,6 @@ __device__ __forceinline__ void lens_force(const Force<FORCE> &F, const WsMem &w
     force_hex_r2(ws, umax, F.ks, F.cu, F.g, x, y, __builtin_fma(x, x, y * y), ax, ay);
   else
     force_lin(ws, umax, F.ks, F.cu, F.g, x, y, ax, ay);
-}
-
-// A value that the whole wavefront reads: through the constant address space it is a scalar load, which does not
-// wait behind the wavefront's stores (vector memory operations complete in order) and takes no vector registers.
-// What it reads was written by an earlier kernel.
-template <bool UNIFORM, class T>
-__device__ __forceinline__ T load(const T *p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (UNIFORM) return *(const __attribute__((address_space(4))) T *)p;
-#endif
-  return *p;
 }
 
 __device__ __forceinline__ void ahead(MState &o, double zk) {
@@ -339,6 +349,7 @@ __device__ __forceinline__ void store_field(const ctraj_record &RC, int i, int64
 template <bool MOL>
 __global__ void __launch_bounds__(256) k_zfaces(KBeam B, ctraj_record RC, ZRows Z, int lens_e, int tile) {
   __shared__ double2 s_out[MOL ? 4 : 1][192];
+  if (load<true>(Z.go) == 0) return;
   const ctraj_elem &E = B.elems[lens_e];
   const double z1 = load<true>(&E.z1), dt = load<true>(&E.p[2]);
   const Grid G{RC.z_start, RC.z_step, RC.cap};
@@ -388,6 +399,7 @@ __global__ void __launch_bounds__(256) k_zfaces(KBeam B, ctraj_record RC, ZRows 
 template <int FORCE, bool MOL>
 __global__ void __launch_bounds__(256) k_zlens(KBeam B, KTab KT, ctraj_record RC, ZRows Z, int lens_e, int tile) {
   __shared__ double2 s_out[MOL ? 4 : 1][192];
+  if (load<true>(Z.go) == 0) return;
   const ctraj_elem &E = B.elems[lens_e];
   const Force<FORCE> F = make_force<FORCE>(E, B.g);
   const double z1 = E.z1, R2 = E.p[1], h = E.p[2], L = E.p[3];
@@ -474,9 +486,76 @@ __global__ void __launch_bounds__(256) k_zlens(KBeam B, KTab KT, ctraj_record RC
   }
 }
 
-__global__ void __launch_bounds__(64) k_zclear(unsigned long long *used, uint32_t *odd) {
-  if (threadIdx.x == 0) *used = 0;
-  if (odd && threadIdx.x == 1) odd[0] = 0;
+// What a run of the three kernels is for, decided before it: that the lens rows of every slice have room, that every
+// molecule can be sampled by them, and that the lens rows of all are within the bounds in which they are the faster
+// form (zgrid_in_two).  One workgroup a slice; the last to end decides.
+struct ZPlan {
+  uint32_t go, done, bad;
+  unsigned long long rows;
+};
+
+struct ZPlanArgs {
+  ZPlan *plan;
+  unsigned long long *used;  // [slices]
+  uint32_t *odd;
+  int64_t slice, cap_rows;
+  double h, z0;  // the lens step and entrance
+  float steps;   // L / h: a molecule's steps are this over its vz
+  double lo, hi;
+};
+
+template <bool MOL>
+__global__ void __launch_bounds__(1024) k_zplan(ctraj_record RC, ZPlanArgs A) {
+  __shared__ unsigned long long s_rows;
+  __shared__ uint32_t s_bad;
+  if (threadIdx.x == 0) s_rows = 0, s_bad = 0;
+  __syncthreads();
+  const int64_t s0 = (int64_t)blockIdx.x * A.slice, n = min(A.slice, RC.n - s0);
+  unsigned long long sum = 0;
+  bool bad = false;
+  constexpr int AT_ONCE = 8;  // loads in flight: the workgroup is alone on its CU
+  for (int64_t k0 = threadIdx.x; k0 - threadIdx.x < n; k0 += AT_ONCE * 1024) {
+    double vz[AT_ONCE];
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u) {
+      const int64_t k = k0 + u * 1024;
+      vz[u] = k < n ? RC.in.vz[RC.index ? RC.index[s0 + k] : s0 + k] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u) {
+      const bool here = k0 + u * 1024 < n, ok = moves_on(vz[u] * A.h, A.z0);
+      uint32_t rows = ok ? (uint32_t)fminf(A.steps * __builtin_amdgcn_rcpf((float)vz[u]), 0x1p24f) + 2u : 0u;
+      bad = bad || (here && !ok);
+      if constexpr (!MOL) {  // padded to the longest of the 64
+        for (int o = 32; o > 0; o >>= 1) rows = max(rows, (uint32_t)__shfl_xor((int)rows, o));
+      }
+      sum += rows;
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+  if (lane_id() == 0) atomicAdd(&s_rows, sum);
+  if (bad) s_bad = 1;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  A.used[blockIdx.x] = 0;
+  uint32_t no = s_bad | (uint32_t)(s_rows > (unsigned long long)A.cap_rows);
+  unsigned long long rows = s_rows;
+  if (gridDim.x > 1) {
+    atomicAdd(&A.plan->rows, rows);
+    if (no) atomicOr(&A.plan->bad, 1u);
+    __threadfence();
+    if (atomicAdd(&A.plan->done, 1u) != gridDim.x - 1) return;
+    __threadfence();
+    rows = atomicAdd(&A.plan->rows, 0ull);
+    no = atomicOr(&A.plan->bad, 0u);
+  }
+  const bool go = !no && (double)rows >= A.lo && (double)rows <= A.hi;
+  A.plan->go = go;
+  A.odd[0] = go ? 0u : ZGRID_ALL;
+}
+
+__global__ void __launch_bounds__(64) k_zclear(ZPlan *plan) {
+  if (threadIdx.x == 0) plan->done = 0, plan->bad = 0, plan->rows = 0;
 }
 
 using RowsFn = void (*)(KBeam, KTab, ctraj_record, ZRows);
@@ -491,15 +570,14 @@ RowsFn rows_kernel(bool mol, bool circ) {
 
 // Molecules walked and sampled at a time, and the lens rows kept for them (512 MiB): 409 of a molecule's own
 // number each, or 512 where they are padded to the longest of 64
-constexpr int64_t SLICE_MOL = ZGRID_SLICE_MOL, SLICE_FIELD = 32768;
-constexpr int64_t ROWS_MAX = ((int64_t)512 << 20) / 32;
+constexpr int64_t SLICE_MOL = ZGRID_SLICE_MOL, SLICE_FIELD = ZGRID_SLICE_FIELD;
 
 }  // namespace
 
 namespace ctraj {
 
 int record_zgrid(ctraj_ctx *c, const ctraj_record &RC, int lens_e, bool circ_only, const KBeam &B, const KTab &kt,
-                 size_t lds, ZGridPlan &plan) {
+                 size_t lds, const ZGridSteps &steps, ZGridPlan &plan) {
   plan = ZGridPlan{};
   const bool mol = RC.mode == CTRAJ_REC_ZGRID_MOL, hex = c->force == CTRAJ_FORCE_WSPLINE_HEX;
   const RowsFn kr = hex ? rows_kernel<CTRAJ_FORCE_WSPLINE_HEX>(mol, circ_only)
@@ -513,15 +591,16 @@ int record_zgrid(ctraj_ctx *c, const ctraj_record &RC, int lens_e, bool circ_onl
   const int64_t pad = (slice + 63) & ~(int64_t)63;
   ZRows Z{};
   Z.n_face = n_face;
-  Z.cap_rows = std::min<int64_t>(ROWS_MAX, pad * 1024);
+  Z.cap_rows = std::min<int64_t>(ZGRID_ROWS, pad * ZGRID_ROWS_EACH);
   size_t at = 0;
   const auto place = [&](size_t bytes) {
     const size_t p = at;
     at += (bytes + 255) & ~(size_t)255;
     return p;
   };
-  const size_t p_used = place(8), p_odd = place(4 * ((size_t)RC.n + 1)), p_hdr = place(16 * (size_t)pad),
-               p_at = place(8 * (size_t)pad), p_face = place((size_t)pad * n_face * 80),
+  const int64_t slices = (RC.n + slice - 1) / slice;
+  const size_t p_plan = place(sizeof(ZPlan)), p_used = place(8 * (size_t)slices),
+               p_odd = place(4 * ((size_t)RC.n + 1)), p_hdr = place(16 * (size_t)pad), p_at = place(8 * (size_t)pad), p_face = place((size_t)pad * n_face * 80),
                p_lens = place((size_t)Z.cap_rows * 32);
   void *ws = nullptr;
   int rc = lds_limit(c, (const void *)kr, lds);
@@ -531,7 +610,9 @@ int record_zgrid(ctraj_ctx *c, const ctraj_record &RC, int lens_e, bool circ_onl
     return CTRAJ_OK;  // plan.ws stays null: the one-kernel form needs no memory
   }
   char *w = (char *)ws;
-  Z.used = (unsigned long long *)(w + p_used);
+  unsigned long long *used = (unsigned long long *)(w + p_used);
+  ZPlan *zp = (ZPlan *)(w + p_plan);
+  Z.go = &zp->go;
   Z.odd = (uint32_t *)(w + p_odd);
   Z.hdr = (int4 *)(w + p_hdr);
   Z.lens_at = (int64_t *)(w + p_at);
@@ -544,18 +625,24 @@ int record_zgrid(ctraj_ctx *c, const ctraj_record &RC, int lens_e, bool circ_onl
     block *= 2;
   const int tile = mol ? 512 : 16;
   const int tiles = (RC.cap + tile - 1) / tile;
-  hipError_t e = hipSuccess;
+  const ctraj_elem &lens = c->h_elems[lens_e];
+  const ZPlanArgs plan_args{zp, used, Z.odd, slice, Z.cap_rows, lens.p[2], lens.z0, (float)(lens.p[3] / lens.p[2]),
+                            steps.lo * (double)RC.n, steps.hi * (double)RC.n};
+  if (slices > 1) hipLaunchKernelGGL(k_zclear, dim3(1), dim3(64), 0, c->stream, zp);
+  if (mol) hipLaunchKernelGGL(k_zplan<true>, dim3((int)slices), dim3(1024), 0, c->stream, RC, plan_args);
+  else hipLaunchKernelGGL(k_zplan<false>, dim3((int)slices), dim3(1024), 0, c->stream, RC, plan_args);
+  hipError_t e = hipGetLastError();
+  // grids for a whole slice (each asks the runtime for the occupancy, some 8 us, more than a launch)
+  const int64_t items = (mol ? slice : (slice + 63) >> 6) * tiles;
+  const dim3 gr(grid_for(c, (const void *)kr, block, lds, slice, 0)), gf(grid_for(c, (const void *)kf, 256, 0, items * 64, 0)),
+      gl(grid_for(c, (const void *)kl, 256, 0, items * 64, 0));
   for (int64_t s0 = 0; s0 < RC.n && e == hipSuccess; s0 += slice) {
     Z.s0 = s0;
+    Z.used = used + s0 / slice;
     Z.n = std::min(slice, RC.n - s0);
-    hipLaunchKernelGGL(k_zclear, dim3(1), dim3(64), 0, c->stream, Z.used, s0 == 0 ? Z.odd : nullptr);
-    const int g1 = grid_for(c, (const void *)kr, block, lds, Z.n, 0);
-    hipLaunchKernelGGL(kr, dim3(g1), dim3(block), lds, c->stream, B, kt, RC, Z);
-    const int64_t items = (mol ? Z.n : (Z.n + 63) >> 6) * tiles;
-    hipLaunchKernelGGL(kf, dim3(grid_for(c, (const void *)kf, 256, 0, items * 64, 0)), dim3(256), 0, c->stream, B, RC, Z,
-                       lens_e, tile);
-    hipLaunchKernelGGL(kl, dim3(grid_for(c, (const void *)kl, 256, 0, items * 64, 0)), dim3(256), 0, c->stream, B, kt, RC,
-                       Z, lens_e, tile);
+    hipLaunchKernelGGL(kr, gr, dim3(block), lds, c->stream, B, kt, RC, Z);
+    hipLaunchKernelGGL(kf, gf, dim3(256), 0, c->stream, B, RC, Z, lens_e, tile);
+    hipLaunchKernelGGL(kl, gl, dim3(256), 0, c->stream, B, kt, RC, Z, lens_e, tile);
     e = hipGetLastError();
   }
   if (e != hipSuccess) {
