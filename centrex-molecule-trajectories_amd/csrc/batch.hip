@@ -602,9 +602,7 @@ __global__ void __launch_bounds__(256) k_batch_post(BArgs A, BPipe P) {
       queue_get_done(P.q, (int64_t)P.lt[BLT_LIST + j], m, key);
       c = (int)(key & QKEY_INDEX);
       const uint32_t status = (uint32_t)((key >> 40) & 0xff);
-      // x and y in registers of their own: this compiler (ROCm 7.2) keeps them in the 16 bytes they were loaded in and
-      // then overwrites y inside the walk's loop (its own -verify-machineinstrs reports it)
-      asm volatile("" : "+v"(m.x), "+v"(m.y));
+      own_registers(m);
       const BLensC &K = A.lensk[c];
       m.ax = 0.0;
       m.ay = -g;

@@ -366,6 +366,7 @@ __global__ void __launch_bounds__(256) k_propagate(KBeam B, KTab KT, ctraj_run R
           // the row at z1 stores (0, -g, 0) (configuration mode); the reference lens's exit hop was made
           // by k_lens with its stored a = l1 and ended with the same row
           m.ax = 0.0; m.ay = -B.g; m.az = 0.0;
+          own_registers(m);
           label = B.label_detected;
           const uint32_t f0 = wc.faces;
           if (KM == KM_CIRC && (B.tame & walk_tame(m)))

@@ -93,6 +93,20 @@ __device__ __forceinline__ void drift_tame(MState &m, double zf, double iv, doub
   m.t = m.t + dt;
 }
 
+// A queue entry's molecule in registers of its own, before a walk.  The entry is read in 16-byte pieces, and this
+// compiler (ROCm 7.2) may keep two fields of one piece together as one value through the walk's loop; its register
+// coalescer has then lost track of one of them, which the loop overwrote (k_batch_post counted molecules twice).  An
+// empty asm on the fields does not separate them for certain, a move that the compiler cannot join does.  The build
+// has the machine code verified (build.py), which reports the fault.
+__device__ __forceinline__ void own_registers(MState &m) {
+  const auto own = [](double &v) {
+    double r;
+    asm("v_mov_b64 %0, %1" : "=v"(r) : "v"(v));
+    v = r;
+  };
+  own(m.x); own(m.y); own(m.z); own(m.vx); own(m.vy); own(m.vz); own(m.t);
+}
+
 // walk_plain over circular apertures for a tame molecule.
 template <bool SE>
 __device__ __forceinline__ bool walk_circ_tame(const ctraj_elem *__restrict__ elems, int e0, int e1, double g, MState &m,
