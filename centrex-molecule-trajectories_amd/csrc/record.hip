@@ -513,18 +513,22 @@ __global__ void __launch_bounds__(1024) k_zplan(ctraj_record RC, ZPlanArgs A) {
   const int64_t s0 = (int64_t)blockIdx.x * A.slice, n = min(A.slice, RC.n - s0);
   unsigned long long sum = 0;
   bool bad = false;
-  constexpr int AT_ONCE = 8;  // loads in flight: the workgroup is alone on its CU
+  constexpr int AT_ONCE = 16;  // loads in flight: the workgroup is alone on its CU
   for (int64_t k0 = threadIdx.x; k0 - threadIdx.x < n; k0 += AT_ONCE * 1024) {
     double vz[AT_ONCE];
+    int64_t at[AT_ONCE];
 #pragma unroll
-    for (int u = 0; u < AT_ONCE; ++u) {
-      const int64_t k = k0 + u * 1024;
-      vz[u] = k < n ? RC.in.vz[RC.index ? RC.index[s0 + k] : s0 + k] : 0.0;
+    for (int u = 0; u < AT_ONCE; ++u) at[u] = s0 + min(k0 + u * 1024, n - 1);
+    if (RC.index) {
+#pragma unroll
+      for (int u = 0; u < AT_ONCE; ++u) at[u] = RC.index[at[u]];
     }
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u) vz[u] = RC.in.vz[at[u]];
 #pragma unroll
     for (int u = 0; u < AT_ONCE; ++u) {
       const bool here = k0 + u * 1024 < n, ok = moves_on(vz[u] * A.h, A.z0);
-      uint32_t rows = ok ? (uint32_t)fminf(A.steps * __builtin_amdgcn_rcpf((float)vz[u]), 0x1p24f) + 2u : 0u;
+      uint32_t rows = here && ok ? (uint32_t)fminf(A.steps * __builtin_amdgcn_rcpf((float)vz[u]), 0x1p24f) + 2u : 0u;
       bad = bad || (here && !ok);
       if constexpr (!MOL) {  // padded to the longest of the 64
         for (int o = 32; o > 0; o >>= 1) rows = max(rows, (uint32_t)__shfl_xor((int)rows, o));
