@@ -49,7 +49,7 @@ struct Tables {
 // Where one r table sits in Tables::rt.  The host resolves a lens's table id into these before
 // launch: ctraj_elem.table = knot offset, .reserved = knot count, .p[6] = 1/(r_1 - r_0), the
 // first and last knots .p[4] = r_0, .p[5] = r_last (slots the spline forces use for their scales) and
-// .p[7] = 1 where the table, g and the step dz are of moderate size (ref_tame).
+// .p[7] = 1 where the table and g are of moderate size (resolve_elems; ref_step tests the rest at every step).
 struct RDesc {
   int off, n;
   double invh, r0, rlast;
@@ -360,16 +360,17 @@ __device__ __forceinline__ void ref_step_plain(const Force<FORCE> &F, const Tabl
 // The reference's example lens is bound by the latency of one molecule's steps: four dependent force
 // evaluations of a square root, a table look-up and two divisions, then divisions by 6.  Written plainly,
 // a step is 600 VALU instructions and some 70 branches, because every division and square root carries its
-// scaling for extreme exponents.  Between 2^-200 and 2^200 (ref_tame: the state, checked every step; dt, vz,
-// g and the table, checked once) nothing needs scaling, and the same correctly rounded results come from
-// shared pieces:
+// scaling for extreme exponents.  Between 2^-200 and 2^200 (the state, vz and dt, which ref_step tests at every
+// step; g and the table, which the host has tested: RDesc) nothing needs scaling, and the results come from shared
+// pieces:
 //   * sqrt: the compiler's own Goldschmidt sequence without the scaling; its half reciprocal h1, refined
 //     once against r, is the reciprocal that both divisions by r share;
-//   * a quotient n / d from y = 1/d (relative error at most 2^-53): q near n y, then q + (n - q d) y, the
+//   * a quotient n / d from y near 1/d (relative error about 2^-53): q near n y, then q + (n - q d) y, the
 //     final two operations of the hardware's division sequence (q = a_r (x y) is ready one operation after
-//     a_r);
-//   * n / 6 likewise from the constant 1/6 (its error is a quarter of an ulp, so q is within one ulp and the
-//     corrected quotient is the correctly rounded one);
+//     a_r).  y is not the hardware's own reciprocal, so that the quotient is the correctly rounded one is not
+//     proved (its error before rounding is some 2^-104 of it); the tests compare it with the oracle's bit for bit;
+//   * n / 6 likewise from the constant 1/6, the correctly rounded reciprocal, with q within one ulp: there the
+//     corrected quotient is the correctly rounded one (Markstein's theorem);
 //   * the table segment is guessed from the first estimate of the square root while it is refined, and checked
 //     against the final r;
 //   * 2 a and a / 2 are exact, so each goes with its sum into one fused operation;

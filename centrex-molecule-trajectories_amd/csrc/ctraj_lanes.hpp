@@ -39,9 +39,8 @@ struct LaneMol {
 // the zero components of the acceleration), and a wavefront runs nearly every face of the beamline.  With
 // a = (0, -g, 0) and faces, z, vz and g of moderate size (walk_tame_elems on the host, walk_tame per molecule) the
 // same values come from 22:
-//   * every face's time is the correctly rounded (zf - z) / vz from one reciprocal of vz, by the last two
-//     operations of the hardware's own division sequence (nothing needs its scaling: a face is nonzero, so zf - z
-//     is zero or at least 2^-160);
+//   * every face's time (zf - z) / vz by the operations of the compiled division, of which the reciprocal's are made
+//     once for all faces (nothing needs its scaling: a face is nonzero, so zf - z is zero or at least 2^-160);
 //   * 0 dt^2 / 2 and 0 dt add +0, which changes only a -0;
 //   * (a dt^2) / 2 is exact and goes with its sum into one fused operation; dt = 0 adds zeros (velocities are
 //     finite), where the plain drift leaves the molecule as it is.

@@ -33,9 +33,10 @@ class SmoothFlux:
     """The objective over a fixed molecule sample on one device.
 
     ``x, y, vx, vy, eps`` are host arrays (uploaded once); ``sigma_vz`` scales eps into vz.
-    ``ckpt_every`` bounds the lens checkpoint interval (the library takes checkpoints more often where
-    memory allows; results do not depend on it); ``max_steps`` bounds the full RK4 steps per lens
-    (default: what the slowest molecule of the evaluated parameter sets needs).
+    ``ckpt_every`` bounds the lens checkpoint interval: with gradients the library keeps one every 4 steps,
+    whatever is asked for, while that store stays within 2 GiB and the device has room for it, and the store
+    stays with the context (results do not depend on it); ``max_steps`` bounds the full RK4 steps per lens
+    (default: what the slowest molecule of the evaluated parameter sets needs) and with them the store.
 
     The molecules are uploaded in order of eps, hence of vz for every parameter set: each wavefront
     of the kernel takes 64 consecutive molecules through every lens step without refill, and

@@ -362,7 +362,11 @@ typedef struct ctraj_smooth {
   double *J;                            /* device [n_cfg] */
   double *grad;                         /* device [n_cfg][n_params], or NULL: objective only */
   int64_t *n_capped;                    /* device [1] or NULL: += molecules whose lens step count was cut to max_steps */
-  int32_t ckpt_every;                   /* K >= 1: at most K steps between checkpoints */
+  int32_t ckpt_every;                   /* K >= 1: at most K steps between checkpoints.  With gradients and K > 4 a
+                                         * checkpoint is kept every 4 steps while that store stays within 2 GiB and
+                                         * the device has room for it, whatever K (results do not depend on it); the
+                                         * store (1.1 GB for 520 steps and 262,144 molecules or more, less for
+                                         * fewer) stays with the context */
   int32_t max_steps;                    /* full RK4 steps per lens at most (>= 1); bounds the checkpoint store */
   int32_t block;                        /* threads per block, multiple of 64 up to 512 (0 = 256, or with gradients
                                          * by the molecules, as many up to 1024 as the LDS of one CU holds) */
