@@ -128,7 +128,7 @@ class Context:
         self.bound = None  # the CompiledBeamline currently set on the device
         self.lock = threading.RLock()
         self._pinned = None  # (address, uint8 view), made on first use
-        self._uploads, self._uploads_lock = [], threading.Lock()  # host arrays whose copies are queued
+        self._uploads, self._uploads_lock = [], threading.RLock()  # host arrays whose copies are queued
 
     # --- memory ---
     def alloc(self, n, dtype=np.float64) -> DeviceArray:

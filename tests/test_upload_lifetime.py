@@ -64,3 +64,11 @@ def test_a_failed_wait_keeps_them(stubbed, monkeypatch):
     assert alive() is not None
     ctx.sync()
     assert alive() is None
+
+
+def test_a_wait_inside_the_list(stubbed):
+    """A collection may run anywhere, also where the list is changed, and its finalizers may wait for the stream."""
+    lib, ctx = stubbed
+    with ctx._uploads_lock:
+        ctx.sync()
+    assert "ctraj_sync" in lib.calls
